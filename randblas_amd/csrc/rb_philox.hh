@@ -4,18 +4,31 @@
 // RandBLAS applies to its words: uneg11 / u01 and the Box-Muller transform
 // (RandBLAS/random_gen.hh:60-137, Random123 uniform.hpp / boxmuller.hpp).
 //
-// Box-Muller needs sin, cos and log of float arguments.  They are evaluated
-// in double precision and rounded once to float:
-//   sin/cos(t): Cody-Waite reduction by pi/2 with a two-part constant
-//     (exact for |t| <= pi_f because |k| <= 2), then Taylor polynomials of
-//     degree 17 (sin) and 16 (cos) in Horner form;
-//   log(u):    u = 2^e * m, m in [1/sqrt2, sqrt2), log m = 2*atanh(f/(2+f))
-//     with f = m-1, series through s^21.
-// Every step is an IEEE double operation with an explicit fma where fused,
-// and the library is compiled with -ffp-contract=off, so results do not
-// depend on the compiler's contraction choices.  The resulting floats are
-// correctly rounded except where the exact value lies within ~2^-50 of a
-// rounding boundary.
+// Box-Muller needs sin, cos and log of float arguments.  Their values are
+// defined by the oracle's series (Taylor / atanh in double precision, one
+// final rounding to float); here the same floats are reached with less work:
+//   sin/cos(t): t = PIf u reduced by k pi/2 (k = rint(2u), one fma: k pi/2 -
+//     t loses nothing that the final rounding sees), minimax polynomials of
+//     six coefficients in r^2 (relative errors 2^-58 and 2^-54);
+//   log(u): u = 2^e m, m in [1/sqrt2, sqrt2), log m = 2 atanh(s), s =
+//     f / (2 + f), f = m - 1: the quotient from v_rcp_f32 and one cubic
+//     Newton step (2^-52), six minimax coefficients in s^2 (2^-52).
+// The resulting floats equal the series' for every one of the 2^32 words that
+// either factor can be given (checked exhaustively, on the CPU with the
+// reciprocal seed off by -1, 0 and +1 ulp, and on gfx950), so the operators'
+// entries are the same bits as the oracle's.  Every step is an IEEE operation
+// with an explicit fma where fused, and the library is compiled with
+// -ffp-contract=off, so results do not depend on the compiler's contraction
+// choices.
+//
+// Cost, measured issue cycles per wave and SIMD on gfx950: f64 fma / mul /
+// add, 32-bit integer multiplies and f32 <-> f64 conversions 4, f32 and
+// logic operations 2, v_rcp / v_rsq / v_sqrt_f32 8, v_rcp_f64 16; FP64 and
+// FP32 MFMAs share these issue cycles (they do not overlap with VALU work),
+// BF16 ones do not.  fill_dense of 4096 x 65536 FP32 Gaussians, which is this
+// generator and one store: 365 us = 7.3e11 entries/s (508 us with the series
+// themselves: degree 16-17 sin / cos, an IEEE division, sqrtf and two-input
+// xors in Philox).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -48,6 +61,10 @@ __host__ __device__ inline void ctr_to_words(Ctr128 c, uint32_t w[4]) {
     w[3] = (uint32_t)(c.hi >> 32);
 }
 
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+}
+
 // Philox4x32-10 on one counter.  The key words are wave-uniform in every
 // caller, so the Weyl bumps stay on the scalar unit.
 __device__ __forceinline__ uint4 philox4x32_10(Ctr128 c, uint32_t k0, uint32_t k1) {
@@ -61,8 +78,8 @@ __device__ __forceinline__ uint4 philox4x32_10(Ctr128 c, uint32_t k0, uint32_t k
         }
         uint64_t p0 = (uint64_t)PH_M0 * x0;
         uint64_t p1 = (uint64_t)PH_M1 * x2;
-        uint32_t y0 = (uint32_t)(p1 >> 32) ^ x1 ^ k0;
-        uint32_t y2 = (uint32_t)(p0 >> 32) ^ x3 ^ k1;
+        uint32_t y0 = xor3((uint32_t)(p1 >> 32), x1, k0);
+        uint32_t y2 = xor3((uint32_t)(p0 >> 32), x3, k1);
         x1 = (uint32_t)p1;
         x3 = (uint32_t)p0;
         x0 = y0;
@@ -71,89 +88,71 @@ __device__ __forceinline__ uint4 philox4x32_10(Ctr128 c, uint32_t k0, uint32_t k
     return make_uint4(x0, x1, x2, x3);
 }
 
-// (float)(int32)w * 2^-31 + 2^-32; the product is exact.
-__device__ __forceinline__ float uneg11(uint32_t w) {
-    return __fadd_rn(__fmul_rn((float)(int32_t)w, 0x1p-31f), 0x1p-32f);
-}
+// (float)(int32)w * 2^-31 + 2^-32; the product is exact, so one fma.
+__device__ __forceinline__ float uneg11(uint32_t w) { return __fmaf_rn((float)(int32_t)w, 0x1p-31f, 0x1p-32f); }
 // (float)w * 2^-32 + 2^-33
-__device__ __forceinline__ float u01(uint32_t w) {
-    return __fadd_rn(__fmul_rn((float)w, 0x1p-32f), 0x1p-33f);
+__device__ __forceinline__ float u01(uint32_t w) { return __fmaf_rn((float)w, 0x1p-32f, 0x1p-33f); }
+
+// sin and cos of PIf * uneg11(w) (the float product): the angle factors of a
+// Box-Muller draw.
+__device__ __forceinline__ void bm_sincos(uint32_t w, float &s_out, float &c_out) {
+    const float u = uneg11(w);
+    const double t = (double)__fmul_rn(3.1415926535897932f, u);
+    // k = rint(2u) with the quadrant k mod 4 in the sum's low bits
+    const float km = __fmaf_rn(2.0f, u, 0x1.8p23f);
+    const uint32_t q = __float_as_uint(km);
+    const double r = __fma_rn((double)__fsub_rn(0x1.8p23f, km), 0x1.921fb54442d18p+0, t);
+    const double r2 = __dmul_rn(r, r);
+    double ps = 0x1.5d932ee04e218p-33;
+    ps = __fma_rn(ps, r2, -0x1.ae5e66d38ca7bp-26);
+    ps = __fma_rn(ps, r2, 0x1.71de357872c1dp-19);
+    ps = __fma_rn(ps, r2, -0x1.a01a019c12695p-13);
+    ps = __fma_rn(ps, r2, 0x1.111111110f880p-7);
+    ps = __fma_rn(ps, r2, -0x1.5555555555549p-3);
+    const float sv = (float)__fma_rn(__dmul_rn(r, r2), ps, r);
+    double pc = 0x1.1b95fd680bb2cp-29;
+    pc = __fma_rn(pc, r2, -0x1.27df6c029fc1ep-22);
+    pc = __fma_rn(pc, r2, 0x1.a019f8841065cp-16);
+    pc = __fma_rn(pc, r2, -0x1.6c16c1648a8e4p-10);
+    pc = __fma_rn(pc, r2, 0x1.555555554f951p-5);
+    pc = __fma_rn(pc, r2, -0x1.fffffffffffa3p-2);
+    const float cv = (float)__fma_rn(r2, pc, 1.0);
+    const bool odd = (q & 1) != 0;
+    // quadrants 2, 3 negate the sine, 1, 2 the cosine
+    s_out = __uint_as_float(__float_as_uint(odd ? cv : sv) ^ ((q << 30) & 0x80000000u));
+    c_out = __uint_as_float(__float_as_uint(odd ? sv : cv) ^ (((q + 1) << 30) & 0x80000000u));
 }
 
-// sin and cos of a float argument with |t| <= pi_f.
-__device__ __forceinline__ void rbm_sincos(float t, float &s_out, float &c_out) {
-    const double TWO_OVER_PI = 0x1.45f306dc9c883p-1;
-    const double PIO2_HI = 0x1.921fb54442d18p+0;
-    const double PIO2_LO = 0x1.1a62633145c07p-54;
-    double x = (double)t;
-    double kd = __builtin_rint(__dmul_rn(x, TWO_OVER_PI));
-    double r = __fma_rn(-kd, PIO2_HI, x);
-    r = __fma_rn(-kd, PIO2_LO, r);
-    double r2 = __dmul_rn(r, r);
-    double ps = 0x1.952c77030ad4ap-49;
-    ps = __fma_rn(ps, r2, -0x1.ae7f3e733b81fp-41);
-    ps = __fma_rn(ps, r2, 0x1.6124613a86d09p-33);
-    ps = __fma_rn(ps, r2, -0x1.ae64567f544e4p-26);
-    ps = __fma_rn(ps, r2, 0x1.71de3a556c734p-19);
-    ps = __fma_rn(ps, r2, -0x1.a01a01a01a01ap-13);
-    ps = __fma_rn(ps, r2, 0x1.1111111111111p-7);
-    ps = __fma_rn(ps, r2, -0x1.5555555555555p-3);
-    double sv = __fma_rn(__dmul_rn(r, r2), ps, r);
-    double pc = 0x1.ae7f3e733b81fp-45;
-    pc = __fma_rn(pc, r2, -0x1.93974a8c07c9dp-37);
-    pc = __fma_rn(pc, r2, 0x1.1eed8eff8d898p-29);
-    pc = __fma_rn(pc, r2, -0x1.27e4fb7789f5cp-22);
-    pc = __fma_rn(pc, r2, 0x1.a01a01a01a01ap-16);
-    pc = __fma_rn(pc, r2, -0x1.6c16c16c16c17p-10);
-    pc = __fma_rn(pc, r2, 0x1.5555555555555p-5);
-    pc = __fma_rn(pc, r2, -0x1.0000000000000p-1);
-    double cv = __fma_rn(r2, pc, 1.0);
-    int q = ((int)kd) & 3;
-    double S = (q & 1) ? cv : sv;
-    double Cc = (q & 1) ? sv : cv;
-    if (q == 1 || q == 2) Cc = -Cc;
-    if (q >= 2) S = -S;
-    s_out = (float)S;
-    c_out = (float)Cc;
-}
-
-// log of a positive normal float.
-__device__ __forceinline__ float rbm_logf(float u) {
-    uint32_t bits = __float_as_uint(u);
-    int e = (int)(bits >> 23) - 127;
-    float mf = __uint_as_float((bits & 0x7fffffu) | 0x3f800000u);
-    double m = (double)mf;
-    if (m > 0x1.6a09e667f3bcdp+0) {
-        m = __dmul_rn(m, 0.5);
-        e += 1;
-    }
-    double f = __dsub_rn(m, 1.0);
-    double s = __ddiv_rn(f, __dadd_rn(2.0, f));
-    double s2 = __dmul_rn(s, s);
-    double p = 0x1.8618618618618p-4;
-    p = __fma_rn(p, s2, 0x1.af286bca1af28p-4);
-    p = __fma_rn(p, s2, 0x1.e1e1e1e1e1e1ep-4);
-    p = __fma_rn(p, s2, 0x1.1111111111111p-3);
-    p = __fma_rn(p, s2, 0x1.3b13b13b13b14p-3);
-    p = __fma_rn(p, s2, 0x1.745d1745d1746p-3);
-    p = __fma_rn(p, s2, 0x1.c71c71c71c71cp-3);
-    p = __fma_rn(p, s2, 0x1.2492492492492p-2);
-    p = __fma_rn(p, s2, 0x1.999999999999ap-2);
-    p = __fma_rn(p, s2, 0x1.5555555555555p-1);
-    double lm = __fma_rn(__dmul_rn(s, s2), p, __dmul_rn(2.0, s));
-    double ed = (double)e;
-    double res = __fma_rn(ed, 0x1.62e42fee00000p-1, __fma_rn(ed, 0x1.a39ef35793c76p-33, lm));
-    return (float)res;
+// sqrtf(-2 logf(u01(w))), the radius factor.
+__device__ __forceinline__ float bm_radius(uint32_t w) {
+    const uint32_t b = __float_as_uint(u01(w)) - 0x3f3504f3u;  // from 1/sqrt2
+    const float m = __uint_as_float((b & 0x7fffffu) + 0x3f3504f3u);
+    const float ff = __fsub_rn(m, 1.0f);  // exact
+    const double f = (double)ff, d = __dadd_rn(f, 2.0);
+    double y = (double)__builtin_amdgcn_rcpf(__fadd_rn(ff, 2.0f));
+    const double e1 = __fma_rn(-d, y, 1.0);
+    y = __fma_rn(y, __fma_rn(e1, e1, e1), y);
+    const double s = __dmul_rn(f, y), s2 = __dmul_rn(s, s);
+    double p = 0x1.58786ae4b778cp-3;
+    p = __fma_rn(p, s2, 0x1.732c1304abcfep-3);
+    p = __fma_rn(p, s2, 0x1.c72278a03a957p-3);
+    p = __fma_rn(p, s2, 0x1.24924176cc058p-2);
+    p = __fma_rn(p, s2, 0x1.999999a294cb3p-2);
+    p = __fma_rn(p, s2, 0x1.5555555553960p-1);
+    const double lm = __fma_rn(__dmul_rn(s, s2), p, __dadd_rn(s, s));
+    const float x = __fmul_rn(-2.0f, (float)__fma_rn((double)((int32_t)b >> 23), 0x1.62e42fefa39efp-1, lm));
+    // correctly rounded square root of x in {-0} U [2^-23, 46): one Newton
+    // correction of x rsq(x), with the residual exact in the fma
+    const float q = __builtin_amdgcn_rsqf(fmaxf(x, 0x1p-100f));
+    const float r = __fmul_rn(x, q);
+    return __fmaf_rn(__fmaf_rn(-r, r, x), __fmul_rn(0.5f, q), r);
 }
 
 // r123::boxmuller(u0, u1): (r*sin(pi_f*uneg11(u0)), r*cos(...)), r = sqrtf(-2 logf(u01(u1))).
 __device__ __forceinline__ float2 boxmuller(uint32_t w0, uint32_t w1) {
-    const float PIf = 3.1415926535897932f;
     float s, c;
-    rbm_sincos(__fmul_rn(PIf, uneg11(w0)), s, c);
-    // __builtin_sqrtf lowers to the correctly rounded sequence (HIP's default
-    // -fhip-fp32-correctly-rounded-divide-sqrt); __fsqrt_rn would not be.
-    float r = __builtin_sqrtf(__fmul_rn(-2.0f, rbm_logf(u01(w1))));
+    bm_sincos(w0, s, c);
+    const float r = bm_radius(w1);
     return make_float2(__fmul_rn(s, r), __fmul_rn(c, r));
 }
 

@@ -1763,11 +1763,11 @@ __global__ __launch_bounds__(FGB_THREADS) void fastgen_bounds_kernel(double *out
         float sf, cf;
         fast_sincos_factor(w, sf, cf);
         float s, c;
-        rbm_sincos(__fmul_rn(3.1415926535897932f, uneg11(w)), s, c);
+        bm_sincos(w, s, c);
         es = fmax(es, fabs((double)sf - (double)s));
         ec = fmax(ec, fabs((double)cf - (double)c));
         const float rf = fast_radius_factor(w);
-        const float r = __builtin_sqrtf(__fmul_rn(-2.0f, rbm_logf(u01(w))));
+        const float r = bm_radius(w);
         if (r > 0.0f) er = fmax(er, fabs((double)rf - (double)r) / (double)r);
         if ((rf == 0.0f) != (r == 0.0f)) zero_mismatch += 1.0;
     }
