@@ -16,6 +16,7 @@
 #include <rocprim/device/device_scan.hpp>
 
 #include "rbx_internal.hh"
+#include "rbx_chain.hh"
 
 namespace rbx {
 
@@ -148,110 +149,336 @@ __global__ __launch_bounds__(256) void iid_cdf_kernel(Ctr128 ctr, uint32_t k0, u
     }
 }
 
-// The prefix sums in the reference's order, so they round exactly as its
-// loop does: one workgroup streams the weights through LDS in blocks of
-// CDF_BLK (double-buffered: waves 1-3 load block b + 1 while thread 0 adds
-// up block b), thread 0 runs the sequential chain sum = sum + max(w[i], 0)
-// over LDS, and the block's partial sums are written back coalesced.
-// status: 0 ok (total[0] = 1 / sum); 1 + i: w[i] < error_if_below (w[0..i)
+// weights_to_cdf: the prefix sums in the reference's order, with the bits of
+// its loop  sum = sum + max(w[i], 0).  The loop is one dependent addition per
+// weight (10.4 ms for 10^6 FP64 weights on one thread, 10 ns an addition);
+// inside a binade of the sum it is integer arithmetic that scans in parallel
+// (rbx_chain.hh), so the work is five short kernels over blocks of CDF_BLK:
+//   cdf_sums_kernel     block sums in FP64, in any order (a guess only), and
+//                       the first weight below error_if_below
+//   cdf_guess_kernel    their prefix sums: the binade each block is in
+//   cdf_advance_kernel  each block's advance in its guessed binade
+//   cdf_chain_kernel    one workgroup composes the blocks' advances in order,
+//                       64 at a time, as long as the exact sum is in the
+//                       guessed binade and stays there; a block that fails
+//                       the test (a binade is left inside it, or the guess
+//                       was wrong) is summed term by term in integer scans
+//                       with the exact exponent, one more for every binade
+//                       left.  No result depends on the guesses.
+//   cdf_write_kernel    each block's partial sums from its exact start, scaled
+// 10^6 FP64 weights: 9 blocks leave a binade.  Bound by latency: the chain
+// kernel's dependent scans.  Arrays of a few blocks skip the first three.
+// Meta: status 0 ok (inv = 1 / sum); 1 + i: w[i] < error_if_below (w[0..i)
 // hold the partial sums, as when the reference throws there); -1: the total
 // is below sqrt(n) * eps (w holds the partial sums, unscaled).
-constexpr int CDF_BLK = 2048;
+constexpr int CDF_BLK = 2048, CDF_PER = CDF_BLK / 256;
+constexpr int64_t CDF_DIRECT = 4;  // blocks that the chain kernel takes by itself
+struct CdfMeta {
+    long long status, first;  // first: weights before the first refused one
+    double inv;
+};
+
 template <typename T>
-__global__ __launch_bounds__(256) void weights_to_cdf_kernel(int64_t n, T *w, T error_if_below, long long *status,
-                                                             T *inv_total) {
-    __shared__ __attribute__((aligned(16))) T buf[2][CDF_BLK];
-    __shared__ int stop_sh;
-    const int tid = threadIdx.x, wave = tid >> 6;
-    const int64_t nb = (n + CDF_BLK - 1) / CDF_BLK;
-    auto load = [&](int64_t b, T *dst, int t0, int nt) {
-        const int64_t i0 = b * CDF_BLK;
-        for (int e = t0; e < CDF_BLK; e += nt)
-            if (i0 + e < n) dst[e] = w[i0 + e];
-    };
-    if (nb > 0) load(0, buf[0], tid, 256);
-    T sum = (T)0;  // thread 0's running sum
-    for (int64_t b = 0; b < nb; ++b) {
-        T *cur = buf[b & 1];
-        const int64_t i0 = b * CDF_BLK;
-        const int len = (int)(n - i0 < CDF_BLK ? n - i0 : CDF_BLK);
-        if (tid == 0) stop_sh = len;
-        __syncthreads();  // block b loaded; the previous write-back done
-        for (int e = tid; e < len; e += 256)
-            if (!(cur[e] >= error_if_below)) atomicMin(&stop_sh, e);
-        __syncthreads();
-        const int stop = stop_sh;  // entries [0, stop) of the block are summed
-        // val = max(val, 0) (std::max order), in parallel, off the chain
-        for (int e = tid; e < stop; e += 256)
-            if (cur[e] < (T)0) cur[e] = (T)0;
-        __syncthreads();
-        if (wave != 0 && stop == len && b + 1 < nb) load(b + 1, buf[(b + 1) & 1], tid - 64, 192);
-        if (tid == 0) {
-            // the chain alone: 16-byte LDS reads and writes; the next group
-            // of 8 vectors is read before this group's sums are formed, so
-            // the chain never waits on LDS latency (the read position is
-            // clamped inside the block buffer; values past `stop` are unused)
-            using V = std::conditional_t<sizeof(T) == 8, double2, float4>;
-            constexpr int PV = 16 / sizeof(T);  // values per vector
-            constexpr int GV = 8 * PV;          // values per group
-            T s_ = sum;
-            int e = 0;
-            V v[8];
+__global__ __launch_bounds__(256) void cdf_sums_kernel(int64_t n, const T *w, T error_if_below, double *bsum,
+                                                       int *bbad) {
+    __shared__ double red[4];
+    __shared__ int bad_sh;
+    const int tid = threadIdx.x;
+    const int64_t i0 = (int64_t)blockIdx.x * CDF_BLK;
+    if (tid == 0) bad_sh = CDF_BLK;
+    __syncthreads();
+    double v = 0.0;
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = *(const V *)(cur + u * PV);
-            for (; e + GV <= stop; e += GV) {
-                const int ne = e + GV < CDF_BLK - GV ? e + GV : CDF_BLK - GV;
-                V nx[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) nx[u] = *(const V *)(cur + ne + u * PV);
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    T *x = reinterpret_cast<T *>(&v[u]);
-#pragma unroll
-                    for (int q = 0; q < PV; ++q) {
-                        s_ = s_ + x[q];
-                        x[q] = s_;
-                    }
-                    *(V *)(cur + e + u * PV) = v[u];
-                }
-#pragma unroll
-                for (int u = 0; u < 8; ++u) v[u] = nx[u];
-            }
-            for (; e < stop; ++e) {
-                s_ = s_ + cur[e];
-                cur[e] = s_;
-            }
-            sum = s_;
+    for (int q = 0; q < CDF_PER; ++q) {
+        const int e = tid + 256 * q;
+        if (i0 + e < n) {
+            const T x = w[i0 + e];
+            if (!(x >= error_if_below)) atomicMin(&bad_sh, e);
+            v += x > (T)0 ? (double)x : 0.0;
         }
-        __syncthreads();
-        for (int e = tid; e < stop; e += 256) w[i0 + e] = cur[e];
-        if (stop < len) {
-            if (tid == 0) *status = 1 + i0 + stop;
-            return;
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
+    if ((tid & 63) == 0) red[tid >> 6] = v;
+    __syncthreads();
+    if (tid == 0) {
+        bsum[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+        bbad[blockIdx.x] = bad_sh;
+    }
+}
+
+// bsum[0 .. nb) -> exclusive prefix sums in bsum[0 .. nb]; first refused weight
+__global__ __launch_bounds__(1024) void cdf_guess_kernel(int64_t n, int64_t nb, double *bsum, const int *bbad,
+                                                         CdfMeta *meta) {
+    __shared__ double wsum[16];
+    __shared__ unsigned long long first_sh;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (tid == 0) first_sh = (unsigned long long)n;
+    __syncthreads();
+    double carry = 0.0;
+    for (int64_t b0 = 0; b0 < nb; b0 += 1024) {
+        const int64_t b = b0 + tid;
+        const double x = b < nb ? bsum[b] : 0.0;
+        if (b < nb && bbad[b] < CDF_BLK)
+            atomicMin(&first_sh, (unsigned long long)(b * CDF_BLK + bbad[b]));
+        double v = x;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const double y = __shfl_up(v, off);
+            if (lane >= off) v += y;
         }
+        if (lane == 63) wsum[wave] = v;
+        __syncthreads();
+        double pre = carry, tot = carry;
+        for (int q = 0; q < 16; ++q) {
+            if (q < wave) pre += wsum[q];
+            tot += wsum[q];
+        }
+        if (b < nb) bsum[b] = pre + (v - x);
+        carry = tot;
+        __syncthreads();
     }
     if (tid == 0) {
-        const T floor_sum = (T)sqrt((double)n) * std::numeric_limits<T>::epsilon();
-        if (!(sum >= floor_sum)) {
-            *status = -1;
-        } else {
-            *inv_total = (T)1 / sum;
-            *status = 0;
+        bsum[nb] = carry;
+        meta->first = (long long)first_sh;
+    }
+}
+
+template <typename T>
+__device__ __forceinline__ Advance shfl_up_advance(Advance a, int off) {
+    return Advance{(int64_t)__shfl_up((long long)a.d0, off), (int64_t)__shfl_up((long long)a.d1, off)};
+}
+// inclusive scan of the lanes' advances
+template <typename T>
+__device__ __forceinline__ Advance wave_scan_advance(Advance a, int lane) {
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const Advance p = shfl_up_advance<T>(a, off);
+        if (lane >= off) a = chain_compose<T>(p, a);
+    }
+    return a;
+}
+
+// A block's weights from memory into LDS, negative ones (not below the bound) as 0.
+template <typename T>
+__device__ __forceinline__ void cdf_load_block(const T *w, int len, T *wbuf, int tid) {
+#pragma unroll
+    for (int q = 0; q < CDF_PER; ++q) {
+        const int e = tid + 256 * q;
+        if (e < len) {
+            const T x = w[e];
+            wbuf[e] = x < (T)0 ? (T)0 : x;
         }
     }
 }
 
-// w[i] = w[i] * (1 / sum) (blas::scal), when the sums succeeded
 template <typename T>
-__global__ __launch_bounds__(256) void cdf_scale_kernel(int64_t n, T *w, const long long *status,
-                                                        const T *inv_total) {
-    if (*status != 0) return;
-    const T inv = *inv_total;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        w[i] = w[i] * inv;
+__global__ __launch_bounds__(256) void cdf_advance_kernel(const T *w, const double *prefix, const CdfMeta *meta,
+                                                          Advance *adv, int *bexp) {
+    __shared__ T wbuf[CDF_BLK];
+    __shared__ Advance wtot[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t b = blockIdx.x, i0 = b * CDF_BLK;
+    const int64_t left = meta->first - i0;
+    const int len = left <= 0 ? 0 : (left < CDF_BLK ? (int)left : CDF_BLK);
+    const int e = chain_exp<T>(chain_bits((T)prefix[b]));
+    if (e != chain_exp<T>(chain_bits((T)prefix[b + 1]))) {  // leaves its binade: the chain kernel's work
+        if (tid == 0) bexp[b] = -1;
+        return;
+    }
+    cdf_load_block(w + i0, len, wbuf, tid);
+    __syncthreads();
+    Advance a{0, 0};
+#pragma unroll
+    for (int q = 0; q < CDF_PER; ++q) {
+        const int i = CDF_PER * tid + q;
+        if (i < len) a = chain_compose<T>(a, chain_term<T>(wbuf[i], e));
+    }
+    a = wave_scan_advance<T>(a, lane);
+    if (lane == 63) wtot[wave] = a;
+    __syncthreads();
+    if (tid == 0) {
+        a = wtot[0];
+#pragma unroll
+        for (int q = 1; q < 4; ++q) a = chain_compose<T>(a, wtot[q]);
+        adv[b] = a;
+        bexp[b] = e;
+    }
 }
 
-__global__ void i64_zero_kernel(long long *p) { *p = 0; }
+// start[b]: the bits of the sum before block b, or -1 when this kernel has
+// written the block's partial sums itself.  adv == nullptr: every block is
+// summed here, and the refused weight looked for here.
+template <typename T>
+__global__ __launch_bounds__(256) void cdf_chain_kernel(int64_t n, T *w, T error_if_below, int64_t nb,
+                                                        const Advance *adv, const int *bexp, int64_t *start,
+                                                        CdfMeta *meta) {
+    __shared__ T wbuf[CDF_BLK], obuf[CDF_BLK];
+    __shared__ Advance wtot[4];
+    __shared__ long long base_sh;
+    __shared__ int cross_sh, stop_sh;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int64_t first = adv ? (int64_t)meta->first : n;
+    int64_t bits = 0;  // the running sum, the same in every thread
+    int64_t b = 0;
+    while (b < nb && b * CDF_BLK < first) {
+        const int e0 = chain_exp<T>(bits);
+        if (adv) {
+            // as many of the next 64 blocks as stay in this binade
+            const int64_t q = b + lane;
+            const bool ok = q < nb && bexp[q] == e0;
+            Advance a = ok ? adv[q] : Advance{chain_cap<T>(), chain_cap<T>()};
+            a = wave_scan_advance<T>(a, lane);
+            const int64_t nx = bits + ((bits & 1) ? a.d1 : a.d0);
+            const unsigned long long out = __ballot(!ok || (uint64_t)nx >= chain_limit<T>(e0));
+            const int f = out ? (int)__builtin_ctzll(out) : 64;
+            const int64_t before = (int64_t)__shfl_up((long long)nx, 1);
+            if (wave == 0 && lane < f) start[q] = lane == 0 ? bits : before;
+            if (f > 0) {
+                bits = (int64_t)__shfl((long long)nx, f - 1);
+                b += f;
+                continue;
+            }
+        }
+        const int64_t i0 = b * CDF_BLK;
+        const int64_t left = first - i0;
+        int len = left < CDF_BLK ? (int)left : CDF_BLK;
+        if (tid == 0) stop_sh = len;
+        __syncthreads();  // also: the last block's obuf has been written out
+#pragma unroll
+        for (int q = 0; q < CDF_PER; ++q) {
+            const int i = tid + 256 * q;
+            if (i < len) {
+                const T x = w[i0 + i];
+                if (!(x >= error_if_below)) atomicMin(&stop_sh, i);
+                wbuf[i] = x < (T)0 ? (T)0 : x;
+            }
+        }
+        __syncthreads();
+        if (stop_sh < len) {
+            len = stop_sh;
+            first = i0 + len;
+        }
+        int pos = 0;  // terms of the block already in the sum
+        while (true) {
+            const int e = chain_exp<T>(bits);
+            const uint64_t limit = chain_limit<T>(e);
+            Advance t[CDF_PER], a{0, 0};
+#pragma unroll
+            for (int q = 0; q < CDF_PER; ++q) {
+                const int i = CDF_PER * tid + q;
+                t[q] = i >= pos && i < len ? chain_term<T>(wbuf[i], e) : Advance{0, 0};
+                a = chain_compose<T>(a, t[q]);
+            }
+            const Advance incl = wave_scan_advance<T>(a, lane);
+            Advance excl = shfl_up_advance<T>(incl, 1);
+            if (lane == 0) excl = Advance{0, 0};
+            if (lane == 63) wtot[wave] = incl;
+            if (tid == 0) cross_sh = CDF_BLK;
+            __syncthreads();
+            Advance pre{0, 0}, tot{0, 0};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (q == wave) pre = tot;
+                tot = chain_compose<T>(tot, wtot[q]);
+            }
+            excl = chain_compose<T>(pre, excl);
+            int64_t cur = bits + ((bits & 1) ? excl.d1 : excl.d0);
+            int cross = CDF_BLK;
+            if ((uint64_t)cur < limit) {
+#pragma unroll
+                for (int q = 0; q < CDF_PER; ++q) {
+                    const int i = CDF_PER * tid + q;
+                    if (i >= pos && i < len && cross == CDF_BLK) {
+                        const int64_t nx = cur + ((cur & 1) ? t[q].d1 : t[q].d0);
+                        if ((uint64_t)nx >= limit) {
+                            cross = i;
+                        } else {
+                            cur = nx;
+                            obuf[i] = chain_value<T>(cur);
+                        }
+                    }
+                }
+                if (cross < CDF_BLK) atomicMin(&cross_sh, cross);
+            }
+            __syncthreads();
+            const int first_cross = cross_sh;
+            if (first_cross == CDF_BLK) {
+                bits += (bits & 1) ? tot.d1 : tot.d0;
+                break;
+            }
+            // the term that leaves the binade: one addition in T
+            if (cross == first_cross) {
+                const T s = chain_value<T>(cur) + wbuf[cross];
+                obuf[cross] = s;
+                base_sh = (long long)chain_bits(s);
+            }
+            __syncthreads();
+            bits = (int64_t)base_sh;
+            pos = first_cross + 1;
+        }
+        __syncthreads();
+        for (int i = tid; i < len; i += 256) w[i0 + i] = obuf[i];
+        if (tid == 0) start[b] = -1;
+        ++b;
+    }
+    if (tid == 0) {
+        const T sum = chain_value<T>(bits);
+        const T floor_sum = (T)sqrt((double)n) * std::numeric_limits<T>::epsilon();
+        const bool ok = first == n && sum >= floor_sum;
+        meta->first = (long long)first;
+        meta->status = first < n ? 1 + (long long)first : (ok ? 0 : -1);
+        meta->inv = ok ? (double)((T)1 / sum) : 1.0;
+    }
+}
+
+// w[i] = partial sum * (1 / sum) (blas::scal), or the plain partial sums
+// (inv = 1) when the sums failed
+template <typename T>
+__global__ __launch_bounds__(256) void cdf_write_kernel(T *w, const int64_t *start, const CdfMeta *meta) {
+    __shared__ T buf[CDF_BLK];
+    __shared__ Advance wtot[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t i0 = (int64_t)blockIdx.x * CDF_BLK;
+    const int64_t left = meta->first - i0;
+    if (left <= 0) return;
+    const int len = left < CDF_BLK ? (int)left : CDF_BLK;
+    const T inv = (T)meta->inv;
+    const int64_t bits = start[blockIdx.x];
+    if (bits < 0) {
+        for (int i = tid; i < len; i += 256) w[i0 + i] = w[i0 + i] * inv;
+        return;
+    }
+    cdf_load_block(w + i0, len, buf, tid);
+    __syncthreads();
+    const int e = chain_exp<T>(bits);
+    Advance t[CDF_PER], a{0, 0};
+#pragma unroll
+    for (int q = 0; q < CDF_PER; ++q) {
+        const int i = CDF_PER * tid + q;
+        t[q] = i < len ? chain_term<T>(buf[i], e) : Advance{0, 0};
+        a = chain_compose<T>(a, t[q]);
+    }
+    const Advance incl = wave_scan_advance<T>(a, lane);
+    Advance excl = shfl_up_advance<T>(incl, 1);
+    if (lane == 0) excl = Advance{0, 0};
+    if (lane == 63) wtot[wave] = incl;
+    __syncthreads();
+    Advance pre{0, 0};
+    for (int q = 0; q < wave; ++q) pre = chain_compose<T>(pre, wtot[q]);
+    excl = chain_compose<T>(pre, excl);
+    int64_t cur = bits + ((bits & 1) ? excl.d1 : excl.d0);
+#pragma unroll
+    for (int q = 0; q < CDF_PER; ++q) {
+        const int i = CDF_PER * tid + q;
+        if (i < len) {
+            cur += (cur & 1) ? t[q].d1 : t[q].d0;
+            buf[i] = chain_value<T>(cur) * inv;
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < len; i += 256) w[i0 + i] = buf[i];
+}
 
 static void next_state(const rbx_rng_state *state, uint64_t counters, rbx_rng_state *next) {
     if (next == nullptr) return;
@@ -303,19 +530,35 @@ template <typename T>
 static void weights_to_cdf_impl(int64_t n, T *w, T error_if_below, hipStream_t st) {
     RBX_REQUIRE(n >= 0);
     RBX_REQUIRE(n == 0 || w != nullptr);
-    long long *status = (long long *)scratch(SCRATCH_SMALL, 2 * sizeof(long long), st);
-    T *inv_total = (T *)(status + 1);
-    hipLaunchKernelGGL(i64_zero_kernel, dim3(1), dim3(1), 0, st, status);
-    hipLaunchKernelGGL((weights_to_cdf_kernel<T>), dim3(1), dim3(256), 0, st, n, w, error_if_below, status,
-                       inv_total);
-    int64_t blocks = (n + 255) / 256;
-    if (blocks > 4096) blocks = 4096;
-    if (blocks > 0)
-        hipLaunchKernelGGL((cdf_scale_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, st, n, w,
-                           (const long long *)status, (const T *)inv_total);
-    RBX_HIP(hipGetLastError());
+    const int64_t nb = (n + CDF_BLK - 1) / CDF_BLK;
+    RBX_REQUIRE(nb < (1ll << 31));
+    const bool direct = nb <= CDF_DIRECT;
+    // meta | start | adv | prefix | bexp | bbad
+    char *ws = (char *)scratch(SCRATCH_SMALL, 64 + (size_t)nb * (8 + 16 + 8 + 4 + 4) + 8, st);
+    CdfMeta *meta = (CdfMeta *)ws;
+    int64_t *start = (int64_t *)(ws + 64);
+    Advance *adv = (Advance *)(start + nb);
+    double *bsum = (double *)(adv + nb);
+    int *bexp = (int *)(bsum + nb + 1), *bbad = bexp + nb;
+    {
+        ProfScope prof("weights_to_cdf_kernel", st);
+        const dim3 grid((unsigned)nb);
+        if (!direct) {
+            hipLaunchKernelGGL((cdf_sums_kernel<T>), grid, dim3(256), 0, st, n, (const T *)w, error_if_below, bsum,
+                               bbad);
+            hipLaunchKernelGGL(cdf_guess_kernel, dim3(1), dim3(1024), 0, st, n, nb, bsum, (const int *)bbad, meta);
+            hipLaunchKernelGGL((cdf_advance_kernel<T>), grid, dim3(256), 0, st, (const T *)w, (const double *)bsum,
+                               (const CdfMeta *)meta, adv, bexp);
+        }
+        hipLaunchKernelGGL((cdf_chain_kernel<T>), dim3(1), dim3(256), 0, st, n, w, error_if_below, nb,
+                           direct ? (const Advance *)nullptr : (const Advance *)adv, (const int *)bexp, start, meta);
+        if (nb > 0)
+            hipLaunchKernelGGL((cdf_write_kernel<T>), grid, dim3(256), 0, st, w, (const int64_t *)start,
+                               (const CdfMeta *)meta);
+        RBX_HIP(hipGetLastError());
+    }
     long long h = 0;
-    RBX_HIP(hipMemcpyAsync(&h, status, sizeof(h), hipMemcpyDeviceToHost, st));
+    RBX_HIP(hipMemcpyAsync(&h, &meta->status, sizeof(h), hipMemcpyDeviceToHost, st));
     RBX_HIP(hipStreamSynchronize(st));
     if (h > 0)
         RBX_FAIL(RBX_INVALID_ARG, "weights_to_cdf: w[%lld] is below error_if_below = %e", h - 1,

@@ -113,6 +113,36 @@ def test_weights_to_cdf_blocks_bit_exact(rb, orc, dtype, n):
     assert np.array_equal(host(wd), ref)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [1, 2047, 8192, 8193, 150_001])
+@pytest.mark.parametrize("kind", ["ties", "powers", "decay", "subnormal", "spikes", "constant"])
+def test_weights_to_cdf_binades_bit_exact(rb, orc, dtype, n, kind):
+    """Weights that make the running sum round half way, change binade often,
+    start subnormal or stop growing: bit for bit the oracle's sequential sums,
+    with one workgroup alone (up to 8192 weights) and with composed blocks."""
+    rng = np.random.default_rng(n + len(kind))
+    tiny = np.finfo(dtype).tiny
+    if kind == "ties":  # halves of the sum's spacing, for many binades
+        w = rng.integers(0, 8, n) * 0.125 + np.ldexp(rng.integers(0, 2, n), -rng.integers(0, 60, n))
+    elif kind == "powers":
+        w = np.ldexp(1.0 + rng.integers(0, 2, n), rng.integers(-60, 20, n))
+    elif kind == "decay":
+        w = rng.random(n) * np.exp2(-np.arange(n) * (200.0 / n)) + 1e-3
+    elif kind == "subnormal":  # then normal, so that the total is accepted
+        w = rng.random(n) * float(tiny) * 4
+        w[-1:] = 1e6
+    elif kind == "spikes":
+        w = np.where(rng.random(n) < 1e-3, np.ldexp(1.0, rng.integers(0, 30, n)), rng.random(n) * 1e-3) + 1e-6
+    else:
+        w = np.full(n, 0.1)
+    w = w.astype(dtype)
+    wd = torch.from_numpy(w.copy()).to(DEV)
+    rb.weights_to_cdf(n, wd)
+    ref, st = orc.weights_to_cdf(w)
+    assert st == 0
+    assert np.array_equal(host(wd), ref)
+
+
 def test_weights_to_cdf_error_in_a_later_block(rb, orc):
     """A weight below error_if_below at index 5000 (the third block): the
     entries before it hold the sequential partial sums, the rest are
