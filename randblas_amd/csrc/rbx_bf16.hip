@@ -797,952 +797,6 @@ static void bf16_split_sketch(char layout, char opS, char opA, int64_t d, int64_
     }
 }
 
-// Scratch of the wide-tile paths, or nullptr when the device cannot provide
-// it: the caller then runs the tile kernels, which need none.
-static void *wide_scratch(size_t bytes, hipStream_t stream) {
-    try {
-        return scratch(SCRATCH_BF16, bytes, stream);
-    } catch (const Fail &f) {
-        if (f.st != RBX_OUT_OF_MEMORY) throw;
-        clear_error();
-        return nullptr;
-    }
-}
-
-// ---------------------------------------------------------------- wide FP32 tiles
-// The plain FP32 fused sketch C = alpha * X * Y + beta * C with X the
-// generated operator (M x K, rows along K) and Y the dense operand (K x N),
-// for large interior shapes: the pair kernel's structure with FP32 operands.
-// Y is packed once into FP32 fragment runs; one 512-thread workgroup per
-// (64-row block, 256 CB-column block, K-split) generates each 32-deep
-// operator chunk once into LDS (exact FP32 values, as the other kernels) and
-// applies it to all of the block's columns with v_mfma_f32_32x32x2f32, so
-// every operator entry is generated once per 1024 columns (CB = 4; 512 / 256
-// for narrower outputs) instead of once per 256.  Partials go to scratch and
-// are combined by bf16_reduce_kernel (FP64, split order).
-//
-// Packed Y: for 32-column block cb and 16-deep K step s, lane l's eight
-// floats are Y[16 s + 2 q + l / 32][32 cb + l % 32], q = 0..7 (the B
-// operands of the step's eight MFMAs), at ((cb * KS + s) * 64 + l) * 8 + q.
-// The operator chunk in LDS uses the same order within each row: k = 16 st +
-// kk sits at 16 st + 8 (kk % 2) + kk / 2.
-constexpr int FW_LDK = 36;  // 32 k per row + 4 pad (floats)
-// Largest packed operand + partials the wide kernels take in scratch; bigger
-// problems run on the tile kernels, which need none.
-constexpr size_t WIDE_SCRATCH_MAX = 16ull << 30;
-static size_t align256b(size_t x) { return (x + 255) / 256 * 256; }
-
-__device__ __forceinline__ int fw_pos(int k) { return (k & ~15) + 8 * (k & 1) + ((k & 15) >> 1); }
-
-// Tail columns of the wide kernels: up to WIDE_TAIL output columns past the
-// last whole tile (the right-hand side of [A b], a ragged edge) are formed by
-// the threads that generate the operator, from the four entries each holds
-// in registers per chunk, with VALU FMAs: the operator is generated once for
-// the tiles and the tail together.  The generator of operator rows along K
-// holds one row's four consecutive k (one accumulator per column); the one of
-// counters along the rows holds four rows at one k (four per column).  The
-// dense values of chunk c + 1 are loaded right after chunk c's are used, into
-// the same registers, so they have a whole chunk's MFMAs to arrive (a copy
-// from a second buffer would wait for the load at once).  TW
-// columns are always loaded and accumulated (TW = 1, or 4 with the unused
-// ones repeating the last real column), so the chunk loop has no branch: a
-// load under a branch would make the compiler's memory-counter waits for
-// the MFMA operands conservative.
-constexpr int WIDE_TAIL = 4;
-// The tail's columns: dense column j's element k at col[j][k * rs[j]], its
-// output's element i at out[j][i * ors[j]]; entries nt .. WIDE_TAIL - 1 of
-// col / rs repeat entry nt - 1.
-template <typename T>
-struct TailCols {
-    const T *col[WIDE_TAIL];
-    int64_t rs[WIDE_TAIL];
-    T *out[WIDE_TAIL];
-    int64_t ors[WIDE_TAIL];
-    int nt;
-};
-template <typename T, bool ROWS, int TW>
-struct WideTail {
-    static constexpr int R = ROWS ? 4 : 1;  // output rows per thread
-    static constexpr int E = ROWS ? 1 : 4;  // dense values per column per chunk
-    T acc[TW][R];
-    T cur[TW][E];  // the dense values of the chunk being generated
-
-    __device__ __forceinline__ void zero() {
-#pragma unroll
-        for (int j = 0; j < TW; ++j)
-#pragma unroll
-            for (int r = 0; r < R; ++r) acc[j][r] = (T)0;
-    }
-    // cur = dense values of the thread's k (k .. k + E - 1), every tail column
-    __device__ __forceinline__ void load(const TailCols<T> &tc, int64_t k) {
-#pragma unroll
-        for (int j = 0; j < TW; ++j)
-#pragma unroll
-            for (int e = 0; e < E; ++e) cur[j][e] = tc.col[j][(k + e) * tc.rs[j]];
-    }
-    // acc += the chunk's operator entries (ent[0..3]) times cur
-    __device__ __forceinline__ void step(const T (&ent)[4]) {
-#pragma unroll
-        for (int j = 0; j < TW; ++j) {
-            if constexpr (ROWS) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[j][r] = fma(ent[r], cur[j][0], acc[j][r]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc[j][0] = fma(ent[e], cur[j][e], acc[j][0]);
-            }
-        }
-    }
-    // The workgroup's 64 x nt partial into out[j * M + row], out = the
-    // split's tail partials shifted to the block's first row.  Rows along K:
-    // the eight threads of a row are adjacent lanes (butterfly).  Counters
-    // along the rows: lanes l, l ^ 16, l ^ 32, l ^ 48 of a wave share rows
-    // (butterfly), then the eight waves are summed in order through `red`
-    // (8 * TW * 64 values of LDS free for reuse).  Every thread of the
-    // workgroup calls this (it has a barrier).
-    __device__ __forceinline__ void finish(int nt, int tid, int frow, int fcell, T *red, T *out, int64_t M) {
-        const int lane = tid & 63, wave = tid >> 6;
-        if constexpr (!ROWS) {
-#pragma unroll
-            for (int j = 0; j < TW; ++j) {
-                T v = acc[j][0];
-                v += __shfl_xor(v, 1);
-                v += __shfl_xor(v, 2);
-                v += __shfl_xor(v, 4);
-                if (j < nt && fcell == 0) out[j * M + frow] = v;
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < TW; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    T v = acc[j][r];
-                    v += __shfl_xor(v, 16);
-                    v += __shfl_xor(v, 32);
-                    if (lane < 16) red[(wave * TW + j) * 64 + frow + r] = v;
-                }
-            __syncthreads();
-            if (tid < 64 * nt) {
-                const int j = tid >> 6, row = tid & 63;
-                T v = red[j * 64 + row];
-#pragma unroll
-                for (int w = 1; w < BF_FTHR / 64; ++w) v += red[(w * TW + j) * 64 + row];
-                out[j * M + row] = v;
-            }
-        }
-    }
-};
-
-// The tail's outputs: out[j][i * ors[j]] = alpha * (sum over splits of
-// tpart[(s * nt + j) * M + i]) + beta * out, FP64 sums.  G threads per output
-// entry: G = 1 sums the splits in order; G = 64 (many splits) has lane l sum
-// splits l, l + 64, ..., then a butterfly (a fixed order).
-template <typename T, int G>
-__global__ __launch_bounds__(256) void wide_tail_reduce_kernel(const T *tpart, int nS, int64_t M, TailCols<T> tc,
-                                                               double alpha, double beta) {
-    const int nt = tc.nt;
-    const int g = threadIdx.x % G;
-    const int64_t e = (int64_t)blockIdx.x * (256 / G) + threadIdx.x / G;
-    if (e >= M * nt) return;  // uniform per group
-    const int64_t i = e % M;
-    const int j = (int)(e / M);
-    double v = 0.0;
-    for (int s = g; s < nS; s += G) v += (double)tpart[((int64_t)s * nt + j) * M + i];
-    if constexpr (G == 64) {
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
-        if (g != 0) return;
-    }
-    T *c = nullptr;
-    int64_t rs = 0;
-#pragma unroll
-    for (int q = 0; q < WIDE_TAIL; ++q)
-        if (q == j) {
-            c = tc.out[q];
-            rs = tc.ors[q];
-        }
-    c += i * rs;
-    double out = alpha * v;
-    if (beta != 0.0) out += beta * (double)(*c);
-    *c = (T)out;
-}
-
-template <typename T>
-static void launch_tail_reduce(const T *tpart, int nS, int64_t M, const TailCols<T> &tc, double alpha, double beta,
-                               hipStream_t st) {
-    const int64_t n = M * tc.nt;
-    if (nS <= 16)
-        hipLaunchKernelGGL((wide_tail_reduce_kernel<T, 1>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, tpart,
-                           nS, M, tc, alpha, beta);
-    else
-        hipLaunchKernelGGL((wide_tail_reduce_kernel<T, 64>), dim3((unsigned)((n + 3) / 4)), dim3(256), 0, st, tpart,
-                           nS, M, tc, alpha, beta);
-}
-
-
-// How many of the columns past the whole tiles, [Nf, N), the wide kernel
-// forms in its tail, the last nt of them (0: none; the others go to the
-// caller as a rest problem), or -1 when the problem cannot run on the wide
-// kernel.  The widest tiles (cb = 4) have no registers to spare for a tail.
-// A problem whose last column lives apart (xD / xC) needs that column in the
-// tail and whole 64-row blocks (a rest problem cannot carry it).
-static int wide_tail_cols(const GemmProblem &pb, int64_t Mf, int64_t Nf, int cb) {
-    const int64_t rem = pb.N - Nf;
-    if (pb.xD != nullptr || pb.xC != nullptr) {
-        if (pb.M != Mf || cb == 4 || rem < 1) return -1;
-        return rem <= WIDE_TAIL ? (int)rem : 1;
-    }
-    return (rem >= 1 && rem <= WIDE_TAIL && cb < 4) ? (int)rem : 0;
-}
-
-// The tail's columns N - nt .. N - 1: dense column c at D[k * drs + c * dcs],
-// output at C[i * crs + c * ccs], the last one at xD / xC when given.
-template <typename T>
-static TailCols<T> wide_tail_io(const GemmProblem &pb, int nt) {
-    TailCols<T> tc{};
-    tc.nt = nt;
-    for (int j = 0; j < WIDE_TAIL; ++j) {
-        if (j >= nt) {  // unused slots repeat the last column (loaded, never written)
-            tc.col[j] = tc.col[nt - 1];
-            tc.rs[j] = tc.rs[nt - 1];
-            tc.out[j] = nullptr;
-            tc.ors[j] = 0;
-            continue;
-        }
-        const int64_t c = pb.N - nt + j;
-        const bool last = c == pb.N - 1;
-        tc.col[j] = (last && pb.xD) ? (const T *)pb.xD : (const T *)pb.D + c * pb.dcs;
-        tc.rs[j] = (last && pb.xD) ? pb.xdrs : pb.drs;
-        tc.out[j] = (last && pb.xC) ? (T *)pb.xC : (T *)pb.C + c * pb.ccs;
-        tc.ors[j] = (last && pb.xC) ? pb.xcrs : pb.crs;
-    }
-    return tc;
-}
-
-// Unit-stride K: one workgroup per (32-column block, 256-deep K range), the
-// tile staged through LDS (as split_kunit_kernel).
-template <bool VEC>
-__global__ __launch_bounds__(256) void pack_f32_kunit_kernel(const float *A, int64_t cs, int64_t K, int64_t N,
-                                                             int64_t Kp, float *packed) {
-    __shared__ __attribute__((aligned(16))) float tile[32][SPL_LD];
-    const int tid = threadIdx.x;
-    const int64_t KS = Kp / 16;
-    const int64_t cb = blockIdx.y;
-    const int64_t kt0 = (int64_t)blockIdx.x * SPL_KT;
-    const int q4 = tid & 63, c0 = tid >> 6;
-    const int64_t k = kt0 + 4 * q4;
-    float4 v[8];
-#pragma unroll
-    for (int p = 0; p < 8; ++p) {
-        const int64_t j = cb * 32 + c0 + 4 * p;
-        const float *src = A + k + j * cs;
-        if (VEC && j < N && k + 3 < K) {
-            v[p] = *(const float4 *)src;
-        } else {
-            v[p].x = (j < N && k < K) ? src[0] : 0.0f;
-            v[p].y = (j < N && k + 1 < K) ? src[1] : 0.0f;
-            v[p].z = (j < N && k + 2 < K) ? src[2] : 0.0f;
-            v[p].w = (j < N && k + 3 < K) ? src[3] : 0.0f;
-        }
-    }
-#pragma unroll
-    for (int p = 0; p < 8; ++p) *(float4 *)&tile[c0 + 4 * p][4 * q4] = v[p];
-    __syncthreads();
-    const int64_t steps = (KS - kt0 / 16) < 16 ? (KS - kt0 / 16) : 16;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int task = tid + 256 * i;
-        const int st = task >> 6, l = task & 63;
-        if (st >= steps) break;
-        const float *src = &tile[l & 31][16 * st + (l >> 5)];
-        float4 lo, hi;
-        lo.x = src[0]; lo.y = src[2]; lo.z = src[4]; lo.w = src[6];
-        hi.x = src[8]; hi.y = src[10]; hi.z = src[12]; hi.w = src[14];
-        float *dst = packed + ((cb * KS + kt0 / 16 + st) * 64 + l) * 8;
-        *(float4 *)dst = lo;
-        *(float4 *)(dst + 4) = hi;
-    }
-}
-
-// Any strides: one thread per packed float.
-__global__ __launch_bounds__(256) void pack_f32_kernel(const float *A, int64_t rs, int64_t cs, int64_t K, int64_t N,
-                                                       int64_t Kp, int64_t Np, float *packed) {
-    const int64_t KS = Kp / 16, total = (Np / 32) * KS * 512;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
-        const int q = (int)(e & 7), l = (int)((e >> 3) & 63);
-        const int64_t run = e >> 9, s = run % KS, cb = run / KS;
-        const int64_t k = 16 * s + 2 * q + (l >> 5), j = 32 * cb + (l & 31);
-        packed[e] = (k < K && j < N) ? A[k * rs + j * cs] : 0.0f;
-    }
-}
-
-struct F32WideProblem {
-    int64_t M, N, Kp;  // M, N multiples of 64 / the tile width; Kp of the 32-deep chunk
-    GenMap g;
-    const float *packed;
-    float *part;   // nS x M x N, row-major
-    int64_t kw;    // K per split (multiple of 32)
-    int nMB, nNB, nS;
-    // tail columns (TAIL instantiations), partials at
-    // tpart[(split * tc.nt + j) * M + row]
-    TailCols<float> tc;
-    float *tpart;
-};
-
-template <bool GAUSS, bool ROWS, int CB, int TW>
-__global__ __launch_bounds__(BF_FTHR, 1) void f32_wide_kernel(F32WideProblem pb) {
-    constexpr int RB = 2, MT = 64, NT = 256 * CB;  // CB 32-column blocks per wave
-    __shared__ __attribute__((aligned(16))) float Ss[2][MT * FW_LDK];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int W = pb.nMB * pb.nNB * pb.nS;
-    const int L = blockIdx.x;
-    const int t = (W % 8 == 0) ? (L % 8) * (W / 8) + L / 8 : L;  // XCD-aware: one K-split per XCD run
-    const int mb = t % pb.nMB;
-    const int rest = t / pb.nMB;
-    const int nb = rest % pb.nNB;
-    const int sp = rest / pb.nNB;
-    const int64_t m0 = (int64_t)mb * MT, n0 = (int64_t)nb * NT;
-    const int64_t kbeg = (int64_t)sp * pb.kw;
-    int64_t kend = kbeg + pb.kw;
-    if (kend > pb.Kp) kend = pb.Kp;
-    const int nchunks = (int)((kend - kbeg) / 32);
-    const GenMap g = pb.g;
-
-    f32x16 acc[RB][CB];
-#pragma unroll
-    for (int i = 0; i < RB; ++i)
-#pragma unroll
-        for (int j = 0; j < CB; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    const int64_t wcol = n0 + wave * (32 * CB);
-    const int64_t KS = pb.Kp / 16;
-    const float *bbase = pb.packed + ((wcol >> 5) * KS * 64 + lane) * 8;
-    const int64_t bblk = KS * 512;  // floats between column blocks
-    const int64_t s_first = kbeg / 16, s_last = kend / 16 - 1;
-
-    // generator, operator rows along K (!ROWS): thread owns cell (tid & 7) of
-    // operator row tid / 8; counters along the rows (ROWS): thread owns rows
-    // 4 (tid & 15) .. + 3 of operator column tid / 16 of the chunk
-    const int frow = ROWS ? 4 * (tid & 15) : tid >> 3, fcell = ROWS ? tid >> 4 : tid & 7;
-    const uint64_t foff = ROWS ? (uint64_t)((g.a_off + kbeg + fcell) * g.P + ((g.b_off + m0) >> 2) + (tid & 15))
-                               : (uint64_t)((g.a_off + m0 + frow) * g.P + ((g.b_off + kbeg) >> 2) + fcell);
-    const uint64_t fstep = ROWS ? 32 * (uint64_t)g.P : 8;  // counters per chunk
-    // tail columns: only the first column block's workgroups form them
-    // (cb < 4: the output has one column block, nb == 0)
-    WideTail<float, ROWS, TW == 0 ? 1 : TW> tl;
-    const int64_t tk = kbeg + (ROWS ? fcell : 4 * fcell);  // the thread's first k of chunk 0
-    if constexpr (TW > 0) {
-        tl.zero();
-        tl.load(pb.tc, tk);
-    }
-    auto gen_chunk = [&](int c, float *lds) {
-        const float4 v = gen4(GAUSS, ctr_add(g.ctr, foff + fstep * (uint64_t)c), g.k0, g.k1);
-        const float ent[4] = {entry_value<float>(v.x, GAUSS), entry_value<float>(v.y, GAUSS),
-                              entry_value<float>(v.z, GAUSS), entry_value<float>(v.w, GAUSS)};
-        if constexpr (ROWS) {
-            const int pos = fw_pos(fcell);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) lds[(frow + e) * FW_LDK + pos] = ent[e];
-        } else {
-            float *row = lds + frow * FW_LDK;
-            const int k0 = 4 * fcell;  // even: k0, k0 + 2 share the even half; k0 + 1, k0 + 3 the odd half
-            float2 ev, od;
-            ev.x = ent[0];
-            od.x = ent[1];
-            ev.y = ent[2];
-            od.y = ent[3];
-            *(float2 *)(row + fw_pos(k0)) = ev;
-            *(float2 *)(row + fw_pos(k0 + 1)) = od;
-        }
-        if constexpr (TW > 0) {
-            tl.step(ent);
-            tl.load(pb.tc, tk + 32 * (int64_t)(c + 1 < nchunks ? c + 1 : c));  // the next chunk's
-        }
-    };
-
-    // B operands of one step: lo = q 0..3, hi = q 4..7 of block j
-    float4 blo[CB], bhi[CB];
-#pragma unroll
-    for (int j = 0; j < CB; ++j) {
-        blo[j] = *(const float4 *)(bbase + j * bblk + s_first * 512);
-        bhi[j] = *(const float4 *)(bbase + j * bblk + s_first * 512 + 4);
-    }
-
-    auto step = [&](const float *S, int ks, int64_t s_next) {
-        __builtin_amdgcn_s_setprio(1);
-        float4 alo[RB], ahi[RB];
-#pragma unroll
-        for (int i = 0; i < RB; ++i) {
-            const float *src = S + (32 * i + (lane & 31)) * FW_LDK + 16 * ks + 8 * (lane >> 5);
-            alo[i] = *(const float4 *)src;
-            ahi[i] = *(const float4 *)(src + 4);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int j = 0; j < CB; ++j)
-#pragma unroll
-                for (int i = 0; i < RB; ++i)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(f4_get(alo[i], q), f4_get(blo[j], q), acc[i][j],
-                                                                     0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < CB; ++j) blo[j] = *(const float4 *)(bbase + j * bblk + s_next * 512);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int j = 0; j < CB; ++j)
-#pragma unroll
-                for (int i = 0; i < RB; ++i)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(f4_get(ahi[i], q), f4_get(bhi[j], q), acc[i][j],
-                                                                     0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < CB; ++j) bhi[j] = *(const float4 *)(bbase + j * bblk + s_next * 512 + 4);
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_setprio(0);
-    };
-
-    const bool late = (wave & 4) != 0;
-    gen_chunk(0, Ss[0]);
-    __syncthreads();
-    if constexpr (TW == 0) {
-        for (int c = 0; c < nchunks; ++c) {
-            const float *S = Ss[c & 1];
-            float *Sn = Ss[(c + 1) & 1];
-            const int64_t s0 = s_first + 2 * c;
-            const bool more = c + 1 < nchunks;
-            if (more && !late) gen_chunk(c + 1, Sn);
-            step(S, 0, s0 + 1);
-            step(S, 1, s0 + 2 > s_last ? s_last : s0 + 2);
-            if (more && late) gen_chunk(c + 1, Sn);
-            __syncthreads();
-        }
-    } else {
-        // with a tail: one loop per wave role and the last chunk peeled, so
-        // no branch surrounds the tail's loads inside a loop (the compiler's
-        // memory-counter waits for the MFMA operands stay exact)
-        const int last = nchunks - 1;
-        if (!late) {
-            for (int c = 0; c < last; ++c) {
-                gen_chunk(c + 1, Ss[(c + 1) & 1]);
-                step(Ss[c & 1], 0, s_first + 2 * c + 1);
-                step(Ss[c & 1], 1, s_first + 2 * c + 2);
-                __syncthreads();
-            }
-        } else {
-            for (int c = 0; c < last; ++c) {
-                step(Ss[c & 1], 0, s_first + 2 * c + 1);
-                step(Ss[c & 1], 1, s_first + 2 * c + 2);
-                gen_chunk(c + 1, Ss[(c + 1) & 1]);
-                __syncthreads();
-            }
-        }
-        step(Ss[last & 1], 0, s_first + 2 * last + 1);
-        step(Ss[last & 1], 1, s_last);
-        __syncthreads();
-    }
-
-    if constexpr (TW > 0)
-        if (nb == 0) tl.finish(pb.tc.nt, tid, frow, fcell, &Ss[0][0], pb.tpart + (int64_t)sp * pb.tc.nt * pb.M + m0, pb.M);
-
-    float *P = pb.part + (int64_t)sp * pb.M * pb.N;
-#pragma unroll
-    for (int i = 0; i < RB; ++i)
-#pragma unroll
-        for (int j = 0; j < CB; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int64_t gi = m0 + i * 32 + out_row32(lane, r);
-                const int64_t gj = wcol + j * 32 + (lane & 31);
-                P[gi * pb.N + gj] = acc[i][j][r];
-            }
-}
-
-// Launches a wide-tile FP32 kernel instantiation by (family, orientation).
-template <int CB, int TW>
-static void launch_f32_wide(bool gauss, bool rows, dim3 grid, const F32WideProblem &w, hipStream_t st) {
-    if (gauss && rows) hipLaunchKernelGGL((f32_wide_kernel<true, true, CB, TW>), grid, dim3(BF_FTHR), 0, st, w);
-    else if (gauss) hipLaunchKernelGGL((f32_wide_kernel<true, false, CB, TW>), grid, dim3(BF_FTHR), 0, st, w);
-    else if (rows) hipLaunchKernelGGL((f32_wide_kernel<false, true, CB, TW>), grid, dim3(BF_FTHR), 0, st, w);
-    else hipLaunchKernelGGL((f32_wide_kernel<false, false, CB, TW>), grid, dim3(BF_FTHR), 0, st, w);
-}
-// by tail width: none, one column, two to four
-template <int CB>
-static void launch_f32_wide_tw(bool gauss, bool rows, int nt, dim3 grid, const F32WideProblem &w, hipStream_t st) {
-    if (nt == 0) launch_f32_wide<CB, 0>(gauss, rows, grid, w, st);
-    else if (nt == 1) launch_f32_wide<CB, 1>(gauss, rows, grid, w, st);
-    else launch_f32_wide<CB, WIDE_TAIL>(gauss, rows, grid, w, st);
-}
-
-// Runs the part of an FP32 fused-sketch problem that the wide kernel covers
-// (rows [0, Mf) x columns [0, Nf), Mf and Nf multiples of 64 and 1024) and
-// returns in rest[] the remaining sub-problems, for the caller's tile kernels
-// (-1: the wide kernel does not apply and nothing ran).
-int f32_wide_run(const GemmProblem &pb, GemmProblem rest[2], hipStream_t stream) {
-    if (!pb.gen_is_x || pb.sbuf != nullptr || (pb.g.b_off & 3) != 0) return -1;
-    if (pb.K < 1024 || pb.K % 32 != 0 || pb.M < 64 || pb.N < 256) return -1;
-    // the widest tile (1024, 512 or 256 columns) the output holds; the
-    // columns past the last whole tile run on the tile kernels
-    const int cb = pb.N >= 1024 ? 4 : (pb.N >= 512 ? 2 : 1);
-    const int64_t NT = 256 * cb;
-    const int64_t Mf = pb.M / 64 * 64, Nf = pb.N / NT * NT, K = pb.K;
-    const int nt = wide_tail_cols(pb, Mf, Nf, cb);
-    if (nt < 0) return -1;
-    F32WideProblem w{};
-    w.M = Mf;
-    w.N = Nf;
-    w.Kp = K;
-    w.g = pb.g;
-    w.nMB = (int)(Mf / 64);
-    w.nNB = (int)(Nf / NT);
-    int64_t kw = 4096;
-    const int64_t tiles = (int64_t)w.nMB * w.nNB;
-    const int64_t want = (4 * (int64_t)num_cus() + tiles - 1) / tiles;
-    const int64_t kw_fill = (K + want - 1) / want;
-    if (kw_fill < kw) kw = kw_fill;
-    kw = (kw + 31) / 32 * 32;
-    if (kw < 32) kw = 32;
-    // short K over a large output: thin K-splits would cost more partial
-    // traffic than the tile kernels' plain pass (measured at 4096 x 1024,
-    // K = 1024)
-    if (K < 2048 && kw < 256 && Mf * Nf > (1ll << 20)) return -1;
-    w.kw = kw;
-    w.nS = (int)((K + kw - 1) / kw);
-    if ((int64_t)w.nMB * w.nNB * w.nS >= (1ll << 31)) return -1;
-    const size_t packed_bytes = align256b((size_t)safe_mul(K, Nf) * 4);
-    const size_t part_bytes = align256b((size_t)safe_mul(safe_mul(w.nS, Mf), Nf) * 4);
-    const size_t tail_bytes = (size_t)w.nS * nt * Mf * 4;
-    // the tile kernels need no scratch
-    if (packed_bytes + part_bytes + tail_bytes > WIDE_SCRATCH_MAX) return -1;
-    char *ws = (char *)wide_scratch(packed_bytes + part_bytes + tail_bytes, stream);
-    if (ws == nullptr) return -1;
-    w.packed = (const float *)ws;
-    w.part = (float *)(ws + packed_bytes);
-    const float *Y = (const float *)pb.D;
-    w.tc = wide_tail_io<float>(pb, nt);
-    w.tpart = (float *)(ws + packed_bytes + part_bytes);
-    {
-        ProfScope prof("f32_pack_kernel", stream);
-        if (pb.drs == 1) {
-            const int64_t kt = (K + SPL_KT - 1) / SPL_KT;
-            RBX_REQUIRE(kt < (1ll << 31) && Nf / 32 <= 65535);
-            const dim3 grid((unsigned)kt, (unsigned)(Nf / 32));
-            if (pb.dcs % 4 == 0 && ((uintptr_t)Y & 15) == 0)
-                hipLaunchKernelGGL(pack_f32_kunit_kernel<true>, grid, dim3(256), 0, stream, Y, pb.dcs, K, Nf, K,
-                                   (float *)w.packed);
-            else
-                hipLaunchKernelGGL(pack_f32_kunit_kernel<false>, grid, dim3(256), 0, stream, Y, pb.dcs, K, Nf, K,
-                                   (float *)w.packed);
-        } else {
-            hipLaunchKernelGGL(pack_f32_kernel, dim3(65536), dim3(256), 0, stream, Y, pb.drs, pb.dcs, K, Nf, K, Nf,
-                               (float *)w.packed);
-        }
-        RBX_HIP(hipGetLastError());
-    }
-    {
-        ProfScope prof("f32_wide_kernel", stream);
-        const dim3 grid((unsigned)(w.nMB * w.nNB * w.nS));
-        const bool rows = w.g.b_along_rows != 0;
-        const bool gauss = w.g.gauss != 0;
-        if (cb == 4) launch_f32_wide<4, 0>(gauss, rows, grid, w, stream);  // no tail at cb = 4
-        else if (cb == 2) launch_f32_wide_tw<2>(gauss, rows, nt, grid, w, stream);
-        else launch_f32_wide_tw<1>(gauss, rows, nt, grid, w, stream);
-        RBX_HIP(hipGetLastError());
-    }
-    {
-        ProfScope prof("f32_reduce_kernel", stream);
-        const dim3 grid = reduce_grid(Mf, Nf);
-        hipLaunchKernelGGL((bf16_reduce_kernel<float, float>), grid, dim3(256), 0, stream, (const float *)w.part, w.nS, Mf, Nf,
-                           pb.alpha, pb.beta, (float *)pb.C, pb.crs, pb.ccs);
-        if (nt > 0)
-            launch_tail_reduce<float>(w.tpart, w.nS, Mf, w.tc, pb.alpha, pb.beta, stream);
-        RBX_HIP(hipGetLastError());
-    }
-    int nr = 0;
-    if (pb.M > Mf) {  // rows [Mf, M) x all columns: the operator's rows advance along a
-        GemmProblem r = pb;
-        r.M = pb.M - Mf;
-        if (pb.g.b_along_rows) r.g.b_off = pb.g.b_off + Mf;
-        else r.g.a_off = pb.g.a_off + Mf;
-        r.C = (float *)pb.C + Mf * pb.crs;
-        rest[nr++] = r;
-    }
-    if (pb.N - nt > Nf) {  // rows [0, Mf) x columns [Nf, N - nt)
-        GemmProblem r = pb;
-        r.xD = nullptr;
-        r.xC = nullptr;
-        r.M = Mf;
-        r.N = pb.N - nt - Nf;
-        r.D = Y + Nf * pb.dcs;
-        r.C = (float *)pb.C + Nf * pb.ccs;
-        rest[nr++] = r;
-    }
-    return nr;
-}
-
-// ---------------------------------------------------------------- wide FP64 tiles
-// The plain FP64 fused sketch on the same plan as f32_wide_kernel, with
-// v_mfma_f64_16x16x4f64: 64 x 128 CB tiles, 512 columns at CB = 4 (the FP64
-// accumulators of a 64 x 1024 tile would not fit), so each operator entry is
-// generated once per 512 columns (the tile kernels: once per 256).  Packed Y: for 16-column block jb
-// and 16-deep step s, lane l's four doubles are Y[16 s + 4 q + l / 16][16 jb +
-// l % 16], q = 0..3, at ((jb * KS + s) * 64 + l) * 4 + q; the operator chunk
-// in LDS holds k = 16 st + kk at 16 st + 4 (kk % 4) + kk / 4.  Partials are
-// FP64; K-splits are longer (FP64 chains need no bounding).
-constexpr int DW_LDK = 36;  // doubles per LDS row: 32 k + 4 pad
-typedef double f64x4 __attribute__((ext_vector_type(4)));
-typedef double f64x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ int dw_pos(int k) { return (k & ~15) + 4 * (k & 3) + ((k & 15) >> 2); }
-
-__global__ __launch_bounds__(256) void pack_f64_kernel(const double *A, int64_t rs, int64_t cs, int64_t K, int64_t N,
-                                                       int64_t Kp, int64_t Np, double *packed) {
-    const int64_t KS = Kp / 16, total = (Np / 16) * KS * 256;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
-        const int q = (int)(e & 3), l = (int)((e >> 2) & 63);
-        const int64_t run = e >> 8, s = run % KS, jb = run / KS;
-        const int64_t k = 16 * s + 4 * q + (l >> 4), j = 16 * jb + (l & 15);
-        packed[e] = (k < K && j < N) ? A[k * rs + j * cs] : 0.0;
-    }
-}
-
-// Unit-stride K (column-major A): one workgroup per (16-column block, 256-deep
-// K range); each column's 256 doubles are 16 threads' contiguous 16-byte
-// loads, staged through LDS and written as the block's 16 runs.
-constexpr int DPK_LD = 258;  // doubles per LDS row (256 + pad)
-template <bool VEC>
-__global__ __launch_bounds__(256) void pack_f64_kunit_kernel(const double *A, int64_t cs, int64_t K, int64_t N,
-                                                             int64_t Kp, double *packed) {
-    __shared__ __attribute__((aligned(16))) double tile[16][DPK_LD];
-    const int tid = threadIdx.x;
-    const int64_t KS = Kp / 16;
-    const int64_t jb = blockIdx.y;
-    const int64_t kt0 = (int64_t)blockIdx.x * SPL_KT;
-    const int c = tid >> 4, p0 = tid & 15;
-    const int64_t j = jb * 16 + c;
-    f64x2 v[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int64_t k = kt0 + 2 * (16 * i + p0);
-        const double *src = A + k + j * cs;
-        if (VEC && j < N && k + 1 < K) {
-            v[i] = *(const f64x2 *)src;
-        } else {
-            v[i][0] = (j < N && k < K) ? src[0] : 0.0;
-            v[i][1] = (j < N && k + 1 < K) ? src[1] : 0.0;
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) *(f64x2 *)&tile[c][2 * (16 * i + p0)] = v[i];
-    __syncthreads();
-    const int64_t steps = (KS - kt0 / 16) < 16 ? (KS - kt0 / 16) : 16;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int task = tid + 256 * i;
-        const int st = task >> 6, l = task & 63;
-        if (st >= steps) break;
-        const double *src = &tile[l & 15][16 * st + (l >> 4)];
-        f64x2 lo, hi;
-        lo[0] = src[0];
-        lo[1] = src[4];
-        hi[0] = src[8];
-        hi[1] = src[12];
-        double *dst = packed + ((jb * KS + kt0 / 16 + st) * 64 + l) * 4;
-        *(f64x2 *)dst = lo;
-        *(f64x2 *)(dst + 2) = hi;
-    }
-}
-
-struct F64WideProblem {
-    int64_t M, N, Kp;
-    GenMap g;
-    const double *packed;
-    double *part;  // nS x M x N, row-major
-    int64_t kw;
-    int nMB, nNB, nS;
-    TailCols<double> tc;  // tail columns, as in F32WideProblem
-    double *tpart;
-};
-
-
-template <bool GAUSS, bool ROWS, int CB, int TW>
-__global__ __launch_bounds__(BF_FTHR, 1) void f64_wide_kernel(F64WideProblem pb) {
-    constexpr int RB = 4, MT = 64, NT = 128 * CB;  // CB 16-column blocks per wave
-    __shared__ __attribute__((aligned(16))) double Ss[2][MT * DW_LDK];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int W = pb.nMB * pb.nNB * pb.nS;
-    const int L = blockIdx.x;
-    const int t = (W % 8 == 0) ? (L % 8) * (W / 8) + L / 8 : L;
-    const int mb = t % pb.nMB;
-    const int rest = t / pb.nMB;
-    const int nb = rest % pb.nNB;
-    const int sp = rest / pb.nNB;
-    const int64_t m0 = (int64_t)mb * MT, n0 = (int64_t)nb * NT;
-    const int64_t kbeg = (int64_t)sp * pb.kw;
-    int64_t kend = kbeg + pb.kw;
-    if (kend > pb.Kp) kend = pb.Kp;
-    const int nchunks = (int)((kend - kbeg) / 32);
-    const GenMap g = pb.g;
-
-    f64x4 acc[RB][CB];
-#pragma unroll
-    for (int i = 0; i < RB; ++i)
-#pragma unroll
-        for (int j = 0; j < CB; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
-
-    const int64_t wcol = n0 + wave * (16 * CB);
-    const int64_t KS = pb.Kp / 16;
-    const double *bbase = pb.packed + ((wcol >> 4) * KS * 64 + lane) * 4;
-    const int64_t bblk = KS * 256;  // doubles between 16-column blocks
-    const int64_t s_first = kbeg / 16, s_last = kend / 16 - 1;
-
-    const int frow = ROWS ? 4 * (tid & 15) : tid >> 3, fcell = ROWS ? tid >> 4 : tid & 7;
-    const uint64_t foff = ROWS ? (uint64_t)((g.a_off + kbeg + fcell) * g.P + ((g.b_off + m0) >> 2) + (tid & 15))
-                               : (uint64_t)((g.a_off + m0 + frow) * g.P + ((g.b_off + kbeg) >> 2) + fcell);
-    const uint64_t fstep = ROWS ? 32 * (uint64_t)g.P : 8;
-    // tail columns: only the first column block's workgroups form them
-    // (cb < 4: the output has one column block, nb == 0)
-    WideTail<double, ROWS, TW == 0 ? 1 : TW> tl;
-    const int64_t tk = kbeg + (ROWS ? fcell : 4 * fcell);  // the thread's first k of chunk 0
-    if constexpr (TW > 0) {
-        tl.zero();
-        tl.load(pb.tc, tk);
-    }
-    auto gen_chunk = [&](int c, double *lds) {
-        const float4 v = gen4(GAUSS, ctr_add(g.ctr, foff + fstep * (uint64_t)c), g.k0, g.k1);
-        const double ent[4] = {entry_value<double>(v.x, GAUSS), entry_value<double>(v.y, GAUSS),
-                               entry_value<double>(v.z, GAUSS), entry_value<double>(v.w, GAUSS)};
-        if constexpr (ROWS) {
-            const int pos = dw_pos(fcell);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) lds[(frow + e) * DW_LDK + pos] = ent[e];
-        } else {
-            double *row = lds + frow * DW_LDK;
-            const int k0 = 4 * fcell;
-            row[dw_pos(k0)] = ent[0];
-            row[dw_pos(k0 + 1)] = ent[1];
-            row[dw_pos(k0 + 2)] = ent[2];
-            row[dw_pos(k0 + 3)] = ent[3];
-        }
-        if constexpr (TW > 0) {
-            tl.step(ent);
-            tl.load(pb.tc, tk + 32 * (int64_t)(c + 1 < nchunks ? c + 1 : c));  // the next chunk's
-        }
-    };
-
-    // B operands of one step: lo = q 0..1, hi = q 2..3 of block j
-    f64x2 blo[CB], bhi[CB];
-#pragma unroll
-    for (int j = 0; j < CB; ++j) {
-        blo[j] = *(const f64x2 *)(bbase + j * bblk + s_first * 256);
-        bhi[j] = *(const f64x2 *)(bbase + j * bblk + s_first * 256 + 2);
-    }
-
-    auto step = [&](const double *S, int ks, int64_t s_next) {
-        __builtin_amdgcn_s_setprio(1);
-        f64x2 alo[RB], ahi[RB];
-#pragma unroll
-        for (int i = 0; i < RB; ++i) {
-            const double *src = S + (16 * i + (lane & 15)) * DW_LDK + 16 * ks + 4 * (lane >> 4);
-            alo[i] = *(const f64x2 *)src;
-            ahi[i] = *(const f64x2 *)(src + 2);
-        }
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int j = 0; j < CB; ++j)
-#pragma unroll
-                for (int i = 0; i < RB; ++i)
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(alo[i][q], blo[j][q], acc[i][j], 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < CB; ++j) blo[j] = *(const f64x2 *)(bbase + j * bblk + s_next * 256);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int j = 0; j < CB; ++j)
-#pragma unroll
-                for (int i = 0; i < RB; ++i)
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ahi[i][q], bhi[j][q], acc[i][j], 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < CB; ++j) bhi[j] = *(const f64x2 *)(bbase + j * bblk + s_next * 256 + 2);
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_setprio(0);
-    };
-
-    const bool late = (wave & 4) != 0;
-    gen_chunk(0, Ss[0]);
-    __syncthreads();
-    if constexpr (TW == 0) {
-        for (int c = 0; c < nchunks; ++c) {
-            const double *S = Ss[c & 1];
-            double *Sn = Ss[(c + 1) & 1];
-            const int64_t s0 = s_first + 2 * c;
-            const bool more = c + 1 < nchunks;
-            if (more && !late) gen_chunk(c + 1, Sn);
-            step(S, 0, s0 + 1);
-            step(S, 1, s0 + 2 > s_last ? s_last : s0 + 2);
-            if (more && late) gen_chunk(c + 1, Sn);
-            __syncthreads();
-        }
-    } else {
-        // with a tail: one loop per wave role and the last chunk peeled, so
-        // no branch surrounds the tail's loads inside a loop (the compiler's
-        // memory-counter waits for the MFMA operands stay exact)
-        const int last = nchunks - 1;
-        if (!late) {
-            for (int c = 0; c < last; ++c) {
-                gen_chunk(c + 1, Ss[(c + 1) & 1]);
-                step(Ss[c & 1], 0, s_first + 2 * c + 1);
-                step(Ss[c & 1], 1, s_first + 2 * c + 2);
-                __syncthreads();
-            }
-        } else {
-            for (int c = 0; c < last; ++c) {
-                step(Ss[c & 1], 0, s_first + 2 * c + 1);
-                step(Ss[c & 1], 1, s_first + 2 * c + 2);
-                gen_chunk(c + 1, Ss[(c + 1) & 1]);
-                __syncthreads();
-            }
-        }
-        step(Ss[last & 1], 0, s_first + 2 * last + 1);
-        step(Ss[last & 1], 1, s_last);
-        __syncthreads();
-    }
-
-    if constexpr (TW > 0)
-        if (nb == 0) tl.finish(pb.tc.nt, tid, frow, fcell, &Ss[0][0], pb.tpart + (int64_t)sp * pb.tc.nt * pb.M + m0, pb.M);
-
-    // element r of a 16 x 16 FP64 block: row l / 16 + 4 r, column l % 16
-    double *P = pb.part + (int64_t)sp * pb.M * pb.N;
-#pragma unroll
-    for (int i = 0; i < RB; ++i)
-#pragma unroll
-        for (int j = 0; j < CB; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int64_t gi = m0 + i * 16 + (lane >> 4) + 4 * r;
-                const int64_t gj = wcol + j * 16 + (lane & 15);
-                P[gi * pb.N + gj] = acc[i][j][r];
-            }
-}
-
-template <int CB, int TW>
-static void launch_f64_wide(bool gauss, bool rows, dim3 grid, const F64WideProblem &w, hipStream_t st) {
-    if (gauss && rows) hipLaunchKernelGGL((f64_wide_kernel<true, true, CB, TW>), grid, dim3(BF_FTHR), 0, st, w);
-    else if (gauss) hipLaunchKernelGGL((f64_wide_kernel<true, false, CB, TW>), grid, dim3(BF_FTHR), 0, st, w);
-    else if (rows) hipLaunchKernelGGL((f64_wide_kernel<false, true, CB, TW>), grid, dim3(BF_FTHR), 0, st, w);
-    else hipLaunchKernelGGL((f64_wide_kernel<false, false, CB, TW>), grid, dim3(BF_FTHR), 0, st, w);
-}
-// by tail width: none, one column, two to four
-template <int CB>
-static void launch_f64_wide_tw(bool gauss, bool rows, int nt, dim3 grid, const F64WideProblem &w, hipStream_t st) {
-    if (nt == 0) launch_f64_wide<CB, 0>(gauss, rows, grid, w, st);
-    else if (nt == 1) launch_f64_wide<CB, 1>(gauss, rows, grid, w, st);
-    else launch_f64_wide<CB, WIDE_TAIL>(gauss, rows, grid, w, st);
-}
-
-int f64_wide_run(const GemmProblem &pb, GemmProblem rest[2], hipStream_t stream) {
-    if (!pb.gen_is_x || pb.sbuf != nullptr || (pb.g.b_off & 3) != 0) return -1;
-    if (pb.K < 1024 || pb.K % 32 != 0 || pb.M < 64 || pb.N < 128) return -1;
-    const int cb = pb.N >= 512 ? 4 : (pb.N >= 256 ? 2 : 1);
-    const int64_t NT = 128 * cb;
-    const int64_t Mf = pb.M / 64 * 64, Nf = pb.N / NT * NT, K = pb.K;
-    const int nt = wide_tail_cols(pb, Mf, Nf, cb);
-    if (nt < 0) return -1;
-    F64WideProblem w{};
-    w.M = Mf;
-    w.N = Nf;
-    w.Kp = K;
-    w.g = pb.g;
-    w.nMB = (int)(Mf / 64);
-    w.nNB = (int)(Nf / NT);
-    int64_t kw = 16384;
-    const int64_t tiles = (int64_t)w.nMB * w.nNB;
-    // about four workgroups per CU; exactly one per CU when the tiles divide
-    // the CUs (one round, a quarter of the partial sums: 4% faster at 16 tiles)
-    const int64_t cus = num_cus();
-    const int64_t want = cus % tiles == 0 ? cus / tiles : (4 * cus + tiles - 1) / tiles;
-    const int64_t kw_fill = (K + want - 1) / want;
-    if (kw_fill < kw) kw = kw_fill;
-    kw = (kw + 31) / 32 * 32;
-    if (kw < 32) kw = 32;
-    if (K < 2048 && kw < 256 && Mf * Nf > (1ll << 20)) return -1;  // as in f32_wide_run
-    w.kw = kw;
-    w.nS = (int)((K + kw - 1) / kw);
-    if ((int64_t)w.nMB * w.nNB * w.nS >= (1ll << 31)) return -1;
-    const size_t packed_bytes = align256b((size_t)safe_mul(K, Nf) * 8);
-    const size_t part_bytes = align256b((size_t)safe_mul(safe_mul(w.nS, Mf), Nf) * 8);
-    const size_t tail_bytes = (size_t)w.nS * nt * Mf * 8;
-    if (packed_bytes + part_bytes + tail_bytes > WIDE_SCRATCH_MAX) return -1;
-    char *ws = (char *)wide_scratch(packed_bytes + part_bytes + tail_bytes, stream);
-    if (ws == nullptr) return -1;
-    w.packed = (const double *)ws;
-    w.part = (double *)(ws + packed_bytes);
-    const double *Y = (const double *)pb.D;
-    w.tc = wide_tail_io<double>(pb, nt);
-    w.tpart = (double *)(ws + packed_bytes + part_bytes);
-    {
-        ProfScope prof("f64_pack_kernel", stream);
-        if (pb.drs == 1) {
-            const int64_t kt = (K + SPL_KT - 1) / SPL_KT;
-            RBX_REQUIRE(kt < (1ll << 31) && Nf / 16 <= 65535);
-            const dim3 grid((unsigned)kt, (unsigned)(Nf / 16));
-            if (pb.dcs % 2 == 0 && ((uintptr_t)Y & 15) == 0)
-                hipLaunchKernelGGL(pack_f64_kunit_kernel<true>, grid, dim3(256), 0, stream, Y, pb.dcs, K, Nf, K,
-                                   (double *)w.packed);
-            else
-                hipLaunchKernelGGL(pack_f64_kunit_kernel<false>, grid, dim3(256), 0, stream, Y, pb.dcs, K, Nf, K,
-                                   (double *)w.packed);
-        } else {
-            hipLaunchKernelGGL(pack_f64_kernel, dim3(65536), dim3(256), 0, stream, Y, pb.drs, pb.dcs, K, Nf, K, Nf,
-                               (double *)w.packed);
-        }
-        RBX_HIP(hipGetLastError());
-    }
-    {
-        ProfScope prof("f64_wide_kernel", stream);
-        const dim3 grid((unsigned)(w.nMB * w.nNB * w.nS));
-        const bool rows = w.g.b_along_rows != 0;
-        const bool gauss = w.g.gauss != 0;
-        if (cb == 4) launch_f64_wide<4, 0>(gauss, rows, grid, w, stream);  // no tail at cb = 4
-        else if (cb == 2) launch_f64_wide_tw<2>(gauss, rows, nt, grid, w, stream);
-        else launch_f64_wide_tw<1>(gauss, rows, nt, grid, w, stream);
-        RBX_HIP(hipGetLastError());
-    }
-    {
-        ProfScope prof("f64_reduce_kernel", stream);
-        const dim3 grid = reduce_grid(Mf, Nf);
-        hipLaunchKernelGGL((bf16_reduce_kernel<double, double>), grid, dim3(256), 0, stream, (const double *)w.part,
-                           w.nS, Mf, Nf, pb.alpha, pb.beta, (double *)pb.C, pb.crs, pb.ccs);
-        if (nt > 0)
-            launch_tail_reduce<double>(w.tpart, w.nS, Mf, w.tc, pb.alpha, pb.beta, stream);
-        RBX_HIP(hipGetLastError());
-    }
-    int nr = 0;
-    if (pb.M > Mf) {
-        GemmProblem r = pb;
-        r.M = pb.M - Mf;
-        if (pb.g.b_along_rows) r.g.b_off = pb.g.b_off + Mf;
-        else r.g.a_off = pb.g.a_off + Mf;
-        r.C = (double *)pb.C + Mf * pb.crs;
-        rest[nr++] = r;
-    }
-    if (pb.N - nt > Nf) {
-        GemmProblem r = pb;
-        r.xD = nullptr;
-        r.xC = nullptr;
-        r.M = Mf;
-        r.N = pb.N - nt - Nf;
-        r.D = Y + Nf * pb.dcs;
-        r.C = (double *)pb.C + Nf * pb.ccs;
-        rest[nr++] = r;
-    }
-    return nr;
-}
-
 // ---------------------------------------------------------------- fast generator bounds
 // Measures, over every 32-bit word, the distance of the hardware factors of
 // the fast generator from the portable factors that define the operator:

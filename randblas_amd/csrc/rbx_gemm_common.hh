@@ -1,6 +1,5 @@
 // rbx_gemm_common.hh -- the column-major product description shared by the
-// dense sketch kernels, and the two tile producers: operator tiles generated
-// from Philox counters, and strided dense tiles loaded from memory.
+// dense sketch kernels, and operator tiles generated from Philox counters.
 #pragma once
 #include "rbx_internal.hh"
 
@@ -17,49 +16,14 @@ struct GemmProblem {
     int gen_is_x;         // 1: X = operator, Y = D; 0: X = D, Y = operator
     void *C;
     int64_t crs, ccs;
-    // split K: nsplit > 1 runs K ranges of kw (the last one shorter) as
-    // blockIdx.z, each writing its raw product to part + z * M * N
-    // (column-major M x N); a reduction then forms alpha * sum + beta * C
-    int nsplit = 1;
-    int64_t kw = 0;
-    void *part = nullptr;
     // the last column of D and of C held apart from the rest (a right-hand
     // side beside a matrix): D's column N - 1 at xD[k * xdrs], C's at
-    // xC[i * xcrs]; only the wide kernels' tail takes these
+    // xC[i * xcrs]; only wide_run takes these (K-unit D, unit xdrs)
     const void *xD = nullptr;
     int64_t xdrs = 0;
     void *xC = nullptr;
     int64_t xcrs = 0;
 };
-
-// The sub-problem of K range z: the dense operand and the operator are
-// advanced along K, the output is the split's partial (alpha 1, beta 0).
-template <typename T>
-__device__ __forceinline__ GemmProblem split_view(const GemmProblem &in, int z) {
-    if (in.nsplit <= 1) return in;
-    GemmProblem q = in;
-    const int64_t k0 = (int64_t)z * in.kw;
-    q.K = in.K - k0 < in.kw ? in.K - k0 : in.kw;
-    if (in.gen_is_x) {
-        // X = operator (M x K, K = its column index q), Y = D (K x N, K = row)
-        q.D = (const T *)in.D + k0 * in.drs;
-        if (in.sbuf) q.soff = in.soff + k0 * in.scs;
-        else if (in.g.b_along_rows) q.g.a_off = in.g.a_off + k0;
-        else q.g.b_off = in.g.b_off + k0;
-    } else {
-        // X = D (M x K, K = column), Y = operator (K x N, K = its row index p)
-        q.D = (const T *)in.D + k0 * in.dcs;
-        if (in.sbuf) q.soff = in.soff + k0 * in.srs;
-        else if (in.g.b_along_rows) q.g.b_off = in.g.b_off + k0;
-        else q.g.a_off = in.g.a_off + k0;
-    }
-    q.C = (T *)in.part + (int64_t)z * in.M * in.N;
-    q.crs = 1;
-    q.ccs = in.M;
-    q.alpha = 1.0;
-    q.beta = 0.0;
-    return q;
-}
 
 // Point the problem at S->buff when the operator is materialised
 // (lskge3/rskge3 with S.buff != nullptr: offset_and_ldim, skge.hh:195-198).
@@ -132,27 +96,6 @@ __device__ __forceinline__ void gen_tile(const GenMap &g, int64_t p0, int64_t q0
     }
 }
 
-// Load the PR x QC tile of a strided matrix (element (p,q) at src[p*rs + q*cs])
-// into LDS at lds[(p-p0)*ldp + (q-q0)*ldq], zero-filling outside the limits.
-// Consecutive threads walk the unit-stride direction when there is one.
-template <typename T, int PR, int QC, int NT>
-__device__ __forceinline__ void load_tile(const T *src, int64_t rs, int64_t cs, int64_t p0, int64_t q0, int64_t p_lim,
-                                          int64_t q_lim, T *lds, int ldp, int ldq, int tid) {
-    if (rs == 1) {
-        for (int idx = tid; idx < PR * QC; idx += NT) {
-            const int pp = idx % PR, qq = idx / PR;
-            const int64_t p = p0 + pp, q = q0 + qq;
-            lds[pp * ldp + qq * ldq] = (p < p_lim && q < q_lim) ? src[p + q * cs] : (T)0;
-        }
-    } else {
-        for (int idx = tid; idx < PR * QC; idx += NT) {
-            const int qq = idx % QC, pp = idx / QC;
-            const int64_t p = p0 + pp, q = q0 + qq;
-            lds[pp * ldp + qq * ldq] = (p < p_lim && q < q_lim) ? src[p * rs + q * cs] : (T)0;
-        }
-    }
-}
-
 template <typename T>
 void scale_output(T *C, int64_t M, int64_t N, int64_t crs, int64_t ccs, double beta, hipStream_t stream);
 
@@ -161,19 +104,15 @@ GemmProblem plan_left(char layout, char opS, char opA, int64_t d, int64_t n, int
                       const rbx_dense_skop *S, int64_t ro_s, int64_t co_s, const T *A, int64_t lda, double beta,
                       T *B, int64_t ldb);
 
-// FP32 problems with a generated operator on the X side and large interior
-// shapes: runs the covered part on the wide-tile kernel and returns the
-// remaining sub-problems in rest[] (their count), or -1 when it does not
-// apply (rbx_bf16.hip).
-int f32_wide_run(const GemmProblem &pb, GemmProblem rest[2], hipStream_t stream);
-// The same for FP64 problems (tiles of up to 64 x 512).
-int f64_wide_run(const GemmProblem &pb, GemmProblem rest[2], hipStream_t stream);
+// Runs a problem with the operator on the X side (rbx_wide.hip).
+template <typename T>
+void wide_run(const GemmProblem &pb, hipStream_t stream);
 
 // [B b] = op(S) * [A a] for column-major A (m x n, lda) and B (d x n, ldb)
 // with one more column a (m) -> b (d) held apart, alpha 1, beta 0, in one
-// pass over the generated operator (the wide kernels' tail column).  Returns
-// false, having launched nothing, when the wide kernels do not take the
-// shape (the caller then sketches A and a separately).
+// pass over the generated operator.  Returns false, having launched nothing,
+// when the operator is materialised or m < 4 (the caller then sketches A and
+// a separately).
 template <typename T>
 bool left_sketch_with_column(char opS, int64_t d, int64_t n, int64_t m, const rbx_dense_skop *S, int64_t ro_s,
                              int64_t co_s, const T *A, int64_t lda, const T *a, T *B, int64_t ldb, T *b,

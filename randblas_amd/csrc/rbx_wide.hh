@@ -1,0 +1,479 @@
+// rbx_wide.hh -- fused dense sketches, FP64 and FP32:
+//     C[M x N] = alpha * G[M x K] * Y[K x N] + beta * C
+// G the operator, generated from its Philox counters (or read from memory
+// when it is materialised), Y the dense operand (either unit stride), any
+// sizes and any submatrix of the operator.
+//
+// One 512-thread workgroup per 64 x NT output tile and K range.  Every 32-deep
+// chunk of the tile's operator rows is generated once into LDS (each thread
+// one counter, four entries) while the chunk before it is multiplied: waves
+// 0-3 generate before their MFMAs, waves 4-7 after, so the two waves that
+// share a SIMD are in opposite phases.  The 8 waves form a WM x 8 / WM grid;
+// each owns RB x CB blocks of v_mfma_f{64,32}_16x16x4 (WM * RB = 4, NT = 128
+// CB / WM).  The dense operand goes straight from memory into the MFMA
+// registers, one 16-deep step ahead of its use: lane (g = l / 16, c = l % 16)
+// holds k = 4 g .. 4 g + 3 of its columns, so with unit stride along K a
+// column's 16 k are one run of four lanes' vectors, and with unit stride along
+// N a lane holds CB neighbouring columns of four rows.
+//
+// Sizes that do not fit: K (at least 4) is rounded up to whole chunks, the
+// dense values past it are zeros (the operator's are whatever the counters
+// give); rows and
+// columns past the edge read the edge again and are not stored.  An operator
+// window that starts inside a counter (b_off % 4 != 0) is moved back to the
+// counter's start: ko extra k with zero dense values, or mo extra rows that
+// are not stored.
+#pragma once
+#include "rbx_gemm_common.hh"
+
+namespace rbx {
+
+constexpr int WD_THR = 512, WD_MT = 64, WD_KC = 32;
+
+template <typename T>
+struct WideMma;
+template <>
+struct WideMma<double> {
+    typedef double acc_t __attribute__((ext_vector_type(4)));
+    static constexpr int LDK = 34;  // row stride 68 words: 16 rows' 16-byte reads cover the banks once
+    static __device__ __forceinline__ acc_t mma(double a, double b, acc_t c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int out_row(int lane, int r) { return (lane >> 4) + 4 * r; }
+};
+template <>
+struct WideMma<float> {
+    typedef float acc_t __attribute__((ext_vector_type(4)));
+    static constexpr int LDK = 36;
+    static __device__ __forceinline__ acc_t mma(float a, float b, acc_t c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int out_row(int lane, int r) { return 4 * (lane >> 4) + r; }
+};
+
+// Tail columns: up to WIDE_TAIL output columns past the last whole tile (the
+// right-hand side of [A b]) are formed by the threads that generate the
+// operator, from the four entries each holds per chunk, with VALU FMAs.  The
+// generator of operator rows along K holds one row's four consecutive k (one
+// accumulator per column); the one of counters along the rows holds four rows
+// at one k (four per column).  The dense values of chunk c + 1 are loaded
+// right after chunk c's are used, so they have a chunk's MFMAs to arrive.  TW
+// columns are always loaded and accumulated (TW = 1, or 4 with the unused
+// ones repeating the last real column), so the chunk loop has no branch.
+constexpr int WIDE_TAIL = 4;
+// Dense column j's element k at col[j][k * rs[j]], its output's element i at
+// out[j][i * ors[j]]; entries nt .. WIDE_TAIL - 1 of col / rs repeat nt - 1.
+template <typename T>
+struct TailCols {
+    const T *col[WIDE_TAIL];
+    int64_t rs[WIDE_TAIL];
+    T *out[WIDE_TAIL];
+    int64_t ors[WIDE_TAIL];
+    int nt;
+};
+template <typename T, bool ROWS, int TW>
+struct WideTail {
+    static constexpr int R = ROWS ? 4 : 1;  // output rows per thread
+    static constexpr int E = ROWS ? 1 : 4;  // dense values per column per chunk
+    T acc[TW][R];
+    T cur[TW][E];  // the dense values of the chunk being generated
+
+    __device__ __forceinline__ void zero() {
+#pragma unroll
+        for (int j = 0; j < TW; ++j)
+#pragma unroll
+            for (int r = 0; r < R; ++r) acc[j][r] = (T)0;
+    }
+    // cur = dense values of k .. k + E - 1, zeros outside [0, K)
+    __device__ __forceinline__ void load(const TailCols<T> &tc, int64_t k, int64_t K) {
+#pragma unroll
+        for (int j = 0; j < TW; ++j)
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int64_t q = k + e, in = q < 0 ? 0 : (q < K ? q : K - 1);
+                const T v = tc.col[j][in * tc.rs[j]];
+                cur[j][e] = in == q ? v : (T)0;
+            }
+    }
+    __device__ __forceinline__ void step(const T (&ent)[4]) {
+#pragma unroll
+        for (int j = 0; j < TW; ++j) {
+            if constexpr (ROWS) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[j][r] = fma(ent[r], cur[j][0], acc[j][r]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[j][0] = fma(ent[e], cur[j][e], acc[j][0]);
+            }
+        }
+    }
+    // The workgroup's 64 x nt partial into out[j * Mt + row].  Rows along K:
+    // the eight threads of a row are adjacent lanes (butterfly).  Counters
+    // along the rows: lanes l, l ^ 16, l ^ 32, l ^ 48 of a wave share rows
+    // (butterfly), then the eight waves are summed in order through `red`
+    // (8 * TW * 64 values).  Every thread calls this (it has a barrier).
+    __device__ __forceinline__ void finish(int nt, int tid, int frow, int fcell, T *red, T *out, int64_t Mt) {
+        const int lane = tid & 63, wave = tid >> 6;
+        if constexpr (!ROWS) {
+#pragma unroll
+            for (int j = 0; j < TW; ++j) {
+                T v = acc[j][0];
+                v += __shfl_xor(v, 1);
+                v += __shfl_xor(v, 2);
+                v += __shfl_xor(v, 4);
+                if (j < nt && fcell == 0) out[j * Mt + frow] = v;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < TW; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    T v = acc[j][r];
+                    v += __shfl_xor(v, 16);
+                    v += __shfl_xor(v, 32);
+                    if (lane < 16) red[(wave * TW + j) * 64 + frow + r] = v;
+                }
+            __syncthreads();
+            if (tid < 64 * nt) {
+                const int j = tid >> 6, row = tid & 63;
+                T v = red[j * 64 + row];
+#pragma unroll
+                for (int w = 1; w < WD_THR / 64; ++w) v += red[(w * TW + j) * 64 + row];
+                out[j * Mt + row] = v;
+            }
+        }
+    }
+};
+
+template <typename T>
+struct WideProblem {
+    int64_t M, N, K;       // N without the tail columns
+    GenMap g;              // b_off a multiple of 4
+    const T *S;            // materialised operator: element (i, k) at S[i * srs + k * scs]
+    int64_t srs, scs;
+    int ko, mo;            // extra k / rows in front (see above); one of them is 0
+    const T *D;
+    int64_t drs, dcs;
+    const T *xD;           // column N - 1 (unit stride) when not null
+    T *C, *xC;             // nS == 1: written by the kernel
+    int64_t crs, ccs, xcrs;
+    T alpha, beta;
+    T *part;               // nS > 1: partials, nS x M x ldp
+    int64_t ldp, kw;       // kw: k per range, a multiple of 32
+    int nMB, nNB, nS;
+    TailCols<T> tc;        // tail columns, partials at tpart[(split * tc.nt + j) * 64 nMB + row]
+    T *tpart;
+};
+
+template <typename T, int N>
+struct WideVec {
+    typedef T type __attribute__((ext_vector_type(N), aligned(sizeof(T))));
+};
+
+// The operator: uniform or Gaussian, generated, or read from memory.  ROWS: its
+// counters (or its unit stride) run along the output's rows, else along K.
+enum WideOp { WIDE_UNIFORM = 0, WIDE_GAUSS = 1, WIDE_MEM = 2 };
+
+// NU: the dense operand's unit stride runs along N (else along K).
+template <typename T, int OP, bool ROWS, bool NU, int WM, int CB, int TW>
+__global__ __launch_bounds__(WD_THR, 1) void wide_kernel(const WideProblem<T> pb) {
+    using MM = WideMma<T>;
+    constexpr int RB = 4 / WM, WN = 8 / WM, LDK = MM::LDK;
+    constexpr int NT = 16 * CB * WN;
+    constexpr int RED = TW > 0 ? 8 * TW * 64 : 0;
+    constexpr int LDS_N = 2 * WD_MT * LDK > RED ? 2 * WD_MT * LDK : RED;
+    __shared__ __attribute__((aligned(16))) T Ss[LDS_N];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = wave % WM, wn = wave / WM;
+    const int lc = lane & 15, lg = lane >> 4;
+
+    // XCD-aware tile order: consecutive tiles (same K range and columns, so
+    // the same dense operand) on one XCD
+    const int W = pb.nMB * pb.nNB * pb.nS;
+    const int xcd = blockIdx.x % 8, xi = blockIdx.x / 8;
+    const int t = xcd * (W / 8) + (xcd < W % 8 ? xcd : W % 8) + xi;
+    const int mb = t % pb.nMB;
+    const int rest = t / pb.nMB;
+    const int nb = rest % pb.nNB;
+    const int sp = rest / pb.nNB;
+    const int64_t m0 = (int64_t)mb * WD_MT, n0 = (int64_t)nb * NT;
+    const int64_t Kp = pb.K + pb.ko;
+    const int64_t kbeg = (int64_t)sp * pb.kw;
+    const int64_t kend = kbeg + pb.kw < Kp ? kbeg + pb.kw : Kp;
+    const int nchunks = (int)((kend - kbeg + WD_KC - 1) / WD_KC);
+    const GenMap g = pb.g;
+    constexpr bool GAUSS = OP == WIDE_GAUSS;
+
+    typename MM::acc_t acc[RB][CB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < CB; ++j) acc[i][j] = typename MM::acc_t{0, 0, 0, 0};
+
+    // ---- operator chunk: rows along K (!ROWS): the thread owns cell tid % 8
+    // of row tid / 8; counters along the rows (ROWS): rows 4 (tid % 16) .. + 3
+    // of column tid / 16.  LDS row r, k at Ss[r * LDK + k].
+    const int frow = ROWS ? 4 * (tid & 15) : tid >> 3, fcell = ROWS ? tid >> 4 : tid & 7;
+    const uint64_t foff = ROWS ? (uint64_t)((g.a_off + kbeg + fcell) * g.P + ((g.b_off + m0) >> 2) + (tid & 15))
+                               : (uint64_t)((g.a_off + m0 + frow) * g.P + ((g.b_off + kbeg) >> 2) + fcell);
+    const uint64_t fstep = ROWS ? WD_KC * (uint64_t)g.P : WD_KC / 4;  // counters per chunk
+    WideTail<T, ROWS, TW == 0 ? 1 : TW> tl;
+    const int64_t tk = kbeg - pb.ko + (ROWS ? fcell : 4 * fcell);  // the thread's first k of chunk 0
+    if constexpr (TW > 0) {
+        tl.zero();
+        tl.load(pb.tc, tk, pb.K);
+    }
+    // a materialised operator's entries of the next chunk, loaded a chunk ahead
+    T mem[4];
+    auto load_op = [&](int c) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int64_t r = m0 + frow + (ROWS ? e : 0) - pb.mo;
+            const int64_t k = kbeg - pb.ko + WD_KC * (int64_t)c + (ROWS ? fcell : 4 * fcell + e);
+            const int64_t ri = r < 0 ? 0 : (r < pb.M ? r : pb.M - 1), ki = k < 0 ? 0 : (k < pb.K ? k : pb.K - 1);
+            const T v = pb.S[ri * pb.srs + ki * pb.scs];
+            mem[e] = ri == r && ki == k ? v : (T)0;
+        }
+    };
+    if constexpr (OP == WIDE_MEM) load_op(0);
+    auto gen_chunk = [&](int c, T *lds) {
+        T ent[4];
+        if constexpr (OP == WIDE_MEM) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ent[e] = mem[e];
+        } else {
+            const float4 v = gen4(GAUSS, ctr_add(g.ctr, foff + fstep * (uint64_t)c), g.k0, g.k1);
+            ent[0] = entry_value<T>(v.x, GAUSS);
+            ent[1] = entry_value<T>(v.y, GAUSS);
+            ent[2] = entry_value<T>(v.z, GAUSS);
+            ent[3] = entry_value<T>(v.w, GAUSS);
+        }
+        if constexpr (ROWS) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) lds[(frow + e) * LDK + fcell] = ent[e];
+        } else {
+            T *row = lds + frow * LDK + 4 * fcell;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) row[e] = ent[e];
+        }
+        if constexpr (OP == WIDE_MEM) load_op(c + 1);
+        if constexpr (TW > 0) {
+            tl.step(ent);
+            tl.load(pb.tc, tk + WD_KC * (int64_t)(c + 1), pb.K);  // the next chunk's
+        }
+    };
+
+    // ---- dense operand of one 16-deep step, b[j][q] = Y[16 s + 4 lg + q - ko][column j]
+    const int64_t wcol = n0 + wn * (16 * CB);
+    T b[CB][4];
+    const T *colp[NU ? 1 : CB];   // !NU: column j's element k = 4 lg - ko; NU: column cs of that row
+    int64_t cs = wcol + CB * lc;  // NU: the lane's first column, moved back inside the matrix
+    if constexpr (NU) {
+        if (cs > pb.N - CB) cs = pb.N - CB;
+        colp[0] = pb.D + cs;
+    } else {
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            int64_t col = wcol + 16 * j + lc;
+            if (col > pb.N - 1) col = pb.N - 1;
+            colp[j] = (pb.xD != nullptr && col == pb.N - 1) ? pb.xD : pb.D + col * pb.dcs;
+        }
+    }
+    const int64_t k_lane = 4 * lg - pb.ko;
+    auto is_edge = [&](int64_t s) { return 16 * s < pb.ko || 16 * s + 16 > Kp; };
+    // Addresses of a step's loads: element offset of the lane's four k (!NU)
+    // or of row q (NU), inside the matrix also at the ends of K.
+    int64_t koff, roff[NU ? 4 : 1];
+    auto address = [&](int64_t s) {
+        const int64_t k = 16 * s + k_lane;
+        if constexpr (NU) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) roff[q] = (k + q) * pb.drs;
+            if (is_edge(s)) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int64_t kq = k + q < 0 ? 0 : (k + q < pb.K ? k + q : pb.K - 1);
+                    roff[q] = kq * pb.drs;
+                }
+            }
+        } else {
+            koff = k < 0 ? 0 : (k < pb.K - 4 ? k : pb.K - 4);
+        }
+    };
+    auto load_col = [&](int j) {
+        const typename WideVec<T, 4>::type v = *(const typename WideVec<T, 4>::type *)(colp[NU ? 0 : j] + koff);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) b[j][q] = v[q];
+    };
+    auto load_row = [&](int q) {
+        const T *p = colp[0] + roff[NU ? q : 0];
+        constexpr int V = CB % 4 == 0 ? 4 : (CB % 3 == 0 ? 3 : CB);
+        if constexpr (V == 1) {
+            b[0][q] = *p;
+        } else {
+#pragma unroll
+            for (int h = 0; h < CB / V; ++h) {
+                const typename WideVec<T, V>::type v = *(const typename WideVec<T, V>::type *)(p + V * h);
+#pragma unroll
+                for (int j = 0; j < V; ++j) b[V * h + j][q] = v[j];
+            }
+        }
+    };
+    // A step at the ends of K: zeros outside [0, K), and (!NU) the values back
+    // in their places where the vector was read from inside the matrix.
+    auto fix_edge = [&](int64_t s) {
+        const int64_t k = 16 * s + k_lane;
+        const int64_t d = NU ? 0 : k - (k < 0 ? 0 : (k < pb.K - 4 ? k : pb.K - 4));
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            T v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                v[q] = (T)0;
+                if constexpr (NU) {
+                    v[q] = k + q >= 0 && k + q < pb.K ? b[j][q] : (T)0;
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        if (q + d == u) v[q] = b[j][u];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) b[j][q] = v[q];
+        }
+    };
+
+    // One step: the operands of step s_next are loaded right after this
+    // step's last use of their registers, a whole step ahead (the fence keeps
+    // the compiler from moving the loads next to their use).
+    auto step = [&](const T *S, int ks, int64_t s, int64_t s_next) {
+        if (is_edge(s)) fix_edge(s);
+        address(s_next);
+        __builtin_amdgcn_s_setprio(1);
+        T a[RB][4];
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            const T *src = S + (16 * (RB * wm + i) + lc) * LDK + 16 * ks + 4 * lg;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) a[i][q] = src[q];
+        }
+        if constexpr (NU) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+#pragma unroll
+                for (int j = 0; j < CB; ++j)
+#pragma unroll
+                    for (int i = 0; i < RB; ++i) acc[i][j] = MM::mma(a[i][q], b[j][q], acc[i][j]);
+                load_row(q);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < CB; ++j) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int i = 0; i < RB; ++i) acc[i][j] = MM::mma(a[i][q], b[j][q], acc[i][j]);
+                load_col(j);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __builtin_amdgcn_s_setprio(0);
+    };
+
+    const int64_t s_first = kbeg / 16, s_last = s_first + 2 * nchunks - 1;
+    address(s_first);
+    if constexpr (NU) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) load_row(q);
+    } else {
+#pragma unroll
+        for (int j = 0; j < CB; ++j) load_col(j);
+    }
+
+    const bool late = (wave & 4) != 0;
+    gen_chunk(0, Ss);
+    __syncthreads();
+    for (int c = 0; c < nchunks; ++c) {
+        const T *S = Ss + (c & 1) * (WD_MT * LDK);
+        T *Sn = Ss + ((c + 1) & 1) * (WD_MT * LDK);
+        const int64_t s0 = s_first + 2 * c;
+        const bool more = c + 1 < nchunks;
+        if (more && !late) gen_chunk(c + 1, Sn);
+        step(S, 0, s0, s0 + 1);
+        step(S, 1, s0 + 1, more ? s0 + 2 : s_last);
+        if (more && late) gen_chunk(c + 1, Sn);
+        __syncthreads();
+    }
+
+    if constexpr (TW > 0)
+        if (nb == 0)
+            tl.finish(pb.tc.nt, tid, frow, ROWS ? 0 : fcell, Ss,
+                      pb.tpart + (int64_t)sp * pb.tc.nt * (64 * (int64_t)pb.nMB) + m0, 64 * (int64_t)pb.nMB);
+
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int64_t gi = m0 + 16 * (RB * wm + i) + MM::out_row(lane, r) - pb.mo;
+            if (gi < 0 || gi >= pb.M) continue;
+#pragma unroll
+            for (int j = 0; j < CB; ++j) {
+                // NU: a lane moved back owns only the columns past its neighbour's
+                const int64_t gj = NU ? cs + j : wcol + 16 * j + lc;
+                if (NU ? gj < wcol + CB * lc : gj >= pb.N) continue;
+                const T v = acc[i][j][r];
+                if (pb.part != nullptr) {
+                    pb.part[((int64_t)sp * pb.M + gi) * pb.ldp + gj] = v;
+                } else {
+                    T *c = (pb.xC != nullptr && gj == pb.N - 1) ? pb.xC + gi * pb.xcrs : pb.C + gi * pb.crs + gj * pb.ccs;
+                    T o = pb.alpha * v;
+                    if (pb.beta != (T)0) o = o + pb.beta * (*c);
+                    *c = o;
+                }
+            }
+        }
+}
+
+// Launches the instantiation of a tile width and a number of tail columns.
+template <typename T, int OP, bool ROWS>
+void wide_launch(bool nu, int tile, int tw, const WideProblem<T> &pb, hipStream_t st);
+
+template <typename T, int OP, bool ROWS, bool NU, int WM, int CB, int TW>
+static void wide_launch_one(const WideProblem<T> &pb, hipStream_t st) {
+    hipLaunchKernelGGL((wide_kernel<T, OP, ROWS, NU, WM, CB, TW>), dim3((unsigned)(pb.nMB * pb.nNB * pb.nS)),
+                       dim3(WD_THR), 0, st, pb);
+}
+template <typename T, int OP, bool ROWS, bool NU>
+static void wide_launch_tile(int tile, int tw, const WideProblem<T> &pb, hipStream_t st) {
+    if constexpr (!NU) {
+        if (tw == 1 && tile == 128) return wide_launch_one<T, OP, ROWS, NU, 1, 1, 1>(pb, st);
+        if (tw == 1 && tile == 256) return wide_launch_one<T, OP, ROWS, NU, 1, 2, 1>(pb, st);
+        if (tw > 1 && tile == 128) return wide_launch_one<T, OP, ROWS, NU, 1, 1, WIDE_TAIL>(pb, st);
+        if (tw > 1 && tile == 256) return wide_launch_one<T, OP, ROWS, NU, 1, 2, WIDE_TAIL>(pb, st);
+    }
+    if (tile == 32) return wide_launch_one<T, OP, ROWS, NU, 4, 1, 0>(pb, st);
+    if (tile == 64) return wide_launch_one<T, OP, ROWS, NU, 2, 1, 0>(pb, st);
+    if (tile == 128) return wide_launch_one<T, OP, ROWS, NU, 1, 1, 0>(pb, st);
+    if (tile == 256) return wide_launch_one<T, OP, ROWS, NU, 1, 2, 0>(pb, st);
+    if (tile == 384) return wide_launch_one<T, OP, ROWS, NU, 1, 3, 0>(pb, st);
+    if (tile == 512) return wide_launch_one<T, OP, ROWS, NU, 1, 4, 0>(pb, st);
+    if constexpr (sizeof(T) == 4) {
+        if (tile == 768) return wide_launch_one<T, OP, ROWS, NU, 1, 6, 0>(pb, st);
+        if constexpr (!NU)
+            if (tile == 1024) return wide_launch_one<T, OP, ROWS, NU, 1, 8, 0>(pb, st);
+    }
+    RBX_FAIL(RBX_UNSUPPORTED, "wide kernels: no tile of %d columns", tile);
+}
+
+// One translation unit per (type, operator, orientation) instantiates these.
+#define RBX_WIDE_INSTANCES(T, OP, ROWS)                                                                       \
+    namespace rbx {                                                                                           \
+    template <>                                                                                               \
+    void wide_launch<T, OP, ROWS>(bool nu, int tile, int tw, const WideProblem<T> &pb, hipStream_t st) {      \
+        if (nu) wide_launch_tile<T, OP, ROWS, true>(tile, tw, pb, st);                                        \
+        else wide_launch_tile<T, OP, ROWS, false>(tile, tw, pb, st);                                          \
+    }                                                                                                         \
+    }
+
+}  // namespace rbx

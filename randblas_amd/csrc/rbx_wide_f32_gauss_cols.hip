@@ -1,0 +1,5 @@
+// The wide kernels of FP32 products with a Gaussian operator whose counters run
+// along the contraction.
+#include "rbx_wide.hh"
+
+RBX_WIDE_INSTANCES(float, WIDE_GAUSS, false)
