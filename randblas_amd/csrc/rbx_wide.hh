@@ -24,6 +24,8 @@
 // counter's start: ko extra k with zero dense values, or mo extra rows that
 // are not stored.
 #pragma once
+#include <type_traits>
+
 #include "rbx_gemm_common.hh"
 
 namespace rbx {
@@ -170,20 +172,29 @@ struct WideVec {
     typedef T type __attribute__((ext_vector_type(N), aligned(sizeof(T))));
 };
 
+// Waves per SIMD that the registers are bounded for: two workgroups per CU
+// where the accumulators leave room (the last round of a grid then ends sooner,
+// and one workgroup's barrier is the other's work).
+template <typename T>
+constexpr int wide_waves(int WM, int CB, int TW) {
+    const int acc = 4 / WM * CB * (int)sizeof(T);
+    return acc + 4 * TW * (int)sizeof(T) / 4 <= 48 ? 4 : 2;
+}
+
 // The operator: uniform or Gaussian, generated, or read from memory.  ROWS: its
 // counters (or its unit stride) run along the output's rows, else along K.
 enum WideOp { WIDE_UNIFORM = 0, WIDE_GAUSS = 1, WIDE_MEM = 2 };
 
 // NU: the dense operand's unit stride runs along N (else along K).
 template <typename T, int OP, bool ROWS, bool NU, int WM, int CB, int TW>
-__global__ __launch_bounds__(WD_THR, 1) void wide_kernel(const WideProblem<T> pb) {
+__global__ __launch_bounds__(WD_THR, wide_waves<T>(WM, CB, TW)) void wide_kernel(const WideProblem<T> pb) {
     using MM = WideMma<T>;
     constexpr int RB = 4 / WM, WN = 8 / WM, LDK = MM::LDK;
     constexpr int NT = 16 * CB * WN;
     constexpr int RED = TW > 0 ? 8 * TW * 64 : 0;
     constexpr int LDS_N = 2 * WD_MT * LDK > RED ? 2 * WD_MT * LDK : RED;
     __shared__ __attribute__((aligned(16))) T Ss[LDS_N];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % WM, wn = wave / WM;
     const int lc = lane & 15, lg = lane >> 4;
 
@@ -307,17 +318,21 @@ __global__ __launch_bounds__(WD_THR, 1) void wide_kernel(const WideProblem<T> pb
     };
     auto load_row = [&](int q) {
         const T *p = colp[0] + roff[NU ? q : 0];
-        constexpr int V = CB % 4 == 0 ? 4 : (CB % 3 == 0 ? 3 : CB);
-        if constexpr (V == 1) {
-            b[0][q] = *p;
-        } else {
+        // the lane's CB neighbours in one or two loads (of three or four each)
+        auto piece = [&](auto j0, auto v) {
+            constexpr int J = decltype(j0)::value, V = decltype(v)::value;
+            if constexpr (V == 1) {
+                b[J][q] = p[J];
+            } else {
+                const typename WideVec<T, V>::type x = *(const typename WideVec<T, V>::type *)(p + J);
 #pragma unroll
-            for (int h = 0; h < CB / V; ++h) {
-                const typename WideVec<T, V>::type v = *(const typename WideVec<T, V>::type *)(p + V * h);
-#pragma unroll
-                for (int j = 0; j < V; ++j) b[V * h + j][q] = v[j];
+                for (int j = 0; j < V; ++j) b[J + j][q] = x[j];
             }
-        }
+        };
+        using std::integral_constant;
+        constexpr int V0 = CB <= 4 ? CB : (CB == 5 ? 3 : (CB + 1) / 2);
+        piece(integral_constant<int, 0>{}, integral_constant<int, V0>{});
+        if constexpr (CB > V0) piece(integral_constant<int, V0>{}, integral_constant<int, CB - V0>{});
     };
     // A step at the ends of K: zeros outside [0, K), and (!NU) the values back
     // in their places where the vector was read from inside the matrix.
@@ -455,10 +470,14 @@ static void wide_launch_tile(int tile, int tw, const WideProblem<T> &pb, hipStre
     if (tile == 32) return wide_launch_one<T, OP, ROWS, NU, 4, 1, 0>(pb, st);
     if (tile == 64) return wide_launch_one<T, OP, ROWS, NU, 2, 1, 0>(pb, st);
     if (tile == 128) return wide_launch_one<T, OP, ROWS, NU, 1, 1, 0>(pb, st);
+    if (tile == 192) return wide_launch_one<T, OP, ROWS, NU, 2, 3, 0>(pb, st);
     if (tile == 256) return wide_launch_one<T, OP, ROWS, NU, 1, 2, 0>(pb, st);
+    if (tile == 320) return wide_launch_one<T, OP, ROWS, NU, 2, 5, 0>(pb, st);
     if (tile == 384) return wide_launch_one<T, OP, ROWS, NU, 1, 3, 0>(pb, st);
+    if (tile == 448) return wide_launch_one<T, OP, ROWS, NU, 2, 7, 0>(pb, st);
     if (tile == 512) return wide_launch_one<T, OP, ROWS, NU, 1, 4, 0>(pb, st);
     if constexpr (sizeof(T) == 4) {
+        if (tile == 640) return wide_launch_one<T, OP, ROWS, NU, 1, 5, 0>(pb, st);
         if (tile == 768) return wide_launch_one<T, OP, ROWS, NU, 1, 6, 0>(pb, st);
         if constexpr (!NU)
             if (tile == 1024) return wide_launch_one<T, OP, ROWS, NU, 1, 8, 0>(pb, st);

@@ -143,15 +143,22 @@ static WidePlan wide_plan(const GemmProblem &pb, int ko, int mo, bool NU, bool s
     const int64_t Kp = pb.K + ko, chunks = (Kp + WD_KC - 1) / WD_KC;
     const int64_t nMB = (pb.M + mo + WD_MT - 1) / WD_MT;
     const int cus = num_cus();
-    static const int tiles[] = {32, 64, 128, 256, 384, 512, 768, 1024};
+    // columns, waves along the rows, blocks per wave (wide_launch_tile)
+    static const struct { int cols, wm, cb; } tiles[] = {
+        {32, 4, 1},  {64, 2, 1},  {128, 1, 1}, {192, 2, 3}, {256, 1, 2}, {320, 2, 5},
+        {384, 1, 3}, {448, 2, 7}, {512, 1, 4}, {640, 1, 5}, {768, 1, 6}, {1024, 1, 8}};
     WidePlan best{};
     double best_t = 1e300;
-    for (int tile : tiles) {
+    for (const auto &tl : tiles) {
+        const int tile = tl.cols;
         if (F64 && tile > 512) break;
         // (FP32, unit stride along N) the 1024-wide form has too few registers
         if (NU && tile == 1024) break;
-        const int cb = tile >= 128 ? tile / 128 : 1;
-        if (NU && pb.N < cb) continue;
+        if (NU && pb.N < tl.cb) continue;
+        // two waves read the same columns: only where one tile is the whole
+        // output (100000 columns, K = 2000, FP32: 448 wide 630 us, 512 wide 590)
+        if (tl.wm == 2 && tile > 64 && pb.N > tile) continue;
+        const bool two = wide_waves<T>(tl.wm, tl.cb, 0) == 4;  // two workgroups per CU
         for (int tail = 0; tail < 2; ++tail) {
             int tw = 0;
             if (tail) {
@@ -170,7 +177,9 @@ static WidePlan wide_plan(const GemmProblem &pb, int ko, int mo, bool NU, bool s
                 ns = (chunks + cps - 1) / cps;
                 const double part = (double)ns * (double)pb.M * (double)pb.N * sizeof(T);
                 if (ns > 1 && part > (double)WIDE_PART_MAX) continue;
-                const double rounds = (double)((wgs * ns + cus - 1) / cus);
+                // with two workgroups on a CU the last round overlaps the one before
+                double rounds = (double)((wgs * ns + cus - 1) / cus);
+                if (two && rounds > 1) rounds = std::min(rounds, (double)(wgs * ns) / cus + 0.5);
                 double t = rounds * (cps * chunk_clk + fixed) / mhz;
                 if (ns > 1) t += 5.0 + 2.0 * part / 3.5e6;
                 if (tail) t += 3.0;
