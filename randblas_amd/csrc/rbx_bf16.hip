@@ -336,7 +336,7 @@ __global__ __launch_bounds__(BF_FTHR, 1) void bf16_skge_pair_kernel(Bf16Problem 
     constexpr int MT = 32 * RB, NT = 256 * CB;
     constexpr int RPP = BF_FTHR / PCPR, NCELL = MT / RPP;  // rows per generation pass, cells per thread
     __shared__ __attribute__((aligned(16))) uint16_t Ss[2][MT * PLDK];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
     // XCD-aware tile order: consecutive tiles (same K-split) land on one XCD
     const int W = pb.nMB * pb.nNB * pb.nS;
@@ -364,10 +364,23 @@ __global__ __launch_bounds__(BF_FTHR, 1) void bf16_skge_pair_kernel(Bf16Problem 
 
     const int64_t wcol = n0 + wave * (32 * CB);
     const int64_t KS = pb.Kp / 16;
+    const int64_t bstep_blk = KS * (TERMS * 512);
     // lane's B operand for block j, K step s, term t:
     //   planes + (((wcol/32 + j)*KS + s)*TERMS + t)*512 + lane*8
-    const uint16_t *bbase = pb.planes + (wcol >> 5) * KS * (TERMS * 512) + lane * 8;
-    const int64_t bstep_blk = KS * (TERMS * 512);
+    const uint16_t *bbase = pb.planes + (wcol >> 5) * KS * (TERMS * 512);
+    const uint32_t boff = lane * 16;  // bytes
+    // B operand of a block's step (its terms' runs start at the scalar `run`):
+    // the lane's offset is the load's own 32-bit one, no vector address arithmetic
+    typedef const __attribute__((address_space(1))) char *gptr;
+    auto load_b = [&](gptr run, int tt) {
+        typedef const __attribute__((address_space(1))) u32x4 *gvec;
+        return __builtin_bit_cast(bf16x8, *(gvec)(run + boff + tt * 1024));
+    };
+    auto run_of = [&](int j, int64_t s) {
+        gptr run = (gptr)(bbase + j * bstep_blk + s * (TERMS * 512));
+        asm("" : "+s"(run));  // keeps the scalar and the lane's part apart
+        return run;
+    };
     const int64_t s_first = kbeg / 16, s_last = kend / 16 - 1;
 
     // generator: thread owns cell (tid % PCPR) of operator rows tid / PCPR + RPP i
@@ -397,8 +410,8 @@ __global__ __launch_bounds__(BF_FTHR, 1) void bf16_skge_pair_kernel(Bf16Problem 
             for (int j = 0; j < CB; ++j) {
                 int64_t s_ld = s_first + bd;
                 if (s_ld > s_last) s_ld = s_last;
-                bq[bd][j][tt] = __builtin_bit_cast(
-                    bf16x8, *(const u32x4 *)(bbase + j * bstep_blk + s_ld * (TERMS * 512) + tt * 512));
+                bq[bd][j][tt] = load_b(run_of(j, s_ld), tt);
+                __builtin_amdgcn_sched_barrier(0);
             }
 
     // one 16-deep K step: block j's B operands for step s + BD are reloaded
@@ -414,6 +427,9 @@ __global__ __launch_bounds__(BF_FTHR, 1) void bf16_skge_pair_kernel(Bf16Problem 
 #if RBX_BF16_PRIO
         __builtin_amdgcn_s_setprio(RBX_BF16_PRIO);
 #endif
+        gptr run[CB];
+#pragma unroll
+        for (int j = 0; j < CB; ++j) run[j] = run_of(j, s_next);
         // term-outer: consecutive MFMAs on one accumulator are RB x CB apart,
         // and each accumulator still adds its terms in order hi, lo, lo2
 #pragma unroll
@@ -423,8 +439,10 @@ __global__ __launch_bounds__(BF_FTHR, 1) void bf16_skge_pair_kernel(Bf16Problem 
 #pragma unroll
                 for (int i = 0; i < RB; ++i)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], bq[bb][j][tt], acc[i][j], 0, 0, 0);
-                bq[bb][j][tt] = __builtin_bit_cast(
-                    bf16x8, *(const u32x4 *)(bbase + j * bstep_blk + s_next * (TERMS * 512) + tt * 512));
+                // after the MFMAs, into the registers they read: moved ahead of
+                // them it would take others (256 and spills)
+                __builtin_amdgcn_sched_barrier(0);
+                bq[bb][j][tt] = load_b(run[j], tt);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
