@@ -160,23 +160,19 @@ struct Bf16Problem {
     int64_t M, N, K, Kp, Np;
     GenMap g;
     const uint16_t *planes;  // fragment-packed terms (see split_kernel)
-    float *part;  // nS x M x N, row-major
+    float *part;  // nS x M x ldp, row-major
+    int64_t ldp;  // N rounded up to a multiple of 4
     int64_t kw;   // K per split (multiple of BF_KC)
     int nMB, nNB, nS;  // row blocks, column blocks and K-splits of the launch
-    int mb0;      // first row block of the launch
     int sp0;      // first K-split of the launch
 };
 
 // 32x32 output block, element r of lane l: row 8*(r/4) + 4*(l/32) + r%4, column l%32.
 __device__ __forceinline__ int out_row32(int lane, int r) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
 
-// FAST: the launched row blocks are interior (m0 + 64 <= M), K is a multiple
-// of the 32-deep chunk (so every chunk is inside the operator), N is a
-// multiple of 256 (every wave owns 8 valid column blocks), and the operator's
-// rows run along K from a counter boundary (b_off % 4 == 0).  Then each thread
-// owns two fixed Philox cells per chunk whose counters advance by 8 per chunk,
-// and no bounds logic is compiled in.  Row blocks start at pb.mb0.
-template <int TERMS, bool FAST>
+// The form for operators whose counters run along the output rows or whose
+// window starts inside a counter; every other call takes the pair kernel.
+template <int TERMS>
 __global__ __launch_bounds__(BF_NTHR, 1) void bf16_skge_kernel(Bf16Problem pb) {
     __shared__ __attribute__((aligned(16))) uint16_t Ss[2][BF_MT * BF_LDK];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -189,7 +185,7 @@ __global__ __launch_bounds__(BF_NTHR, 1) void bf16_skge_kernel(Bf16Problem pb) {
     const int rest = t / pb.nMB;
     const int nb = rest % pb.nNB;
     const int sp = rest / pb.nNB;
-    const int64_t m0 = (int64_t)(mb + pb.mb0) * BF_MT;
+    const int64_t m0 = (int64_t)mb * BF_MT;
     const int64_t n0 = (int64_t)nb * BF_NT;
     const int64_t kbeg = (int64_t)sp * pb.kw;
     int64_t kend = kbeg + pb.kw;
@@ -206,7 +202,7 @@ __global__ __launch_bounds__(BF_NTHR, 1) void bf16_skge_kernel(Bf16Problem pb) {
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
     const int64_t wcol = n0 + wave * 256;        // first column of this wave
-    const bool active = FAST || wcol < pb.Np;    // Np is a multiple of 256: all 8 blocks or none
+    const bool active = wcol < pb.Np;    // Np is a multiple of 256: all 8 blocks or none
     const int64_t KS = pb.Kp / 16;
     // lane's B operand for block j, K step s, term t:
     //   planes + (((wcol/32 + j)*KS + s)*TERMS + t)*512 + lane*8
@@ -214,28 +210,8 @@ __global__ __launch_bounds__(BF_NTHR, 1) void bf16_skge_kernel(Bf16Problem pb) {
     const int64_t bstep_blk = KS * (TERMS * 512);  // elements between column blocks
     const int64_t s_first = kbeg / 16, s_last = kend / 16 - 1;
 
-    // FAST generator cells: thread owns cell (tid & 7) of operator rows
-    // tid/8 and tid/8 + 32 of every chunk
-    const int frow = tid >> 3, fcell = tid & 7;
-    const uint64_t foff = FAST ? (uint64_t)((g.a_off + m0 + frow) * g.P + ((g.b_off + kbeg) >> 2) + fcell) : 0;
-    const uint64_t foff2 = foff + (uint64_t)(32 * g.P);
     auto gen_chunk = [&](int c, uint16_t *lds) {
-        if constexpr (FAST) {
-            const bool gauss = g.gauss != 0;
-#pragma unroll
-            for (int it = 0; it < 2; ++it) {
-                const float4 v = gen4(gauss, ctr_add(g.ctr, (it ? foff2 : foff) + 8 * (uint64_t)c), g.k0, g.k1);
-                uint2 pk;
-                pk.x = (uint32_t)entry_value<uint16_t>(v.x, gauss) |
-                       ((uint32_t)entry_value<uint16_t>(v.y, gauss) << 16);
-                pk.y = (uint32_t)entry_value<uint16_t>(v.z, gauss) |
-                       ((uint32_t)entry_value<uint16_t>(v.w, gauss) << 16);
-                *(uint2 *)(lds + (frow + 32 * it) * BF_LDK + fcell * 4) = pk;
-            }
-        } else {
-            gen_tile<uint16_t, BF_MT, BF_KC, BF_NTHR>(g, m0, kbeg + (int64_t)c * BF_KC, pb.M, pb.K, lds, BF_LDK, 1,
-                                                      tid);
-        }
+        gen_tile<uint16_t, BF_MT, BF_KC, BF_NTHR>(g, m0, kbeg + (int64_t)c * BF_KC, pb.M, pb.K, lds, BF_LDK, 1, tid);
     };
 
     bf16x8 bq[8][TERMS];
@@ -286,7 +262,7 @@ __global__ __launch_bounds__(BF_NTHR, 1) void bf16_skge_kernel(Bf16Problem pb) {
 
     // partial tile -> scratch (row-major M x N per split; lanes walk columns)
     if (!active) return;
-    float *P = pb.part + (int64_t)sp * pb.M * pb.N;
+    float *P = pb.part + (int64_t)sp * pb.M * pb.ldp;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -295,11 +271,11 @@ __global__ __launch_bounds__(BF_NTHR, 1) void bf16_skge_kernel(Bf16Problem pb) {
             for (int r = 0; r < 16; ++r) {
                 const int64_t gi = m0 + i * 32 + out_row32(lane, r);
                 const int64_t gj = wcol + j * 32 + (lane & 31);
-                if (FAST || (gi < pb.M && gj < pb.N)) P[gi * pb.N + gj] = acc[i][j][r];
+                if (gi < pb.M && gj < pb.ldp) P[gi * pb.ldp + gj] = acc[i][j][r];
             }
 }
 
-// Interior tiles, two waves per SIMD.  A 512-thread workgroup owns a
+// Two waves per SIMD.  A 512-thread workgroup owns a
 // (32 RB) x (256 CB) output tile; each of its 8 waves owns all 32 RB rows and
 // 32 CB columns of it (RB x CB blocks of 32 x 32, 16 RB CB accumulator
 // registers, so two waves fit on a SIMD).  The B operands a wave streams per
@@ -308,14 +284,16 @@ __global__ __launch_bounds__(BF_NTHR, 1) void bf16_skge_kernel(Bf16Problem pb) {
 // workgroup, so generation per output column grows as CB shrinks.  Every
 // thread generates RB/2 Philox cells of the next 32-deep chunk per chunk;
 // waves 0-3 generate before their MFMAs and waves 4-7 after them, so the two
-// waves sharing a SIMD (w and w + 4) are in opposite phases.  The same shape
-// conditions as the FAST form of bf16_skge_kernel apply, with the tile
-// (32 RB) x (256 CB).
+// waves sharing a SIMD (w and w + 4) are in opposite phases.  Any sizes: the
+// planes hold zeros past K and N (the operator entries there are whatever the
+// counters give), rows past M are not stored.  The operator's rows run along K
+// from a counter boundary.
 constexpr int BF_FTHR = 512;
 #ifndef RBX_BF16_TALL_RB
 #define RBX_BF16_TALL_RB 2
 #endif
 constexpr int BF_RB = RBX_BF16_TALL_RB, BF_CB = 8 / BF_RB;  // blocks per wave: RB x CB = 8
+static_assert(32 * BF_RB == BF_MT, "both kernels' row blocks are the same");
 // Wave priority while a wave issues its MFMAs (0: unchanged).
 #ifndef RBX_BF16_PRIO
 #define RBX_BF16_PRIO 1
@@ -346,7 +324,7 @@ __global__ __launch_bounds__(BF_FTHR, 1) void bf16_skge_pair_kernel(Bf16Problem 
     const int rest = t / pb.nMB;
     const int nb = rest % pb.nNB;
     const int sp = rest / pb.nNB + pb.sp0;
-    const int64_t m0 = (int64_t)(mb + pb.mb0) * MT;
+    const int64_t m0 = (int64_t)mb * MT;
     const int64_t n0 = (int64_t)nb * NT;
     const int64_t kbeg = (int64_t)sp * pb.kw;
     int64_t kend = kbeg + pb.kw;
@@ -472,7 +450,8 @@ __global__ __launch_bounds__(BF_FTHR, 1) void bf16_skge_pair_kernel(Bf16Problem 
     }
 
     // partial tile -> scratch (row-major M x N per split; lanes walk columns)
-    float *P = pb.part + (int64_t)sp * pb.M * pb.N;
+    float *P = pb.part + (int64_t)sp * pb.M * pb.ldp;
+    const bool inner = m0 + MT <= pb.M && n0 + NT <= pb.ldp;
 #pragma unroll
     for (int i = 0; i < RB; ++i)
 #pragma unroll
@@ -481,61 +460,51 @@ __global__ __launch_bounds__(BF_FTHR, 1) void bf16_skge_pair_kernel(Bf16Problem 
             for (int r = 0; r < 16; ++r) {
                 const int64_t gi = m0 + i * 32 + out_row32(lane, r);
                 const int64_t gj = wcol + j * 32 + (lane & 31);
-                P[gi * pb.N + gj] = acc[i][j][r];
+                if (inner || (gi < pb.M && gj < pb.ldp)) P[gi * pb.ldp + gj] = acc[i][j][r];
             }
 }
 
-// B[i,j] = alpha * sum_s part[s][i*N + j] + beta * B[i*brs + j*bcs], sums in
+// B[i,j] = alpha * sum_s part[s][i*ldp + j] + beta * B[i*brs + j*bcs], sums in
 // FP64 in split order.  RED_R x RED_C tiles (8 x 128): each row of a tile is
 // one 512-byte run of every partial (FP32), long enough for full HBM bursts;
 // a column-major B is written along i after a transpose through LDS.  A 1-D
 // grid of tiles, row-tile major.  With pre != nullptr the sums start from
-// pre[i*N + j], the FP64 sum of splits 0 .. s0 - 1 (bf16_presum_kernel), and
+// pre[i*ldp + j], the FP64 sum of splits 0 .. s0 - 1 (bf16_presum_kernel), and
 // continue with split s0: the same additions in the same order.
 constexpr int RED_R = 8, RED_C = 128;
-template <typename PT, typename OT>
-__global__ __launch_bounds__(256) void bf16_reduce_kernel(const PT *part, int nS, int64_t M, int64_t N,
-                                                          double alpha, double beta, OT *B, int64_t brs,
-                                                          int64_t bcs, const double *pre = nullptr,
-                                                          int s0 = 0) {
+__global__ __launch_bounds__(256) void bf16_reduce_kernel(const float *part, int nS, int64_t M, int64_t N, int64_t ldp,
+                                                          double alpha, double beta, float *B, int64_t brs,
+                                                          int64_t bcs, const double *pre, int s0) {
     __shared__ double tile[RED_R][RED_C + 1];
     const int64_t ntc = (N + RED_C - 1) / RED_C;
     const int64_t i0 = (int64_t)(blockIdx.x / ntc) * RED_R, j0 = (int64_t)(blockIdx.x % ntc) * RED_C;
-    const int64_t total = M * N;
+    const int64_t total = M * ldp;
     {
-        // thread: row r, columns c4 .. c4 + 3, 16-byte loads when whole and
-        // aligned; eight splits' loads are issued together and every sum stays
-        // in split order
+        // thread: row r, columns c4 .. c4 + 3, 16-byte loads; eight splits'
+        // loads are issued together and every sum stays in split order
+        typedef float pt4 __attribute__((ext_vector_type(4)));
         const int r = threadIdx.x / (RED_C / 4), c4 = 4 * (threadIdx.x % (RED_C / 4));
         const int64_t i = i0 + r, j = j0 + c4;
         double v[4] = {0.0, 0.0, 0.0, 0.0};
-        if (i < M) {
+        if (i < M && j < ldp) {
             if (pre != nullptr)
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (j + e < N) v[e] = pre[i * N + j + e];
-            const PT *p = part + i * N + j;
-            if (j + 3 < N && N % 4 == 0) {
-                typedef PT pt4 __attribute__((ext_vector_type(4)));
-                int s = s0;
-                for (; s + 8 <= nS; s += 8) {
-                    pt4 x[8];
+                for (int e = 0; e < 4; ++e) v[e] = pre[i * ldp + j + e];
+            const float *p = part + i * ldp + j;
+            int s = s0;
+            for (; s + 8 <= nS; s += 8) {
+                pt4 x[8];
 #pragma unroll
-                    for (int u = 0; u < 8; ++u) x[u] = *(const pt4 *)(p + (int64_t)(s + u) * total);
+                for (int u = 0; u < 8; ++u) x[u] = *(const pt4 *)(p + (int64_t)(s + u) * total);
 #pragma unroll
-                    for (int u = 0; u < 8; ++u)
+                for (int u = 0; u < 8; ++u)
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) v[e] += (double)x[u][e];
-                }
-                for (; s < nS; ++s) {
-                    const pt4 x = *(const pt4 *)(p + (int64_t)s * total);
+                    for (int e = 0; e < 4; ++e) v[e] += (double)x[u][e];
+            }
+            for (; s < nS; ++s) {
+                const pt4 x = *(const pt4 *)(p + (int64_t)s * total);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] += (double)x[e];
-                }
-            } else {
-                for (int e = 0; e < 4; ++e)
-                    if (j + e < N)
-                        for (int s = s0; s < nS; ++s) v[e] += (double)p[(int64_t)s * total + e];
+                for (int e = 0; e < 4; ++e) v[e] += (double)x[e];
             }
         }
 #pragma unroll
@@ -551,10 +520,10 @@ __global__ __launch_bounds__(256) void bf16_reduce_kernel(const PT *part, int nS
         const int64_t i = i0 + ti, j = j0 + tj;
         if (i < M && j < N) {
             const double v = tile[ti][tj];
-            OT *b = B + i * brs + j * bcs;
+            float *b = B + i * brs + j * bcs;
             double out = alpha * v;
             if (beta != 0.0) out += beta * (double)(*b);
-            *b = (OT)out;
+            *b = (float)out;
         }
     }
 }
@@ -662,10 +631,27 @@ static void bf16_split_sketch(char layout, char opS, char opA, int64_t d, int64_
     pb.N = N;
     pb.K = K;
     pb.Kp = (K + BF_KC - 1) / BF_KC * BF_KC;
-    pb.Np = (N + 255) / 256 * 256;
     pb.g = gen_map(*S, opS, ro_s, co_s, false);
+    // The pair kernel's tile is 256 cb columns wide.  A 32-deep chunk of a tile
+    // costs its MFMAs (also for the zero columns past N) and the operator's
+    // generation, about as much as those of 160 columns with three terms.
+    const bool pair = !pb.g.b_along_rows && (pb.g.b_off & 3) == 0;
+    int cb = BF_NT / 256;
+    if (pair) {
+        int64_t best = 0;
+        for (int c = BF_CB; c >= 1; c /= 2) {
+            const int64_t nb = (N + 256 * c - 1) / (256 * c), cost = nb * (256 * c * n_terms + 480);
+            if (c > 1 && nb * 8 * c > 65535) continue;  // the split's grid
+            if (best == 0 || cost < best) {
+                best = cost;
+                cb = c;
+            }
+        }
+    }
     pb.nMB = (int)((M + BF_MT - 1) / BF_MT);
-    pb.nNB = (int)((N + BF_NT - 1) / BF_NT);
+    pb.nNB = (int)((N + 256 * cb - 1) / (256 * cb));
+    pb.Np = pair ? (int64_t)pb.nNB * 256 * cb : (N + 255) / 256 * 256;
+    pb.ldp = (N + 3) / 4 * 4;
     // K per split: bounded FP32 accumulation chains, and enough workgroups
     int64_t kw = 4096;
     int64_t tiles = (int64_t)pb.nMB * pb.nNB;
@@ -679,21 +665,6 @@ static void bf16_split_sketch(char layout, char opS, char opA, int64_t d, int64_
     RBX_REQUIRE((int64_t)pb.nMB * pb.nNB * pb.nS < (1ll << 31));
 
 
-    // interior row blocks on the two-wave kernel when the shape allows it, the
-    // rest (or everything) on the bounds-checked kernel; the widest tile (256
-    // CB columns, CB = BF_CB, BF_CB / 2, BF_CB / 4) that divides N: narrow
-    // sketches keep the two-wave kernel
-    constexpr int TMT = 32 * BF_RB;
-    int cb = 0;
-    for (int c = BF_CB; c >= 1; c /= 2)
-        if (N % (256 * c) == 0) {
-            cb = c;
-            break;
-        }
-    const bool fast_ok = K % PKC == 0 && cb > 0 && !pb.g.b_along_rows && (pb.g.b_off & 3) == 0;
-    const int nfast = fast_ok ? (int)(M / TMT) : 0;   // row blocks of TMT rows
-    const int nMB_all = pb.nMB;                        // row blocks of BF_MT rows
-    const int nfast64 = nfast * (TMT / BF_MT);
     const bool vec = acs % 4 == 0 && ((uintptr_t)A & 15) == 0;
     const int64_t kt_total = (pb.Kp + SPL_KT - 1) / SPL_KT;
     RBX_REQUIRE(kt_total < (1ll << 31) && pb.Np / 32 <= 65535);
@@ -714,9 +685,6 @@ static void bf16_split_sketch(char layout, char opS, char opA, int64_t d, int64_
     auto main_fast = [&](int sp_first, int sp_count) {
         ProfScope prof("bf16_skge_kernel", stream);
         Bf16Problem q = pb;
-        q.nMB = nfast;
-        q.nNB = (int)(N / (256 * cb));
-        q.mb0 = 0;
         q.sp0 = sp_first;
         q.nS = sp_count;
         const dim3 grid((unsigned)(q.nMB * q.nNB * q.nS));
@@ -725,25 +693,23 @@ static void bf16_split_sketch(char layout, char opS, char opA, int64_t d, int64_
         else if (cb == BF_CB / 2) launch_pair<(BF_CB / 2 > 0 ? BF_CB / 2 : 1)>(n_terms, gs, grid, q, stream);
         else launch_pair<(BF_CB / 4 > 0 ? BF_CB / 4 : 1)>(n_terms, gs, grid, q, stream);
     };
-    // K-range pipeline: when every row block runs on the two-wave kernel, the
-    // split of later K ranges runs on the workspace's helper stream while the
+    // K-range pipeline of the pair kernel: the split of later K ranges runs on the workspace's helper stream while the
     // main kernel multiplies earlier ones (the split's lean waves fit beside
     // the main kernel's on each CU); the caller's stream waits for each range's
     // split before that range's product, so all helper work is joined before
     // the reduction.
     const int64_t tiles_per_split = pb.kw / SPL_KT;
-    const bool pipelined = ars == 1 && nfast > 0 && nMB_all == nfast64 && pb.nS >= 8 && pb.kw % SPL_KT == 0;
+    const bool pipelined = ars == 1 && pair && pb.nS >= 8 && pb.kw % SPL_KT == 0;
     // the pipeline also sums the first K ranges' partials on the helper
     // stream during the last range's product (FP64, M x N)
-    const bool presum = pipelined && (M * N) % 4 == 0;
     const size_t plane_elems = (size_t)safe_mul(pb.Kp, pb.Np);
     const size_t planes_bytes = ((size_t)n_terms * plane_elems * 2 + 255) / 256 * 256;
-    const size_t part_bytes = ((size_t)safe_mul(safe_mul(pb.nS, M), N) * 4 + 255) / 256 * 256;
-    const size_t pre_bytes = presum ? (size_t)safe_mul(M, N) * 8 : 0;
+    const size_t part_bytes = ((size_t)safe_mul(safe_mul(pb.nS, M), pb.ldp) * 4 + 255) / 256 * 256;
+    const size_t pre_bytes = pipelined ? (size_t)safe_mul(M, pb.ldp) * 8 : 0;
     char *ws = (char *)scratch(SCRATCH_BF16, planes_bytes + part_bytes + pre_bytes, stream);
     pb.planes = (const uint16_t *)ws;
     pb.part = (float *)(ws + planes_bytes);
-    double *pre = presum ? (double *)(ws + planes_bytes + part_bytes) : nullptr;
+    double *pre = pipelined ? (double *)(ws + planes_bytes + part_bytes) : nullptr;
     int pre_splits = 0;  // splits already in pre
     if (pipelined) {
         // four equal K ranges: only the first range's split runs alone (at the
@@ -766,7 +732,7 @@ static void bf16_split_sketch(char layout, char opS, char opA, int64_t d, int64_
         for (int c = 0; c < NCH; ++c) {
             if (c > 0) RBX_HIP(hipStreamWaitEvent(stream, ws_event(stream, c), 0));
             main_fast(sb[c], sb[c + 1] - sb[c]);
-            if (presum && c == NCH - 2) {
+            if (c == NCH - 2) {
                 // partials of ranges 0 .. NCH - 2 are complete: sum them on
                 // the helper stream while the last range is multiplied
                 hipEvent_t ready = ws_event(stream, NCH);
@@ -775,12 +741,12 @@ static void bf16_split_sketch(char layout, char opS, char opA, int64_t d, int64_
                 pre_splits = sb[NCH - 1];
                 ProfScope prof("bf16_presum_kernel", hs);
                 hipLaunchKernelGGL(bf16_presum_kernel, dim3((unsigned)num_cus() * 4), dim3(256), 0, hs,
-                                   (const float *)pb.part, pre_splits, M * N, pre);
+                                   (const float *)pb.part, pre_splits, M * pb.ldp, pre);
                 RBX_HIP(hipGetLastError());
                 RBX_HIP(hipEventRecord(ws_event(stream, NCH + 1), hs));
             }
         }
-        if (presum) RBX_HIP(hipStreamWaitEvent(stream, ws_event(stream, NCH + 1), 0));
+        RBX_HIP(hipStreamWaitEvent(stream, ws_event(stream, NCH + 1), 0));
     } else {
         if (ars == 1) {
             split_kunit(0, kt_total, stream);
@@ -793,23 +759,21 @@ static void bf16_split_sketch(char layout, char opS, char opA, int64_t d, int64_
                                pb.Np, n_terms, (uint16_t *)pb.planes);
             RBX_HIP(hipGetLastError());
         }
-        if (nfast > 0) main_fast(0, pb.nS);
-        if (nMB_all > nfast64) {
+        if (pair) {
+            main_fast(0, pb.nS);
+        } else {
             ProfScope prof("bf16_skge_kernel", stream);
-            Bf16Problem q = pb;
-            q.nMB = nMB_all - nfast64;
-            q.mb0 = nfast64;
-            dim3 grid((unsigned)(q.nMB * q.nNB * q.nS));
-            if (n_terms == 1) hipLaunchKernelGGL((bf16_skge_kernel<1, false>), grid, dim3(BF_NTHR), 0, stream, q);
-            else if (n_terms == 2) hipLaunchKernelGGL((bf16_skge_kernel<2, false>), grid, dim3(BF_NTHR), 0, stream, q);
-            else hipLaunchKernelGGL((bf16_skge_kernel<3, false>), grid, dim3(BF_NTHR), 0, stream, q);
+            const dim3 grid((unsigned)(pb.nMB * pb.nNB * pb.nS));
+            if (n_terms == 1) hipLaunchKernelGGL((bf16_skge_kernel<1>), grid, dim3(BF_NTHR), 0, stream, pb);
+            else if (n_terms == 2) hipLaunchKernelGGL((bf16_skge_kernel<2>), grid, dim3(BF_NTHR), 0, stream, pb);
+            else hipLaunchKernelGGL((bf16_skge_kernel<3>), grid, dim3(BF_NTHR), 0, stream, pb);
             RBX_HIP(hipGetLastError());
         }
     }
     {
         const dim3 grid = reduce_grid(M, N);
         ProfScope prof("bf16_reduce_kernel", stream);
-        hipLaunchKernelGGL((bf16_reduce_kernel<float, float>), grid, dim3(256), 0, stream, pb.part, pb.nS, M, N,
+        hipLaunchKernelGGL(bf16_reduce_kernel, grid, dim3(256), 0, stream, (const float *)pb.part, pb.nS, M, N, pb.ldp,
                            (double)alpha, (double)beta, B, brs, bcs, (const double *)pre, pre_splits);
         RBX_HIP(hipGetLastError());
     }

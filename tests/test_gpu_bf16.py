@@ -139,3 +139,14 @@ def test_narrow_tiles_identity_exact(rb, orc, n):
 def test_narrow_tiles_error(rb, orc, n):
     got, same, _ = _case(rb, orc, "C", "N", "N", 130, n, 8192, 3, alpha=0.75, beta=0.5, seed=4)
     assert rel_fro(got, same) <= 1e-6
+
+
+@pytest.mark.parametrize("terms,tol", [(3, 1e-6), (1, 4e-3)])
+@pytest.mark.parametrize("layout", ["C", "R"])
+@pytest.mark.parametrize("d,n,m", [(1, 1, 5), (63, 255, 31), (65, 257, 33), (64, 513, 4097), (200, 1025, 20001),
+                                   (130, 300, 9000)])
+def test_sizes_off_the_tiles(rb, orc, terms, tol, layout, d, n, m):
+    """Rows, columns and K around the two-wave kernel's 64-row, 256-column and
+    32-deep tiles, and enough K splits for the split's pipeline."""
+    got, same, _ = _case(rb, orc, layout, "N", "N", d, n, m, terms, alpha=0.5, beta=-2.0, seed=d)
+    assert rel_fro(got, same) <= tol

@@ -574,3 +574,50 @@ def test_one_column_beta_zero_ignores_nan(rb):
     y = torch.full((20,), float("nan"), dtype=torch.float64, device=DEV)
     rb.lskge3("C", "N", "N", 20, 1, 5000, 1.0, S, 0, 0, x, 5000, 0.0, y, 20)
     assert bool(torch.isfinite(y).all())
+
+
+# ---------------------------------------------------------------- sizes off the tiles
+TILE_EDGES = [(2, 4), (31, 3), (32, 5), (33, 31), (64, 33), (65, 64), (129, 1000), (132, 997), (192, 96), (193, 63),
+              (257, 2049), (260, 100), (320, 40), (321, 70), (384, 34), (448, 129), (449, 65), (512, 32), (513, 95),
+              (641, 96), (768, 33), (1025, 64)]
+
+
+@pytest.mark.parametrize("dtype,tol", [(np.float64, 1e-13), (np.float32, 1e-5)])
+@pytest.mark.parametrize("layout", ["C", "R"])
+@pytest.mark.parametrize("n,m", TILE_EDGES)
+def test_lskge3_tile_edges(rb, orc, dtype, tol, layout, n, m):
+    """Columns around every tile width, K around the 32-deep chunks, operator
+    windows that start inside a counter, both unit strides of A, both counter
+    orientations and families."""
+    got, ref = run_lskge3(rb, orc, dtype, layout, "N", "N", 67, n, m, 0.5, -1.5, ro=n % 4, co=(n // 3) % 4,
+                          pad=(n % 3, 1), axis="LS"[n // 2 % 2], fam="GU"[m % 2], seed=n)
+    assert rel_fro(got, ref) <= tol
+
+
+@pytest.mark.parametrize("layout", ["C", "R"])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_lskge3_nonfinite_data_stays_in_its_column(rb, layout, bad):
+    """K = 33 reaches one row into a chunk whose other rows do not exist, and
+    the operator's window starts inside a counter: an infinity (a NaN) in A's
+    first or last row gives infinities (NaNs) in its column of B alone."""
+    d, n, m = 70, 40, 33
+    A = np.random.default_rng(1).standard_normal((m, n))
+    A[0, 3] = A[m - 1, 7] = bad
+    S = rb.DenseSkOp(rb.DenseDist(d, m + 1), rb.RNGState(5))
+    flat = A.T.reshape(-1) if layout == "C" else A.reshape(-1)
+    B = torch.empty(d * n, dtype=torch.float64, device=DEV)
+    rb.lskge3(layout, "N", "N", d, n, m, 1.0, S, 0, 1, dev(np.ascontiguousarray(flat)), m if layout == "C" else n, 0.0,
+              B, d if layout == "C" else n)
+    got = host(B).reshape(n, d).T if layout == "C" else host(B).reshape(d, n)
+    hit = np.isinf(got) if np.isinf(bad) else np.isnan(got)
+    assert hit[:, [3, 7]].all() and np.isfinite(np.delete(got, [3, 7], axis=1)).all()
+
+
+@pytest.mark.parametrize("opS", ["N", "T"])
+@pytest.mark.parametrize("n,m,co", [(40, 50, 1), (130, 1111, 2), (600, 4100, 3)])
+def test_materialised_operator_same_bits(rb, orc, opS, n, m, co):
+    """A filled operator takes the generated one's places in the product."""
+    a, ref = run_lskge3(rb, orc, np.float64, "C", opS, "N", 90, n, m, 1.0, 0.0, ro=2, co=co, materialise=True)
+    b, _ = run_lskge3(rb, orc, np.float64, "C", opS, "N", 90, n, m, 1.0, 0.0, ro=2, co=co)
+    assert np.array_equal(a, b)
+    assert rel_fro(a, ref) <= 1e-13
