@@ -189,6 +189,35 @@ def test_cdf_search_unsorted_array_bit_exact(rb, orc, dtype):
     assert np.array_equal(host(s), ref)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [1, 2, 65535, 65536, 65537, 150001])
+@pytest.mark.parametrize("kind", ["even", "ties", "steps", "outside", "unsorted", "nan"])
+def test_cdf_search_by_table_bit_exact(rb, orc, dtype, n, kind):
+    """Enough draws for the table search (a multiple of four is not among them), around the size
+    from which it looks at eight entries first: equal entries, long runs of entries whose 31-bit
+    keys agree, values below 0 and above 1, and arrays that are not ascending, which take
+    lower_bound's plain probe sequence."""
+    rng = np.random.default_rng(n + len(kind))
+    a = np.sort(rng.random(n))
+    if kind == "ties":
+        a = np.sort(rng.choice(rng.random(max(1, n // 50)), n))
+    elif kind == "steps":  # half of the entries within 2^-34 of 1/2, a run of zeros in front
+        a = np.sort(np.where(rng.random(n) < 0.5, 0.5 + rng.random(n) * 2.0 ** -34, rng.random(n)))
+        a[:n // 10] = 0.0
+    elif kind == "outside":
+        a = np.sort(3.0 * a - 1.0)
+    elif kind == "unsorted":
+        a = rng.random(n)
+    elif kind == "nan":
+        a[n // 2] = np.nan
+    a = a.astype(dtype)
+    k = 50003
+    s = torch.empty(k, dtype=torch.int64, device=DEV)
+    rb.sample_indices_iid(n, torch.from_numpy(a).to(DEV), k, s, rb.RNGState(key=9, counter=(1, 0, 0, 0)))
+    ref, _ = orc.sample_indices_iid(n, a, k, [1, 0, 0, 0], [9, 0])
+    assert np.array_equal(host(s), ref)
+
+
 # ---------------------------------------------------------------- power-law sparse test data
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("m,n,k,expo,ctr", [(1000, 500, 20000, 2.1, 0), (37, 3, 500, 1.5, 5), (1, 10, 7, 3.0, 2),
