@@ -313,17 +313,18 @@ rbx_status rbx_sparse_skop_free(rbx_sparse_skop *S);
  * every call, coo_spmm_impl.hh:69-91).  For callers that apply one sampled
  * operator many times: builds S->prep from S's current arrays (replacing any
  * earlier copy), so that later lskges calls over the whole operator
- * (ro_s = co_s = 0, d x m = the operator's shape, opS = 'N') with op(A) of unit
- * stride along the contraction skip the per-call sort; results are unchanged
- * bit for bit.  Leaves S->prep NULL, and returns RBX_OK, when the operator is
+ * (ro_s = co_s = 0, d x m = the operator's shape, opS = 'N') skip the per-call
+ * sort; results are unchanged bit for bit.  Leaves S->prep NULL, and returns RBX_OK, when the operator is
  * outside that path (more than 8192 rows, rows of more than 2048 entries on
  * average, a copy above four times the operator's own bytes) or the memory
  * cannot be had.  It finds whether every value is +1 or -1 (as a SASO's
- * are), so that the applies take the signs from the copy's layout and read no
- * values; that check synchronises `stream` once.  The copy is complete when
+ * are), so that the applies to op(A) of unit stride along the contraction take
+ * the signs from the copy's layout and read no values, and whether its rows
+ * are alike; that synchronises `stream` once.  The copy is complete when
  * `stream` reaches this call; it stays valid until S's arrays change, which
  * callers that write them in place signal by calling this again or
- * rbx_sparse_skop_free.  rbx_[sd]fill_sparse_skop calls it itself. */
+ * rbx_sparse_skop_free.  rbx_[sd]fill_sparse_skop does the same itself (and
+ * knows a SASO's values, so it does not synchronise for it). */
 rbx_status rbx_ssparse_skop_prepare(rbx_sparse_skop *S, void *stream);
 rbx_status rbx_dsparse_skop_prepare(rbx_sparse_skop *S, void *stream);
 

@@ -839,6 +839,123 @@ static void launch_rows_vec(bool colmaj, const int64_t *rowptr, const IDX *colid
     RBX_HIP(hipGetLastError());
 }
 
+// Few sparse rows (an operator's) times a row-major Bm of any alignment and
+// leading dimension, C = alpha * A * Bm + beta * C: one wave per row of A and
+// 64 * VEC columns, so a row's columns and values are wave-uniform (scalar
+// loads) and a gather is one contiguous load.  2 U gathers are in flight: the
+// next batch's are issued before a batch is applied.  Per output entry the
+// entries are applied in stored order (CRV_KIB or CRV_JKI above).
+//
+// Bound by the gathered bytes out of the L2s (the rows of a stripe drift apart
+// by more of Bm than an XCD's L2 holds).  S 1500 x 100003, 8 entries a column,
+// prepared, times a row-major 100003 x 333, FP32 / FP64: 198 / 356 us, 5.4 / 6
+// TB/s of gathers, where csr_rows_vec_kernel (94 workgroups of 32 rows, four
+// gathers in flight, Bm copied to aligned rows, the operator sorted again) took
+// 445 / 580; 1000 x 300000 times 40 columns, FP32: 404 us against 1325.  The
+// LDS apply of the column-major case, its tiles loaded from the rows instead,
+// took 335 / 366 us (a tile's 16 or 32 bytes of a row cost a 128-byte line) and
+// is slower still where the sketch has more rows (8000 x 100000, n = 1000, FP32:
+// 1617 us against 478).
+template <typename T, int VEC, bool KIB, int U>
+__global__ __launch_bounds__(256) void csr_stripe_kernel(const int64_t *__restrict__ rowptr,
+                                                         const int32_t *__restrict__ colidx,
+                                                         const T *__restrict__ vals, int64_t mrows, int64_t n, T alpha,
+                                                         T beta, const T *__restrict__ B, int64_t ldb, T *C,
+                                                         int64_t crs, int64_t ccs, int64_t lrow, int nrb, int nstripes) {
+    typedef T V __attribute__((ext_vector_type(VEC), aligned(sizeof(T))));
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    // XCD-aware order: the rows of one stripe on one XCD, whose L2 then holds
+    // the part of Bm that they are all going through
+    const int W = nrb * nstripes, xcd = blockIdx.x % 8, xi = blockIdx.x / 8;
+    const int t = xcd * (W / 8) + (xcd < W % 8 ? xcd : W % 8) + xi;
+    const int64_t i = 4 * (int64_t)(t % nrb) + wave;
+    if (i >= mrows) return;
+    const int64_t p0 = rowptr[i], p1 = rowptr[i + 1];
+    if (p1 - p0 > lrow) return;  // a long row: summed in segments elsewhere
+    // the lane's columns, moved back inside the matrix at its edge
+    const int64_t own = (int64_t)(t / nrb) * (64 * VEC) + lane * VEC;
+    const int64_t cl = own > n - VEC ? n - VEC : own;
+    T *Ci = C + i * crs + cl * ccs;
+    T acc[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) acc[e] = beta != (T)0 && cl + e >= own ? beta * Ci[e * ccs] : (T)0;
+    if (p1 > p0) {
+        const T *Bl = B + cl;
+        auto load = [&](int64_t p, V(&g)[U], T(&v)[U]) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int64_t q = p + u < p1 ? p + u : p1 - 1;  // past the end: the last entry again, not applied
+                v[u] = vals[q];
+                g[u] = *(const V *)(Bl + (int64_t)colidx[q] * ldb);
+            }
+        };
+        auto apply = [&](int64_t p, const V(&g)[U], const T(&v)[U]) {
+            const int cnt = p1 - p < U ? (int)(p1 - p) : U;
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (u < cnt) {
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e)
+                        acc[e] = KIB ? acc[e] + (alpha * v[u]) * g[u][e] : acc[e] + v[u] * (alpha * g[u][e]);
+                }
+        };
+        V g0[U], g1[U];
+        T v0[U], v1[U];
+        load(p0, g0, v0);
+        for (int64_t p = p0; p < p1; p += 2 * U) {
+            load(p + U, g1, v1);
+            apply(p, g0, v0);
+            load(p + 2 * U, g0, v0);
+            apply(p + U, g1, v1);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < VEC; ++e)
+        if (cl + e >= own) Ci[e * ccs] = acc[e];
+}
+
+// Columns per lane: the widest loads whose last stripe is not mostly empty.
+// Weights from the measured times at full stripes (FP32 1000 columns: 691, 522,
+// 464 us with 1, 2, 4; FP64 500 columns: 486, 457).
+template <typename T>
+static int stripe_vec(int64_t n) {
+    constexpr bool F64 = sizeof(T) == 8;
+    auto gain = [&](int vec, double w) {
+        const int64_t cw = 64 * vec;
+        return n < vec ? 0.0 : w * (double)n / (double)((n + cw - 1) / cw * cw);
+    };
+    const double g1 = gain(1, F64 ? 0.92 : 0.8), g2 = gain(2, 1.0), g4 = F64 ? 0.0 : gain(4, 1.08);
+    return g4 > g2 && g4 > g1 ? 4 : (g2 > g1 ? 2 : 1);
+}
+
+// C = alpha * A * Bm + beta * C by csr_stripe_kernel; rows longer than lrow are left out.
+template <typename T>
+static void launch_stripes(const int64_t *rowptr, const int32_t *colidx, const T *vals, int64_t mrows, int64_t n,
+                           T alpha, T beta, const T *B, int64_t ldb, T *C, int64_t crs, int64_t ccs, bool kib,
+                           int64_t lrow, hipStream_t st) {
+    const int vec = stripe_vec<T>(n);
+    const int64_t nrb = (mrows + 3) / 4, ns = (n + 64 * vec - 1) / (64 * vec);
+    RBX_REQUIRE(nrb < (1ll << 31) / ns);
+    const dim3 grid((unsigned)(nrb * ns));
+    auto go = [&](auto vc, auto form) {
+        hipLaunchKernelGGL((csr_stripe_kernel<T, decltype(vc)::value, decltype(form)::value, 8>), grid, dim3(256), 0,
+                           st, rowptr, colidx, vals, mrows, n, alpha, beta, B, ldb, C, crs, ccs, lrow, (int)nrb,
+                           (int)ns);
+    };
+    auto with_form = [&](auto vc) {
+        if (kib) go(vc, std::true_type{});
+        else go(vc, std::false_type{});
+    };
+    if (vec == 1) with_form(std::integral_constant<int, 1>{});
+    else if (vec == 2) with_form(std::integral_constant<int, 2>{});
+    else if constexpr (sizeof(T) == 4) with_form(std::integral_constant<int, 4>{});
+    RBX_HIP(hipGetLastError());
+}
+// Mean row length up to which a row stays one wave's chain (each entry of a
+// row takes about 0.15 us then: 1500 entries 136 us, 6000 entries 703 us, where
+// the segment sums of the row kernels take 293).
+constexpr int64_t STRIPE_MAX_MEAN_ROW = 4096;
+
 // Longest mean row (stored entries per output row) the LDS apply takes: each
 // output is one thread's sequential chain, so rows much longer than this are
 // better served by the row kernels' segment sums.
@@ -862,6 +979,7 @@ struct SparsePrep {
     char *lay;
     size_t lay_bytes;
     bool unit;  // every value is exactly +1 or -1 (the layout carries the signs)
+    int64_t max_row;  // entries of the longest row (0: rows known to be alike)
 };
 constexpr uint64_t PREP_MAGIC = 0x70657270787862ull;
 // the copy may take at most this many times the operator's own bytes
@@ -949,7 +1067,11 @@ static void left_spmm_coo(char layout, char opA, char opB, int64_t d, int64_t n,
             RBX_FAIL(RBX_UNSUPPORTED, "%s: shape outside the allocation-free path", __func__);
         return;
     }
-    {
+    if (prep != nullptr) {
+        row_ptr = prep->row_ptr;
+        ccol = prep->col;
+        cval = (T *)prep->val;
+    } else {
         ProfScope prof("coo_to_csr", st);
         // few output rows: stable counting sort by row; otherwise a radix
         // sort on the (row, column) key
@@ -971,6 +1093,16 @@ static void left_spmm_coo(char layout, char opA, char opB, int64_t d, int64_t n,
         if (csr_lds_apply<T>(row_ptr, ccol, cval, d, n, m, nnz, alpha, beta, B, ldb, C, crs, ccs,
                              kib ? SPF_KIB : SPF_JKI, lws, wsb, st, unit))
             return;
+    }
+    if (brs != 1 && d <= CSRB_MAX_ROWS && nnz <= STRIPE_MAX_MEAN_ROW * d) {
+        ProfScope prof("csr_apply_kernel", st);
+        // an operator whose rows are known to be alike has none to split
+        const bool even = unit || (prep != nullptr && prep->max_row <= long_row_threshold(nnz, d));
+        const int64_t lrow = even ? INT64_MAX
+                                  : launch_long_rows<T, int32_t>(row_ptr, ccol, cval, d, nnz, n, alpha, beta, B, ldb,
+                                                                 C, crs, ccs, st);
+        launch_stripes<T>(row_ptr, ccol, cval, d, n, alpha, beta, B, ldb, C, crs, ccs, kib != 0, lrow, st);
+        return;
     }
     {
         ProfScope prof("csr_apply_kernel", st);
@@ -1050,7 +1182,15 @@ static void prep_free(rbx_sparse_skop *S) {
     delete p;
 }
 
-__global__ void prep_flag_zero_kernel(int *f) { *f = 0; }
+__global__ void prep_flag_zero_kernel(int *f) { f[0] = f[1] = 0; }
+// f[1] = entries of the longest row (nnz fits 31 bits where this is used)
+__global__ __launch_bounds__(256) void longest_row_kernel(const int64_t *rowptr, int64_t mrows, int *f) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    int len = i < mrows ? (int)(rowptr[i + 1] - rowptr[i]) : 0;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) len = max(len, __shfl_xor(len, off));
+    if ((threadIdx.x & 63) == 0) atomicMax(f + 1, len);
+}
 // *f |= 1 when some value is not exactly +1 or -1 (one atomic per wave that saw one)
 template <typename T>
 __global__ __launch_bounds__(256) void unit_values_kernel(const T *v, int64_t n, int *f) {
@@ -1061,28 +1201,16 @@ __global__ __launch_bounds__(256) void unit_values_kernel(const T *v, int64_t n,
 }
 
 // rbx_[sd]sparse_skop_prepare: S->prep for S's current arrays, or null when
-// the operator is outside the LDS apply or the memory cannot be had.  Finding
-// whether every value is +1 or -1 (a SASO's are) reads one flag back, so this
-// synchronises the stream.
+// the operator is outside the LDS apply or the memory cannot be had.  Whether
+// every value is +1 or -1 and the longest row are read back, so this
+// synchronises the stream, except for a SASO sampled by the caller
+// (`sampled_saso`), whose values are and whose rows are alike.
 template <typename T>
-static void prepare_skop(rbx_sparse_skop *S, hipStream_t st) {
+static void prepare_skop(rbx_sparse_skop *S, hipStream_t st, bool sampled_saso = false) {
     prep_free(S);
     if (S->nnz <= 0 || S->vals == nullptr || S->rows == nullptr || S->cols == nullptr) return;
     const int64_t d = S->dist.n_rows, m = S->dist.n_cols, nnz = S->nnz;
     if (d > CSRB_MAX_ROWS || nnz > LDS_APPLY_MAX_MEAN_ROW * d || m >= (int64_t)INT32_MAX) return;
-    bool unit = false;
-    {
-        int *f = (int *)scratch(SCRATCH_SMALL, sizeof(int), st);
-        hipLaunchKernelGGL(prep_flag_zero_kernel, dim3(1), dim3(1), 0, st, f);
-        int64_t nb = (nnz + 255) / 256;
-        if (nb > 4 * (int64_t)num_cus()) nb = 4 * (int64_t)num_cus();
-        hipLaunchKernelGGL((unit_values_kernel<T>), dim3((unsigned)nb), dim3(256), 0, st, (const T *)S->vals, nnz, f);
-        RBX_HIP(hipGetLastError());
-        int h = 1;
-        RBX_HIP(hipMemcpyAsync(&h, f, sizeof(h), hipMemcpyDeviceToHost, st));
-        RBX_HIP(hipStreamSynchronize(st));
-        unit = h == 0;
-    }
     const size_t lay = csr_lds_apply_ws_bytes(d, m, nnz, sizeof(T));
     const size_t bR = align256((size_t)(d + 1) * 8), bC = align256((size_t)nnz * 4);
     const size_t bV = align256((size_t)nnz * sizeof(T));
@@ -1093,6 +1221,18 @@ static void prepare_skop(rbx_sparse_skop *S, hipStream_t st) {
     T *cval;
     if (!csr_build_counting<T>(S->rows, S->cols, (const T *)S->vals, nnz, 0, 0, d, m, &row_ptr, &ccol, &cval, st))
         return;
+    // f[0]: some value is not +1 or -1 (the layout kernel reads it there), f[1]: the longest row
+    int *f = nullptr;
+    if (!sampled_saso) {
+        f = (int *)scratch(SCRATCH_SMALL, 2 * sizeof(int), st);
+        hipLaunchKernelGGL(prep_flag_zero_kernel, dim3(1), dim3(1), 0, st, f);
+        int64_t nb = (nnz + 255) / 256;
+        if (nb > 4 * (int64_t)num_cus()) nb = 4 * (int64_t)num_cus();
+        hipLaunchKernelGGL((unit_values_kernel<T>), dim3((unsigned)nb), dim3(256), 0, st, (const T *)S->vals, nnz, f);
+        hipLaunchKernelGGL(longest_row_kernel, dim3((unsigned)((d + 255) / 256)), dim3(256), 0, st,
+                           (const int64_t *)row_ptr, d, f);
+        RBX_HIP(hipGetLastError());
+    }
     int dev = -1;
     RBX_HIP(hipGetDevice(&dev));
     char *mem = nullptr;
@@ -1116,12 +1256,22 @@ static void prepare_skop(rbx_sparse_skop *S, hipStream_t st) {
     p->val = mem + bR + bC;
     p->lay = mem + bR + bC + bV;
     p->lay_bytes = lay;
-    p->unit = unit;
     S->prep = p;  // owned by S from here, so prep_free releases it on any failure below
     RBX_HIP(hipMemcpyAsync(p->row_ptr, row_ptr, (size_t)(d + 1) * 8, hipMemcpyDeviceToDevice, st));
     RBX_HIP(hipMemcpyAsync(p->col, ccol, (size_t)nnz * 4, hipMemcpyDeviceToDevice, st));
     RBX_HIP(hipMemcpyAsync(p->val, cval, (size_t)nnz * sizeof(T), hipMemcpyDeviceToDevice, st));
-    if (!csr_lds_layout<T>(p->row_ptr, p->col, (const T *)p->val, d, m, nnz, p->lay, lay, st, unit)) prep_free(S);
+    if (!csr_lds_layout<T>(p->row_ptr, p->col, (const T *)p->val, d, m, nnz, p->lay, lay, st, true, f)) {
+        prep_free(S);
+        return;
+    }
+    p->unit = true;
+    p->max_row = 0;
+    if (f == nullptr) return;
+    int h[2] = {1, 0};
+    RBX_HIP(hipMemcpyAsync(h, f, sizeof(h), hipMemcpyDeviceToHost, st));
+    RBX_HIP(hipStreamSynchronize(st));
+    p->unit = h[0] == 0;
+    p->max_row = h[1];
 }
 
 template <typename T>
@@ -1562,7 +1712,7 @@ static void fill_sparse_skop(rbx_sparse_skop *S, hipStream_t st) {
     RBX_REQUIRE(S->vals != nullptr && S->rows != nullptr && S->cols != nullptr);
     prep_free(S);
     S->nnz = fill_sparse_impl<T>(S->dist, (T *)S->vals, S->rows, S->cols, S->seed_state, nullptr, st);
-    prepare_skop<T>(S, st);
+    prepare_skop<T>(S, st, S->dist.major_axis == 'S');
 }
 
 // ---------------------------------------------------------------- allocation-free lskges

@@ -55,10 +55,11 @@ size_t csr_lds_apply_ws_bytes(int64_t d, int64_t m, int64_t nnz, size_t val_size
 // into `ws`, then any number of applies that read it.  Each returns false,
 // with nothing launched, when the shape is outside what the kernel takes.
 // `unit` (the layout's: every value is exactly +1 or -1) lets the applies
-// take each value's sign from its slot instead of loading the value.
+// take each value's sign from its slot instead of loading the value; with
+// `other` the layout is a unit one where *other, on the device, is zero.
 template <typename T>
 bool csr_lds_layout(const int64_t *row_ptr, const int32_t *col, const T *val, int64_t d, int64_t m, int64_t nnz,
-                    char *ws, size_t ws_bytes, hipStream_t st, bool unit);
+                    char *ws, size_t ws_bytes, hipStream_t st, bool unit, const int *other = nullptr);
 template <typename T>
 bool csr_lds_apply_laid(const int64_t *row_ptr, const int32_t *col, const T *val, int64_t d, int64_t n, int64_t m,
                         int64_t nnz, T alpha, T beta, const T *B, int64_t ldb, T *C, int64_t crs, int64_t ccs,

@@ -444,7 +444,8 @@ template <typename T>
 __global__ __launch_bounds__(256) void csr_chunk_slots_kernel(const int64_t *row_ptr, const int32_t *col,
                                                               const T *val, int64_t d, int CK,
                                                               const int32_t *startT, T *Ev, uint16_t *Ep,
-                                                              int unit) {
+                                                              int unit_arg, const int *other) {
+    const bool unit = unit_arg != 0 && (other == nullptr || *other == 0);
     for (int64_t r = blockIdx.x; r < d; r += gridDim.x) {
         const int64_t p1 = row_ptr[r + 1];
         for (int64_t p = row_ptr[r] + threadIdx.x; p < p1; p += blockDim.x) {
@@ -719,7 +720,7 @@ static bool lds_apply_fits(int64_t d, int64_t m, size_t val_size) {
 
 template <typename T>
 bool csr_lds_layout(const int64_t *row_ptr, const int32_t *col, const T *val, int64_t d, int64_t m, int64_t nnz,
-                    char *ws, size_t ws_bytes, hipStream_t st, bool unit) {
+                    char *ws, size_t ws_bytes, hipStream_t st, bool unit, const int *other) {
     if (!lds_apply_fits(d, m, sizeof(T)) || ws == nullptr) return false;
     const LaPlan pl = la_plan(d, m, nnz, sizeof(T));
     RBX_REQUIRE(ws_bytes >= pl.bytes());
@@ -734,7 +735,7 @@ bool csr_lds_layout(const int64_t *row_ptr, const int32_t *col, const T *val, in
     const int64_t cus = num_cus();
     const int64_t sg = d < 4 * cus ? d : 4 * cus;
     hipLaunchKernelGGL((csr_chunk_slots_kernel<T>), dim3((unsigned)sg), dim3(256), 0, st, row_ptr, col, val, d, pl.ck,
-                       (const int32_t *)startT, Ev, Ep, (int)unit);
+                       (const int32_t *)startT, Ev, Ep, (int)unit, other);
     RBX_HIP(hipGetLastError());
     return true;
 }
@@ -799,9 +800,9 @@ template bool csr_lds_apply<float>(const int64_t *, const int32_t *, const float
                                    int64_t, float, float, const float *, int64_t, float *, int64_t, int64_t, int,
                                    char *, size_t, hipStream_t, bool);
 template bool csr_lds_layout<float>(const int64_t *, const int32_t *, const float *, int64_t, int64_t, int64_t,
-                                    char *, size_t, hipStream_t, bool);
+                                    char *, size_t, hipStream_t, bool, const int *);
 template bool csr_lds_layout<double>(const int64_t *, const int32_t *, const double *, int64_t, int64_t, int64_t,
-                                     char *, size_t, hipStream_t, bool);
+                                     char *, size_t, hipStream_t, bool, const int *);
 template bool csr_lds_apply_laid<float>(const int64_t *, const int32_t *, const float *, int64_t, int64_t, int64_t,
                                         int64_t, float, float, const float *, int64_t, float *, int64_t, int64_t, int,
                                         const char *, size_t, hipStream_t, bool);

@@ -746,3 +746,43 @@ def test_lskges_prepared_wide(rb, orc, axis, k, layout, opA, alpha, beta, dtype)
     prof = rb.profile_collect()
     assert "coo_to_csr" not in prof and "csr_lds_apply_kernel" in prof
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("prefill", [False, True])
+@pytest.mark.parametrize("layout,opA", [("R", "N"), ("C", "T")])
+@pytest.mark.parametrize("n", [1, 2, 3, 63, 65, 129, 257, 333])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_lskges_row_major_stripes(rb, orc, n, layout, opA, prefill, dtype):
+    """op(A) with unit stride along the columns, rows that start at any element: every width of a
+    lane's loads (1, 2, 4 columns), last stripes moved back inside the matrix, both summation forms,
+    the operator sampled in the call and prepared.  Bit-identical to the oracle."""
+    d, m = 37, 2003
+    got, ref = _lsk(rb, orc, dtype, layout, "N", opA, (d, m), 6, "S", d, n, m, 0, 0, 0.75, -0.5, prefill=prefill)
+    assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("prepared", [False, True])
+@pytest.mark.parametrize("dtype,tol", [(np.float64, 1e-13), (np.float32, 1e-5)])
+def test_lskges_row_major_uneven_rows(rb, orc, dtype, tol, prepared):
+    """Row-major op(A), an operator with one row of 3000 entries among rows of about 20 and empty
+    ones: the long row is summed in segments, the others stay bit-identical."""
+    rng = np.random.default_rng(9)
+    d, m, n = 300, 20000, 65
+    r = np.concatenate([rng.integers(10, d, 6000), np.full(3000, 4)])
+    c = np.concatenate([rng.integers(0, m, 6000), rng.permutation(m)[:3000]])
+    v = rng.uniform(-2, 2, len(r)).astype(dtype)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+    S = rb.SparseSkOp(rb.SparseDist(d, m, 8), rb.RNGState(5), dtype=torch.float64 if dtype == np.float64 else torch.float32)
+    S.vals, S.rows, S.cols, S.nnz = t(v), t(r.astype(np.int64)), t(c.astype(np.int64)), len(v)
+    if prepared:
+        S.prepare()
+    A = rng.uniform(-1, 1, m * n).astype(dtype)
+    B = t(np.full(d * n, np.nan, dtype))
+    rb.lskges("R", "N", "N", d, n, m, 1.0, S, 0, 0, t(A), n, 0.0, B, n)
+    ref = np.zeros(d * n, dtype)
+    orc.left_spmm_coo("d" if dtype == np.float64 else "s", "R", "N", "N", d, n, m, 1.0, (d, m), v,
+                      r.astype(np.int64), c.astype(np.int64), 0, 0, A, n, 0.0, ref, n)
+    got, ref = host(B).reshape(d, n), ref.reshape(d, n)
+    others = np.arange(d) != 4
+    assert np.array_equal(got[others], ref[others])
+    assert np.linalg.norm(got[4] - ref[4]) <= tol * np.linalg.norm(ref[4])
