@@ -199,6 +199,12 @@ __device__ __forceinline__ float entry_value<float>(float v, bool gauss) {
     return gauss ? v : __fmul_rn(v, 0x1.bb67aep+0f);  // (float)sqrt(3.0)
 }
 
+// The factor of entry_value: (T)v * entry_scale<T>(gauss) are the same bits.
+template <typename T>
+__host__ __device__ constexpr T entry_scale(bool gauss) {
+    return gauss ? (T)1 : (sizeof(T) == 8 ? (T)0x1.bb67ae8584caap+0 : (T)0x1.bb67aep+0f);
+}
+
 // bfloat16 (as its 16 bits) nearest to x, ties to even; x not NaN.
 __host__ __device__ __forceinline__ uint16_t bf16_rne(float x) {
 #ifdef __HIP_DEVICE_COMPILE__

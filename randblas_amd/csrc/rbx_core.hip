@@ -139,6 +139,14 @@ void *scratch(int slot, size_t bytes, hipStream_t stream) {
     return w.ptr[slot];
 }
 
+bool scratch_usable(int slot, size_t bytes, hipStream_t stream) {
+    if (stream_ws(stream).size[slot] >= bytes && bytes > 0) return true;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) == hipSuccess) return cap == hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
+}
+
 void *&stream_blas_handle(hipStream_t stream, void (**destroy)(void *)) {
     StreamWs &w = stream_ws(stream);
     *destroy = w.blas_destroy;

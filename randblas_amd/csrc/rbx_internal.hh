@@ -166,6 +166,9 @@ enum ScratchSlot { SCRATCH_BF16 = 0, SCRATCH_SPARSE_OP = 1, SCRATCH_SPARSE_CSR =
                    SCRATCH_SMALL = 4, SCRATCH_SPARSE_G = 5, SCRATCH_SPLITK = 6, SCRATCH_SOLVE = 7,
                    SCRATCH_SOLVE2 = 8, SCRATCH_LONG_ROWS = 9, SCRATCH_NSLOTS = 10 };
 void *scratch(int slot, size_t bytes, hipStream_t stream);
+// Whether scratch() may be called: not when it would have to grow the slot while
+// `stream` is captured (the memory would belong to the graph).
+bool scratch_usable(int slot, size_t bytes, hipStream_t stream);
 // A helper stream owned by `stream`'s workspace (non-blocking, default
 // priority) and up to WS_EVENTS events, for calls that overlap part of their
 // own work with the rest; such a call joins all helper work back into

@@ -680,21 +680,19 @@ static void iid_uniform_impl(int64_t n, int64_t k, int64_t *samples, T *rademach
 // (14-62 us against 18-204 us for 10^3 to 2^24 draws from 20000), longer ones
 // from a quarter as many draws on (10^6 entries, FP64: 2^17 draws 32 us either
 // way, 2^20 36 against 79 us, 2^24 178 against 875 us).  False, with nothing
-// launched, for the other sizes, without the memory, and while the stream is
-// captured (the table's memory belongs to the stream, not to the graph).
+// launched, for the other sizes and without the memory.
 constexpr int64_t CDF_NEAR_MIN = 1 << 16;
 template <typename T>
 static bool cdf_by_table(int64_t n, const T *cdf, int64_t k, int64_t *samples, Ctr128 ctr, const rbx_rng_state *state,
                          hipStream_t st) {
     if (n < 1 || n >= (int64_t)INT32_MAX || (n > CDF_NEAR_MIN && k < n / 4)) return false;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    RBX_HIP(hipStreamIsCapturing(st, &cap));
-    if (cap != hipStreamCaptureStatusNone) return false;
     const int64_t tb = std::min<int64_t>((std::max<int64_t>(n, CDF_BUCKETS + 1) + 255) / 256, CDF_TABLE_BLOCKS);
     const size_t b_start = (CDF_BUCKETS + 64) * sizeof(uint32_t), b_flags = CDF_TABLE_BLOCKS * sizeof(int);
+    const size_t bytes = b_start + b_flags + (size_t)n * sizeof(uint16_t);
+    if (!scratch_usable(SCRATCH_SPARSE_G, bytes, st)) return false;
     char *ws;
     try {
-        ws = (char *)scratch(SCRATCH_SPARSE_G, b_start + b_flags + (size_t)n * sizeof(uint16_t), st);
+        ws = (char *)scratch(SCRATCH_SPARSE_G, bytes, st);
     } catch (const Fail &f) {
         if (f.st != RBX_OUT_OF_MEMORY) throw;
         clear_error();

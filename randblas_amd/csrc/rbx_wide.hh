@@ -4,17 +4,26 @@
 // when it is materialised), Y the dense operand (either unit stride), any
 // sizes and any submatrix of the operator.
 //
-// One 512-thread workgroup per 64 x NT output tile and K range.  Every 32-deep
-// chunk of the tile's operator rows is generated once into LDS (each thread
-// one counter, four entries) while the chunk before it is multiplied: waves
-// 0-3 generate before their MFMAs, waves 4-7 after, so the two waves that
-// share a SIMD are in opposite phases.  The 8 waves form a WM x 8 / WM grid;
-// each owns RB x CB blocks of v_mfma_f{64,32}_16x16x4 (WM * RB = 4, NT = 128
-// CB / WM).  The dense operand goes straight from memory into the MFMA
+// One 512-thread workgroup per 64 x NT output tile, or per share of such a tile's
+// K (WideWork).  Every 32-deep chunk of the tile's operator rows is generated
+// once into LDS (each thread one counter, four entries) while the chunk before it
+// is multiplied: waves 0-3 generate before their MFMAs, waves 4-7 after, so the
+// two waves that share a SIMD are in opposite phases.  The 8 waves form a WM x 8
+// / WM grid; each owns RB x CB blocks of v_mfma_f{64,32}_16x16x4 (WM * RB = 4, NT
+// = 128 CB / WM).  The dense operand goes straight from memory into the MFMA
 // registers, one 16-deep step ahead of its use: lane (g = l / 16, c = l % 16)
 // holds k = 4 g .. 4 g + 3 of its columns, so with unit stride along K a
 // column's 16 k are one run of four lanes' vectors, and with unit stride along
 // N a lane holds CB neighbouring columns of four rows.
+//
+// What bounds it: the SIMDs' issue, shared by the MFMAs and the generator (FP64
+// 2048 x 131072 x 1000: 6.8 ms of MFMAs at the peak rate, 8.1 ms measured), and
+// how evenly the tiles fill the CUs.  Several columns of tiles need the same
+// operator rows: generated once ahead (WIDE_PRE) instead of once in each, FP64
+// 1032 x 34498 x 1189 takes 1572 us instead of 1716.  A last round of few tiles
+// is shared out instead of leaving CUs idle: FP32 50001 x 777 x 301 (782 tiles on
+// 256 CUs) 392 -> 335 us; with both, the FP32 right sketch 100000 x 2000 to 110
+// columns 568 -> 469 us.
 //
 // Sizes that do not fit: K (at least 4) is rounded up to whole chunks, the
 // dense values past it are zeros (the operator's are whatever the counters
@@ -41,7 +50,10 @@ struct WideMma<double> {
     static __device__ __forceinline__ acc_t mma(double a, double b, acc_t c) {
         return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
     }
-    static __device__ __forceinline__ int out_row(int lane, int r) { return (lane >> 4) + 4 * r; }
+    // The LDS row of a tile's row: the results r of lane l are the MFMA's rows
+    // l / 16 + 4 r, which with this order (4 x 4 within 16 rows, transposed) are
+    // the tile's rows 4 (l / 16) + r, as FP32's are.
+    static __device__ __forceinline__ int lds_row(int y) { return (y & ~15) | 4 * (y & 3) | ((y >> 2) & 3); }
 };
 template <>
 struct WideMma<float> {
@@ -50,7 +62,7 @@ struct WideMma<float> {
     static __device__ __forceinline__ acc_t mma(float a, float b, acc_t c) {
         return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
     }
-    static __device__ __forceinline__ int out_row(int lane, int r) { return 4 * (lane >> 4) + r; }
+    static __device__ __forceinline__ int lds_row(int y) { return y; }
 };
 
 // Tail columns: up to WIDE_TAIL output columns past the last whole tile (the
@@ -147,23 +159,36 @@ struct WideTail {
     }
 };
 
+// How the 64 x tile output tiles and their chunks (32 k each, `chunks` per tile)
+// go to workgroups: the first `whole` tiles to one each, each of the `rest` tiles
+// after them to `each`, all of which do the same share of the chunks; the i-th
+// of tile v writes its sums to the slot v * each + i.
+struct WideWork {
+    int whole, rest, each, nMB, chunks;
+    int q, r;  // chunks = q * each + r
+
+    __host__ __device__ int first(int i) const { return i * q + (i < r ? i : r); }
+};
+
 template <typename T>
 struct WideProblem {
     int64_t M, N, K;       // N without the tail columns
     GenMap g;              // b_off a multiple of 4
     const T *S;            // materialised operator: element (i, k) at S[i * srs + k * scs]
     int64_t srs, scs;
+    const float *pre;      // WIDE_PRE: the operator's chunks (wide_pre_kernel)
+    T scale;               // and its entries' scale
     int ko, mo;            // extra k / rows in front (see above); one of them is 0
     const T *D;
     int64_t drs, dcs;
     const T *xD;           // column N - 1 (unit stride) when not null
-    T *C, *xC;             // nS == 1: written by the kernel
+    T *C, *xC;
     int64_t crs, ccs, xcrs;
     T alpha, beta;
-    T *part;               // nS > 1: partials, nS x M x ldp
-    int64_t ldp, kw;       // kw: k per range, a multiple of 32
-    int nMB, nNB, nS;
-    TailCols<T> tc;        // tail columns, partials at tpart[(split * tc.nt + j) * 64 nMB + row]
+    WideWork wk;
+    T *part;               // partials, one 64 x tile block per slot, rows along C's unit stride
+    int part_cols;         // 1: columns are contiguous (element (i, j) at i * tile + j), 0: rows (i + 64 j)
+    TailCols<T> tc;        // tail columns, partials at tpart[(slot * tc.nt + j) * 64 + row]
     T *tpart;
 };
 
@@ -174,20 +199,25 @@ struct WideVec {
 
 // Waves per SIMD that the registers are bounded for: two workgroups per CU
 // where the accumulators leave room (the last round of a grid then ends sooner,
-// and one workgroup's barrier is the other's work).
+// and one workgroup's barrier is the other's work).  (FP32, unit stride along N:
+// 384 columns spill at 128 registers.)
 template <typename T>
-constexpr int wide_waves(int WM, int CB, int TW) {
-    const int acc = 4 / WM * CB * (int)sizeof(T);
+constexpr int wide_waves(bool NU, int WM, int CB, int TW) {
+    const int acc = 4 / WM * CB * (int)sizeof(T) + (NU && sizeof(T) == 4 ? 8 : 0);
+    if (acc <= 8 && TW == 0) return 8;  // 32 columns: four workgroups (FP64 at three: 2% slower)
     return acc + 4 * TW * (int)sizeof(T) / 4 <= 48 ? 4 : 2;
 }
 
-// The operator: uniform or Gaussian, generated, or read from memory.  ROWS: its
-// counters (or its unit stride) run along the output's rows, else along K.
-enum WideOp { WIDE_UNIFORM = 0, WIDE_GAUSS = 1, WIDE_MEM = 2 };
+// The operator: uniform or Gaussian, generated here, read from memory, or
+// generated ahead of this kernel chunk by chunk (WIDE_PRE, with ROWS = false
+// for either direction).  ROWS: its counters (or its unit stride) run along the
+// output's rows, else along K.
+enum WideOp { WIDE_UNIFORM = 0, WIDE_GAUSS = 1, WIDE_MEM = 2, WIDE_PRE = 3 };
 
 // NU: the dense operand's unit stride runs along N (else along K).
 template <typename T, int OP, bool ROWS, bool NU, int WM, int CB, int TW>
-__global__ __launch_bounds__(WD_THR, wide_waves<T>(WM, CB, TW)) void wide_kernel(const WideProblem<T> pb) {
+__global__ __launch_bounds__(WD_THR, OP == WIDE_MEM ? (wide_waves<T>(NU, WM, CB, TW) == 2 ? 2 : 4)
+                                                     : wide_waves<T>(NU, WM, CB, TW)) void wide_kernel(const WideProblem<T> pb) {
     using MM = WideMma<T>;
     constexpr int RB = 4 / WM, WN = 8 / WM, LDK = MM::LDK;
     constexpr int NT = 16 * CB * WN;
@@ -198,20 +228,28 @@ __global__ __launch_bounds__(WD_THR, wide_waves<T>(WM, CB, TW)) void wide_kernel
     const int wm = wave % WM, wn = wave / WM;
     const int lc = lane & 15, lg = lane >> 4;
 
-    // XCD-aware tile order: consecutive tiles (same K range and columns, so
-    // the same dense operand) on one XCD
-    const int W = pb.nMB * pb.nNB * pb.nS;
-    const int xcd = blockIdx.x % 8, xi = blockIdx.x / 8;
-    const int t = xcd * (W / 8) + (xcd < W % 8 ? xcd : W % 8) + xi;
-    const int mb = t % pb.nMB;
-    const int rest = t / pb.nMB;
-    const int nb = rest % pb.nNB;
-    const int sp = rest / pb.nNB;
+    // ---- this workgroup's chunks c0 .. c0 + nchunks - 1 of tile t.  XCD-aware
+    // order: consecutive tiles (same chunks and columns, so the same dense
+    // operand) on one XCD
+    const WideWork wk = pb.wk;
+    auto xcd_order = [](int b, int n) {
+        const int xcd = b % 8, xi = b / 8;
+        return xcd * (n / 8) + (xcd < n % 8 ? xcd : n % 8) + xi;
+    };
+    int t, c0 = 0, nchunks = wk.chunks, slot = -1;
+    if ((int)blockIdx.x < wk.whole) {
+        t = xcd_order(blockIdx.x, wk.whole);
+    } else {
+        const int o = xcd_order(blockIdx.x - wk.whole, wk.rest * wk.each), i = o / wk.rest, v = o - i * wk.rest;
+        t = wk.whole + v;
+        c0 = wk.first(i);
+        nchunks = wk.first(i + 1) - c0;
+        slot = v * wk.each + i;
+    }
+    const int nb = t / wk.nMB, mb = t - nb * wk.nMB;
     const int64_t m0 = (int64_t)mb * WD_MT, n0 = (int64_t)nb * NT;
+    const int64_t kbeg = (int64_t)c0 * WD_KC;
     const int64_t Kp = pb.K + pb.ko;
-    const int64_t kbeg = (int64_t)sp * pb.kw;
-    const int64_t kend = kbeg + pb.kw < Kp ? kbeg + pb.kw : Kp;
-    const int nchunks = (int)((kend - kbeg + WD_KC - 1) / WD_KC);
     const GenMap g = pb.g;
     constexpr bool GAUSS = OP == WIDE_GAUSS;
 
@@ -222,10 +260,10 @@ __global__ __launch_bounds__(WD_THR, wide_waves<T>(WM, CB, TW)) void wide_kernel
         for (int j = 0; j < CB; ++j) acc[i][j] = typename MM::acc_t{0, 0, 0, 0};
 
     // ---- operator chunk: rows along K (!ROWS): the thread owns cell tid % 8
-    // of row tid / 8; counters along the rows (ROWS): rows 4 (tid % 16) .. + 3
-    // of column tid / 16.  LDS row r, k at Ss[r * LDK + k].
-    const int frow = ROWS ? 4 * (tid & 15) : tid >> 3, fcell = ROWS ? tid >> 4 : tid & 7;
-    const uint64_t foff = ROWS ? (uint64_t)((g.a_off + kbeg + fcell) * g.P + ((g.b_off + m0) >> 2) + (tid & 15))
+    // of LDS row tid / 8; counters along the rows (ROWS): rows 4 (tid % 16) .. + 3
+    // of column tid / 16.  Row r, k at Ss[lds_row(r) * LDK + k].
+    const int frow = ROWS ? 4 * (tid & 15) : MM::lds_row(tid >> 3), fcell = ROWS ? tid >> 4 : tid & 7;
+    uint64_t foff = ROWS ? (uint64_t)((g.a_off + kbeg + fcell) * g.P + ((g.b_off + m0) >> 2) + (tid & 15))
                                : (uint64_t)((g.a_off + m0 + frow) * g.P + ((g.b_off + kbeg) >> 2) + fcell);
     const uint64_t fstep = ROWS ? WD_KC * (uint64_t)g.P : WD_KC / 4;  // counters per chunk
     WideTail<T, ROWS, TW == 0 ? 1 : TW> tl;
@@ -246,14 +284,25 @@ __global__ __launch_bounds__(WD_THR, wide_waves<T>(WM, CB, TW)) void wide_kernel
             mem[e] = ri == r && ki == k ? v : (T)0;
         }
     };
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    f4 pre4;
+    const float *prep = nullptr;
+    if constexpr (OP == WIDE_PRE) {
+        prep = pb.pre + ((int64_t)mb * wk.chunks + c0) * (WD_MT * WD_KC) + frow * WD_KC + 4 * fcell;
+        pre4 = *(const f4 *)prep;
+    }
     if constexpr (OP == WIDE_MEM) load_op(0);
     auto gen_chunk = [&](int c, T *lds) {
         T ent[4];
         if constexpr (OP == WIDE_MEM) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) ent[e] = mem[e];
+        } else if constexpr (OP == WIDE_PRE) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ent[e] = (T)pre4[e] * pb.scale;
         } else {
-            const float4 v = gen4(GAUSS, ctr_add(g.ctr, foff + fstep * (uint64_t)c), g.k0, g.k1);
+            const float4 v = gen4(GAUSS, ctr_add(g.ctr, foff), g.k0, g.k1);
+            foff += fstep;  // (the chunks are generated in order)
             ent[0] = entry_value<T>(v.x, GAUSS);
             ent[1] = entry_value<T>(v.y, GAUSS);
             ent[2] = entry_value<T>(v.z, GAUSS);
@@ -261,13 +310,17 @@ __global__ __launch_bounds__(WD_THR, wide_waves<T>(WM, CB, TW)) void wide_kernel
         }
         if constexpr (ROWS) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) lds[(frow + e) * LDK + fcell] = ent[e];
+            for (int e = 0; e < 4; ++e) lds[MM::lds_row(frow + e) * LDK + fcell] = ent[e];
         } else {
-            T *row = lds + frow * LDK + 4 * fcell;
+            T *row = lds + (tid >> 3) * LDK + 4 * fcell;  // row lds_row(frow)
 #pragma unroll
             for (int e = 0; e < 4; ++e) row[e] = ent[e];
         }
         if constexpr (OP == WIDE_MEM) load_op(c + 1);
+        if constexpr (OP == WIDE_PRE) {  // (one chunk past a tile's last is inside the buffer)
+            prep += WD_MT * WD_KC;
+            pre4 = *(const f4 *)prep;
+        }
         if constexpr (TW > 0) {
             tl.step(ent);
             tl.load(pb.tc, tk + WD_KC * (int64_t)(c + 1), pb.K);  // the next chunk's
@@ -396,7 +449,7 @@ __global__ __launch_bounds__(WD_THR, wide_waves<T>(WM, CB, TW)) void wide_kernel
         __builtin_amdgcn_s_setprio(0);
     };
 
-    const int64_t s_first = kbeg / 16, s_last = s_first + 2 * nchunks - 1;
+    const int64_t s_first = kbeg / 16;
     address(s_first);
     if constexpr (NU) {
 #pragma unroll
@@ -416,36 +469,60 @@ __global__ __launch_bounds__(WD_THR, wide_waves<T>(WM, CB, TW)) void wide_kernel
         const bool more = c + 1 < nchunks;
         if (more && !late) gen_chunk(c + 1, Sn);
         step(S, 0, s0, s0 + 1);
-        step(S, 1, s0 + 1, more ? s0 + 2 : s_last);
+        step(S, 1, s0 + 1, s0 + 2);
         if (more && late) gen_chunk(c + 1, Sn);
         __syncthreads();
     }
 
     if constexpr (TW > 0)
-        if (nb == 0)
-            tl.finish(pb.tc.nt, tid, frow, ROWS ? 0 : fcell, Ss,
-                      pb.tpart + (int64_t)sp * pb.tc.nt * (64 * (int64_t)pb.nMB) + m0, 64 * (int64_t)pb.nMB);
+        tl.finish(pb.tc.nt, tid, frow, ROWS ? 0 : fcell, Ss,
+                  pb.tpart + (int64_t)(slot < 0 ? t : wk.whole + slot) * pb.tc.nt * WD_MT, WD_MT);
 
+    // ---- results: acc[i][j][r] is row 4 lg + r of the i-th 16 rows, column j
+    typedef typename WideVec<T, 4>::type vec4;
+    if (slot >= 0) {
+        T *out = pb.part + (int64_t)slot * (WD_MT * NT);
 #pragma unroll
-    for (int i = 0; i < RB; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int64_t gi = m0 + 16 * (RB * wm + i) + MM::out_row(lane, r) - pb.mo;
-            if (gi < 0 || gi >= pb.M) continue;
+        for (int i = 0; i < RB; ++i) {
+            const int row = 16 * (RB * wm + i) + 4 * lg;
+            if (m0 + row - pb.mo >= pb.M) continue;
 #pragma unroll
             for (int j = 0; j < CB; ++j) {
                 // NU: a lane moved back owns only the columns past its neighbour's
                 const int64_t gj = NU ? cs + j : wcol + 16 * j + lc;
                 if (NU ? gj < wcol + CB * lc : gj >= pb.N) continue;
-                const T v = acc[i][j][r];
-                if (pb.part != nullptr) {
-                    pb.part[((int64_t)sp * pb.M + gi) * pb.ldp + gj] = v;
+                const int col = (int)(gj - n0);
+                if (pb.part_cols) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) out[(row + r) * NT + col] = acc[i][j][r];
                 } else {
-                    T *c = (pb.xC != nullptr && gj == pb.N - 1) ? pb.xC + gi * pb.xcrs : pb.C + gi * pb.crs + gj * pb.ccs;
-                    T o = pb.alpha * v;
-                    if (pb.beta != (T)0) o = o + pb.beta * (*c);
-                    *c = o;
+                    *(vec4 *)(out + row + col * WD_MT) = vec4{acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
                 }
+            }
+        }
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            const int64_t gi = m0 + 16 * (RB * wm + i) + 4 * lg - pb.mo;
+            const int64_t gj = NU ? cs + j : wcol + 16 * j + lc;
+            if (NU ? gj < wcol + CB * lc : gj >= pb.N) continue;  // (as above)
+            const bool apart = pb.xC != nullptr && gj == pb.N - 1;
+            const int64_t rs = apart ? pb.xcrs : pb.crs;
+            T *c = (apart ? pb.xC : pb.C + gj * pb.ccs) + gi * rs;
+            if (rs == 1 && pb.beta == (T)0 && gi >= 0 && gi + 4 <= pb.M) {
+                *(vec4 *)c = vec4{pb.alpha * acc[i][j][0], pb.alpha * acc[i][j][1], pb.alpha * acc[i][j][2],
+                                  pb.alpha * acc[i][j][3]};
+                continue;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (gi + r < 0 || gi + r >= pb.M) continue;
+                T out = pb.alpha * acc[i][j][r];
+                if (pb.beta != (T)0) out = out + pb.beta * c[r * rs];
+                c[r * rs] = out;
             }
         }
 }
@@ -456,8 +533,7 @@ void wide_launch(bool nu, int tile, int tw, const WideProblem<T> &pb, hipStream_
 
 template <typename T, int OP, bool ROWS, bool NU, int WM, int CB, int TW>
 static void wide_launch_one(const WideProblem<T> &pb, hipStream_t st) {
-    hipLaunchKernelGGL((wide_kernel<T, OP, ROWS, NU, WM, CB, TW>), dim3((unsigned)(pb.nMB * pb.nNB * pb.nS)),
-                       dim3(WD_THR), 0, st, pb);
+    hipLaunchKernelGGL((wide_kernel<T, OP, ROWS, NU, WM, CB, TW>), dim3((unsigned)(pb.wk.whole + pb.wk.rest * pb.wk.each)), dim3(WD_THR), 0, st, pb);
 }
 template <typename T, int OP, bool ROWS, bool NU>
 static void wide_launch_tile(int tile, int tw, const WideProblem<T> &pb, hipStream_t st) {

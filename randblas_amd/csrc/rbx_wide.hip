@@ -1,5 +1,6 @@
-// rbx_wide.hip -- plans and launches the fused dense sketches (rbx_wide.hh): the tile width and the K ranges, the reduction of
-// the ranges' partials.
+// rbx_wide.hip -- plans and launches the fused dense sketches (rbx_wide.hh): the
+// tile width, how tiles and chunks are shared out, the operator generated ahead,
+// the reduction of the shared tiles.
 #include <algorithm>
 #include <type_traits>
 
@@ -7,91 +8,112 @@
 
 namespace rbx {
 
-// C[i, j] = alpha * sum_s part[s][i * ldp + j] + beta * C[i, j], FP64 sums in a
-// fixed order; column N - 1 of C apart at xC when given.  A workgroup takes a
-// TR x 4 TQ tile; G threads per four columns sum the splits s = g, g + G, ...,
-// then the G sums are added in order (G > 1 when the output alone has too few
-// entries to keep the loads of many splits in flight).  Tiles with one thread
-// per quad are 8 x 128, 512-byte (FP32) runs of every partial.
-template <typename T, int G>
-__global__ __launch_bounds__(256) void wide_reduce_kernel(const T *part, int nS, int64_t M, int64_t N, int64_t ldp,
-                                                          double alpha, double beta, T *C, int64_t crs, int64_t ccs,
-                                                          T *xC, int64_t xcrs) {
-    constexpr int TR = G == 1 ? 8 : 4, TQ = 256 / G / TR, TC = 4 * TQ;
-    __shared__ double sums[G][TR][TC + 1];
+// The tiles that several workgroups share: C = alpha * (sum of a tile's pieces)
+// + beta * C, FP64 sums in a fixed order; column N - 1 of C apart at xC when
+// given.  A wave takes 256 consecutive entries of the tile's blocks; NW waves
+// share them, wave w summing pieces w, w + NW, ... (NW > 1 when the output alone
+// has too few entries to keep the loads of many pieces in flight), and the NW
+// sums are added in order.  nsub: sub-blocks of a tile.
+template <typename T, int NW>
+__global__ __launch_bounds__(NW < 4 ? 256 : 64 * NW) void wide_reduce_kernel(const WideProblem<T> pb, int tile, int nsub,
+                                                                             double alpha, double beta) {
+    constexpr int WV = NW < 4 ? 4 : NW;
+    __shared__ double sums[NW > 1 ? NW : 1][NW > 1 ? 256 : 1];
     typedef T t4 __attribute__((ext_vector_type(4)));
-    const int64_t ntc = (N + TC - 1) / TC;
-    const int64_t i0 = (int64_t)(blockIdx.x / ntc) * TR, j0 = (int64_t)(blockIdx.x % ntc) * TC;
-    const int tid = threadIdx.x;
-    {
-        const int c4 = 4 * (tid % TQ), r = (tid / TQ) % TR, gq = tid / (TQ * TR);
-        const int64_t i = i0 + r, j = j0 + c4, total = M * ldp;
-        double v[4] = {0.0, 0.0, 0.0, 0.0};
-        if (i < M && j < ldp) {
-            const T *p = part + i * ldp + j;
-            int s = gq;
-            for (; s + 7 * G < nS; s += 8 * G) {
-                t4 x[8];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int v = (int)(blockIdx.x / (unsigned)nsub);
+    const int sub = (int)(blockIdx.x - (unsigned)v * nsub) * (WV / NW) + (NW > 1 ? 0 : wave);
+    const int n = pb.wk.each;
+    // the lane's four entries: rows row .. row + 3 of one column, or (part_cols) columns of one row
+    const int e0 = 256 * sub + 4 * lane;
+    const int row = pb.part_cols ? e0 / tile : e0 % WD_MT, col = pb.part_cols ? e0 - row * tile : e0 / WD_MT;
+    const int t = pb.wk.whole + v, nb = t / pb.wk.nMB;
+    const int64_t i = (int64_t)(t - nb * pb.wk.nMB) * WD_MT - pb.mo + row, j = (int64_t)nb * tile + col;
+    const bool in = e0 < WD_MT * tile && i < pb.M && j < pb.N;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+    if (in) {
+        const int64_t block = WD_MT * (int64_t)tile;
+        const T *p = pb.part + (int64_t)v * n * block + e0;
+        for (int u = NW > 1 ? wave : 0; u < n; u += 8 * NW) {
+            t4 x[8];
 #pragma unroll
-                for (int u = 0; u < 8; ++u) x[u] = *(const t4 *)(p + (int64_t)(s + u * G) * total);
+            for (int q = 0; q < 8; ++q) x[q] = u + q * NW < n ? *(const t4 *)(p + (u + q * NW) * block) : t4{0, 0, 0, 0};
 #pragma unroll
-                for (int u = 0; u < 8; ++u)
+            for (int q = 0; q < 8; ++q)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] += (double)x[u][e];
-            }
-            for (; s < nS; s += G) {
-                const t4 x = *(const t4 *)(p + (int64_t)s * total);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] += (double)x[e];
-            }
+                for (int e = 0; e < 4; ++e) s[e] += (double)x[q][e];
         }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) sums[gq][r][c4 + e] = v[e];
     }
-    __syncthreads();
-    const bool cm = crs == 1;  // consecutive threads along C's unit stride
-    for (int e = tid; e < TR * TC; e += 256) {
-        const int ti = cm ? e % TR : e / TC, tj = cm ? e / TR : e % TC;
-        const int64_t i = i0 + ti, j = j0 + tj;
-        if (i < M && j < N) {
-            double v = sums[0][ti][tj];
+    if constexpr (NW > 1) {
 #pragma unroll
-            for (int q = 1; q < G; ++q) v += sums[q][ti][tj];
-            T *c = (xC != nullptr && j == N - 1) ? xC + i * xcrs : C + i * crs + j * ccs;
-            double out = alpha * v;
-            if (beta != 0.0) out += beta * (double)(*c);
-            *c = (T)out;
+        for (int e = 0; e < 4; ++e) sums[wave][4 * lane + e] = s[e];
+        __syncthreads();
+        if (wave != 0) return;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            s[e] = sums[0][4 * lane + e];
+#pragma unroll
+            for (int q = 1; q < NW; ++q) s[e] += sums[q][4 * lane + e];
         }
+    }
+    if (!in) return;
+    const bool apart = pb.xC != nullptr && j == pb.N - 1;
+    T *c = apart ? pb.xC + i * pb.xcrs : pb.C + i * pb.crs + j * pb.ccs;
+    const int64_t cs = pb.part_cols ? pb.ccs : (apart ? pb.xcrs : pb.crs);
+    // the entries that exist: e >= lo (rows in front of the first), e < hi
+    const int lo = i < 0 ? (int)-i : 0;
+    const int64_t left = pb.part_cols ? pb.N - j : pb.M - i;
+    const int hi = left < 4 ? (int)left : 4;
+    if (cs == 1 && beta == 0.0 && i >= 0 && hi == 4) {
+        typedef T u4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+        *(u4 *)c = u4{(T)(alpha * s[0]), (T)(alpha * s[1]), (T)(alpha * s[2]), (T)(alpha * s[3])};
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if ((pb.part_cols ? i < 0 : e < lo) || e >= hi) continue;
+        double out = alpha * s[e];
+        if (beta != 0.0) out += beta * (double)c[e * cs];
+        c[e * cs] = (T)out;
     }
 }
 
-// The tail's outputs: out[j][i * ors[j]] = alpha * (sum over splits of
-// tpart[(s * nt + j) * Mt + mo + i]) + beta * out, FP64 sums.  G threads per
-// output entry: G = 1 sums the splits in order; G = 64 (many splits) has lane
-// l sum splits l, l + 64, ..., then a butterfly (a fixed order).
-template <typename T, int G>
-__global__ __launch_bounds__(256) void wide_tail_reduce_kernel(const T *tpart, int nS, int64_t M, int64_t Mt, int mo,
-                                                               TailCols<T> tc, double alpha, double beta) {
-    const int nt = tc.nt;
-    const int g = threadIdx.x % G;
-    const int64_t e = (int64_t)blockIdx.x * (256 / G) + threadIdx.x / G;
-    if (e >= M * nt) return;  // uniform per group
-    const int64_t i = e % M;
-    const int j = (int)(e / M);
-    double v = 0.0;
-    for (int s = g; s < nS; s += G) v += (double)tpart[((int64_t)s * nt + j) * Mt + mo + i];
-    if constexpr (G == 64) {
+// The tail's outputs of one row tile per workgroup: out[j][i * ors[j]] = alpha *
+// (sum of the tile's pieces) + beta * out, FP64 sums in a fixed order.  Wave w
+// sums pieces w, w + 16, ..., a row per lane.
+template <typename T>
+__global__ __launch_bounds__(1024) void wide_tail_reduce_kernel(const WideProblem<T> pb, double alpha, double beta) {
+    __shared__ double sums[16][WIDE_TAIL][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int nt = pb.tc.nt;
+    double s[WIDE_TAIL] = {0.0, 0.0, 0.0, 0.0};
+    auto add = [&](int slot) {
+        const T *p = pb.tpart + (int64_t)slot * nt * WD_MT + lane;
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
-        if (g != 0) return;
+        for (int j = 0; j < WIDE_TAIL; ++j)
+            if (j < nt) s[j] += (double)p[j * WD_MT];
+    };
+    const int shared = (int)blockIdx.x - pb.wk.whole;  // which of the shared tiles
+    if (shared >= 0) {
+        for (int u = wave; u < pb.wk.each; u += 16) add(pb.wk.whole + shared * pb.wk.each + u);
+    } else if (wave == 0) {
+        add(blockIdx.x);
     }
+#pragma unroll
+    for (int j = 0; j < WIDE_TAIL; ++j) sums[wave][j][lane] = s[j];
+    __syncthreads();
+    const int64_t i = (int64_t)blockIdx.x * WD_MT + lane - pb.mo;
+    if (wave >= nt || i < 0 || i >= pb.M) return;
+    double v = sums[0][wave][lane];
+#pragma unroll
+    for (int q = 1; q < 16; ++q) v += sums[q][wave][lane];
     T *c = nullptr;
     int64_t rs = 0;
 #pragma unroll
-    for (int q = 0; q < WIDE_TAIL; ++q)
-        if (q == j) {
-            c = tc.out[q];
-            rs = tc.ors[q];
+    for (int j = 0; j < WIDE_TAIL; ++j)
+        if (j == wave) {
+            c = pb.tc.out[j];
+            rs = pb.tc.ors[j];
         }
     c += i * rs;
     double out = alpha * v;
@@ -109,10 +131,35 @@ __global__ __launch_bounds__(256) void pad_k4_kernel(const T *D, int64_t drs, in
     }
 }
 
-// Scratch, or nullptr when the device cannot provide it.
-static void *try_scratch(size_t bytes, hipStream_t stream) {
+// The operator's chunks of 64 rows x 32 k ahead of the products that read them:
+// chunk c of row tile mb at out[(mb * nch + c) * 2048], row r's k .. k + 3 at
+// 32 r + k.  Entries before their scale (exact in FP32).  One workgroup per
+// chunk, one counter per thread; counters along the rows turn in LDS.
+template <bool GAUSS, bool ROWS>
+__global__ __launch_bounds__(WD_THR) void wide_pre_kernel(GenMap g, int64_t nch, float *out) {
+    __shared__ float t[WD_MT][WD_KC + 1];
+    const int tid = threadIdx.x;
+    const int64_t mb = blockIdx.x / nch, c = blockIdx.x - mb * nch, m0 = mb * WD_MT, k0 = c * WD_KC;
+    const int frow = ROWS ? 4 * (tid & 15) : tid >> 3, fcell = ROWS ? tid >> 4 : tid & 7;
+    const uint64_t off = ROWS ? (uint64_t)((g.a_off + k0 + fcell) * g.P + ((g.b_off + m0) >> 2) + (tid & 15))
+                              : (uint64_t)((g.a_off + m0 + frow) * g.P + ((g.b_off + k0) >> 2) + fcell);
+    float4 v = gen4(GAUSS, ctr_add(g.ctr, off), g.k0, g.k1);
+    if constexpr (ROWS) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[frow + e][fcell] = f4_get(v, e);
+        __syncthreads();
+        const float *q = &t[tid >> 3][4 * (tid & 7)];
+        v = make_float4(q[0], q[1], q[2], q[3]);
+    }
+    ((float4 *)out)[(int64_t)blockIdx.x * WD_THR + tid] = v;
+}
+
+// Scratch, or nullptr when the device cannot provide it, or only by growing it
+// while the stream is captured.
+static void *try_scratch(int slot, size_t bytes, hipStream_t stream) {
+    if (!scratch_usable(slot, bytes, stream)) return nullptr;
     try {
-        return scratch(SCRATCH_SPLITK, bytes, stream);
+        return scratch(slot, bytes, stream);
     } catch (const Fail &f) {
         if (f.st != RBX_OUT_OF_MEMORY) throw;
         clear_error();
@@ -120,35 +167,40 @@ static void *try_scratch(size_t bytes, hipStream_t stream) {
     }
 }
 
-// Tile width, tail columns and K ranges of one product.  The time of a
-// workgroup's 32-deep chunk is its MFMAs (64 x tile x 32 at the matrix rate,
-// also for columns that do not exist) plus the operator's generation (2048
-// entries, the same for every tile width); rounds of one workgroup per CU.
-// More K ranges fill the chip, but their partials are written and read.
+// Tile width, tail columns, how the tiles and their chunks are shared out, and
+// whether the operator is generated ahead.  The time of a workgroup's 32-deep
+// chunk is its MFMAs (64 x tile x 32 at the matrix rate, also for columns that do
+// not exist) plus the operator's generation (2048 entries, the same for every
+// tile width) or the read of one generated ahead, which pays when several
+// columns of tiles would generate the same entries.
 struct WidePlan {
-    int tile, tw, nS;
-    int64_t kw;
+    int tile, tw;
+    bool pre;
+    WideWork wk;
+    double t;
 };
-constexpr size_t WIDE_PART_MAX = 16ull << 30;  // partials above this: fewer ranges
+constexpr size_t WIDE_PART_MAX = 16ull << 30;  // bytes of partials: above, tiles are not shared
+constexpr size_t WIDE_PRE_MAX = 2ull << 30;    // bytes of an operator generated ahead
 
 template <typename T>
-static WidePlan wide_plan(const GemmProblem &pb, int ko, int mo, bool NU, bool split_ok) {
+static WidePlan wide_plan(const GemmProblem &pb, int ko, int mo, bool NU, bool split_ok, bool pre_ok) {
     constexpr bool F64 = sizeof(T) == 8;
     // clocks of a CU: 2048 Gaussian entries (measured: 1.2 a clock), chunk overhead,
-    // a workgroup's start and end
-    const double gen = pb.g.gauss ? 1700.0 : 800.0, over = 300.0, fixed = 5000.0, mhz = 2100.0;
+    // a piece's start and end
+    const double gen_here = pb.g.gauss ? 1700.0 : 800.0, gen_pre = 150.0, over = F64 ? 500.0 : 900.0, fixed = 5000.0, mhz = 2100.0;
     const double flop_clk = F64 ? 128.0 : 256.0;
-    // FP32 sums are kept in ranges of at most 4096 terms, FP64 needs no bound
-    const int64_t kw_max = F64 ? 16384 : 4096;
-    const int64_t Kp = pb.K + ko, chunks = (Kp + WD_KC - 1) / WD_KC;
+    // FP32 sums have at most 4096 terms, FP64 ones 16384
+    const int64_t range_max = (F64 ? 16384 : 4096) / WD_KC;
+    const int64_t chunks = (pb.K + ko + WD_KC - 1) / WD_KC;
     const int64_t nMB = (pb.M + mo + WD_MT - 1) / WD_MT;
-    const int cus = num_cus();
+    RBX_REQUIRE(chunks < (1ll << 31));
+    const int64_t cus = num_cus();
     // columns, waves along the rows, blocks per wave (wide_launch_tile)
     static const struct { int cols, wm, cb; } tiles[] = {
         {32, 4, 1},  {64, 2, 1},  {128, 1, 1}, {192, 2, 3}, {256, 1, 2}, {320, 2, 5},
         {384, 1, 3}, {448, 2, 7}, {512, 1, 4}, {640, 1, 5}, {768, 1, 6}, {1024, 1, 8}};
     WidePlan best{};
-    double best_t = 1e300;
+    best.t = 1e300;
     for (const auto &tl : tiles) {
         const int tile = tl.cols;
         if (F64 && tile > 512) break;
@@ -158,7 +210,7 @@ static WidePlan wide_plan(const GemmProblem &pb, int ko, int mo, bool NU, bool s
         // two waves read the same columns: only where one tile is the whole
         // output (100000 columns, K = 2000, FP32: 448 wide 630 us, 512 wide 590)
         if (tl.wm == 2 && tile > 64 && pb.N > tile) continue;
-        const bool two = wide_waves<T>(tl.wm, tl.cb, 0) == 4;  // two workgroups per CU
+        const bool two = wide_waves<T>(NU, tl.wm, tl.cb, 0) >= 4;  // two workgroups per CU
         for (int tail = 0; tail < 2; ++tail) {
             int tw = 0;
             if (tail) {
@@ -166,33 +218,62 @@ static WidePlan wide_plan(const GemmProblem &pb, int ko, int mo, bool NU, bool s
                 if (NU || !split_ok || (tile != 128 && tile != 256) || tw < 1 || tw > WIDE_TAIL) continue;
             }
             const int64_t nNB = tail ? 1 : (pb.N + tile - 1) / tile;
-            const int64_t wgs = nMB * nNB;
-            const double chunk_clk = 64.0 * tile * 64.0 / flop_clk + gen + over + (tw > 1 ? 400.0 : 100.0 * tw);
-            const int64_t ns_min = split_ok ? (Kp + kw_max - 1) / kw_max : 1;
-            for (int r = 0; r <= 8; ++r) {
-                int64_t ns = r == 0 ? ns_min : std::max<int64_t>(ns_min, r * (int64_t)cus / wgs);
-                if (!split_ok) ns = 1;
-                if (ns < 1) ns = 1;
-                const int64_t cps = (chunks + ns - 1) / ns;  // chunks per range
-                ns = (chunks + cps - 1) / cps;
-                const double part = (double)ns * (double)pb.M * (double)pb.N * sizeof(T);
-                if (ns > 1 && part > (double)WIDE_PART_MAX) continue;
-                // with two workgroups on a CU the last round overlaps the one before
-                double rounds = (double)((wgs * ns + cus - 1) / cus);
-                if (two && rounds > 1) rounds = std::min(rounds, (double)(wgs * ns) / cus + 0.5);
-                double t = rounds * (cps * chunk_clk + fixed) / mhz;
-                if (ns > 1) t += 5.0 + 2.0 * part / 3.5e6;
-                if (tail) t += 3.0;
-                if (t < best_t) {
-                    best_t = t;
-                    best = WidePlan{tile, tw, (int)ns, cps * WD_KC};
+            const int64_t tot = nMB * nNB;
+            if (tot >= (1ll << 31)) continue;
+            for (int pre = 0; pre <= (pre_ok && nNB > 1 ? 1 : 0); ++pre) {
+                const double gen = pre ? gen_pre : gen_here;
+                const double t_pre = pre ? 6.0 + (double)(nMB * chunks) * 2048.0 / (pb.g.gauss ? 6.5e5 : 1.1e6) : 0.0;
+                const double chunk_clk = 64.0 * tile * 64.0 / flop_clk + gen + over + (tw > 1 ? 400.0 : 100.0 * tw);
+                // `whole` tiles to one workgroup each, the others to `each`
+                auto consider = [&](int64_t whole, int64_t each) {
+                    WidePlan p{};
+                    WideWork &k = p.wk;
+                    const int64_t rest = tot - whole, pieces = rest * each;
+                    if (whole + pieces >= (1ll << 31)) return;
+                    k.whole = (int)whole;
+                    k.rest = (int)rest;
+                    k.each = (int)each;
+                    k.nMB = (int)nMB;
+                    k.chunks = (int)chunks;
+                    if (rest > 0) {
+                        k.q = (int)(chunks / each);
+                        k.r = (int)(chunks % each);
+                    }
+                    // with two workgroups on a CU the last round overlaps the one before
+                    auto rounds = [&](int64_t wgs) {
+                        const double up = (double)((wgs + cus - 1) / cus);
+                        return two && up > 1 ? std::min(up, (double)wgs / cus + 0.5) : up;
+                    };
+                    p.t = (whole > 0 ? rounds(whole) * (chunks * chunk_clk + fixed) : 0.0) / mhz + t_pre;
+                    if (rest > 0) {
+                        const double part = (double)pieces * WD_MT * tile * sizeof(T);
+                        if (part > (double)WIDE_PART_MAX) return;
+                        p.t += rounds(pieces) * ((double)((chunks + each - 1) / each) * chunk_clk + fixed) / mhz;
+                        p.t += 4.0 + part / 3e6;
+                    }
+                    if (tail) p.t += 3.0;
+                    if (p.t >= best.t) return;
+                    p.tile = tile;
+                    p.tw = tw;
+                    p.pre = pre != 0;
+                    best = p;
+                };
+                if (!split_ok || chunks <= range_max) consider(tot, 0);
+                if (!split_ok) continue;
+                for (int r = 0; r <= 8; ++r) {  // every tile shared
+                    int64_t each = std::max((chunks + range_max - 1) / range_max, r * cus / tot);
+                    each = std::min(each, chunks);
+                    if (each > 1) consider(0, each);
                 }
+                // whole tiles for as long as every CU has one, the others shared
+                const int64_t left = tot % cus;
+                if (chunks <= range_max && tot > cus && left > 0)
+                    for (int r = 1; r <= 2; ++r) {
+                        const int64_t each = std::min(r * cus / left, chunks);
+                        if (each > 1) consider(tot - left, each);
+                    }
             }
         }
-    }
-    if (best.tile == 0) {  // partials too large for any number of ranges
-        const int tile = pb.N < 512 ? 128 : 512;
-        best = WidePlan{tile, 0, 1, chunks * WD_KC};
     }
     return best;
 }
@@ -242,23 +323,32 @@ void wide_run(const GemmProblem &pb, hipStream_t stream) {
     RBX_REQUIRE(!NU || pb.xD == nullptr);
     GemmProblem sized = pb;
     sized.K = w.K;
-    WidePlan p = wide_plan<T>(sized, w.ko, w.mo, NU, true);
-    w.nMB = (int)((pb.M + w.mo + WD_MT - 1) / WD_MT);
-    const int64_t Mt = 64 * (int64_t)w.nMB;
+    const int64_t nMB = (pb.M + w.mo + WD_MT - 1) / WD_MT;
+    const int64_t npre = (w.K + w.ko + WD_KC - 1) / WD_KC;
+    const size_t pre_bytes = ((size_t)safe_mul(nMB, npre) + 1) * (WD_MT * WD_KC * sizeof(float));
+    // (a materialised operator is read in the same shares as a generated one, so
+    // the two give the same bits)
+    bool pre_ok = pb.K >= 4 && pre_bytes <= WIDE_PRE_MAX;
+    WidePlan p = wide_plan<T>(sized, w.ko, w.mo, NU, true, pre_ok);
+    float *pre = nullptr;
+    if (p.pre && w.S == nullptr) {
+        pre = (float *)try_scratch(SCRATCH_BF16, pre_bytes, stream);
+        if (pre == nullptr) p = wide_plan<T>(sized, w.ko, w.mo, NU, true, pre_ok = false);
+    }
     char *ws = nullptr;
     size_t part_bytes = 0;
-    if (p.nS > 1 || p.tw > 0) {
-        w.ldp = (pb.N - p.tw + 3) / 4 * 4;
-        if (p.nS > 1) part_bytes = ((size_t)p.nS * pb.M * w.ldp * sizeof(T) + 255) / 256 * 256;
-        ws = (char *)try_scratch(part_bytes + (size_t)p.nS * p.tw * Mt * sizeof(T), stream);
-        if (ws == nullptr) p = wide_plan<T>(sized, w.ko, w.mo, NU, false);
+    if (p.wk.rest > 0 || p.tw > 0) {
+        const size_t slots = (size_t)p.wk.rest * p.wk.each;
+        part_bytes = (slots * WD_MT * p.tile * sizeof(T) + 255) / 256 * 256;
+        const size_t tails = slots + (size_t)p.wk.whole;
+        ws = (char *)try_scratch(SCRATCH_SPLITK, part_bytes + tails * p.tw * WD_MT * sizeof(T), stream);
+        if (ws == nullptr) p = wide_plan<T>(sized, w.ko, w.mo, NU, false, pre_ok && (pre != nullptr || w.S != nullptr));
     }
-    w.nS = p.nS;
-    w.kw = p.kw;
+    RBX_REQUIRE(p.tile > 0);
+    w.wk = p.wk;
     w.N = pb.N - p.tw;
-    w.nNB = (int)((w.N + p.tile - 1) / p.tile);
-    RBX_REQUIRE((int64_t)w.nMB * w.nNB < (1ll << 31) / w.nS);
-    if (p.nS > 1) w.part = (T *)ws;
+    w.part = (T *)ws;
+    w.part_cols = w.crs != 1;
     if (p.tw > 0) {
         w.tpart = (T *)(ws + part_bytes);
         w.tc.nt = p.tw;
@@ -276,40 +366,47 @@ void wide_run(const GemmProblem &pb, hipStream_t stream) {
         for (int j = 0; j < WIDE_TAIL; ++j) w.tc.col[j] = w.D;
     }
     const bool gauss = pb.g.gauss != 0;
+    if (p.pre && w.S == nullptr) {
+        ProfScope prof("wide_pre_kernel", stream);
+        const dim3 grid((unsigned)(nMB * npre));  // (below 2^31: WIDE_PRE_MAX)
+        if (gauss && rows) hipLaunchKernelGGL((wide_pre_kernel<true, true>), grid, dim3(WD_THR), 0, stream, w.g, npre, pre);
+        else if (gauss) hipLaunchKernelGGL((wide_pre_kernel<true, false>), grid, dim3(WD_THR), 0, stream, w.g, npre, pre);
+        else if (rows) hipLaunchKernelGGL((wide_pre_kernel<false, true>), grid, dim3(WD_THR), 0, stream, w.g, npre, pre);
+        else hipLaunchKernelGGL((wide_pre_kernel<false, false>), grid, dim3(WD_THR), 0, stream, w.g, npre, pre);
+        RBX_HIP(hipGetLastError());
+        w.pre = pre;
+        w.scale = entry_scale<T>(gauss);
+    }
     {
         ProfScope prof(sizeof(T) == 8 ? "f64_wide_kernel" : "f32_wide_kernel", stream);
         if (w.S != nullptr && w.srs == 1) wide_launch<T, WIDE_MEM, true>(NU, p.tile, p.tw, w, stream);
         else if (w.S != nullptr) wide_launch<T, WIDE_MEM, false>(NU, p.tile, p.tw, w, stream);
+        else if (p.pre) wide_launch<T, WIDE_PRE, false>(NU, p.tile, p.tw, w, stream);
         else if (gauss && rows) wide_launch<T, WIDE_GAUSS, true>(NU, p.tile, p.tw, w, stream);
         else if (gauss) wide_launch<T, WIDE_GAUSS, false>(NU, p.tile, p.tw, w, stream);
         else if (rows) wide_launch<T, WIDE_UNIFORM, true>(NU, p.tile, p.tw, w, stream);
         else wide_launch<T, WIDE_UNIFORM, false>(NU, p.tile, p.tw, w, stream);
         RBX_HIP(hipGetLastError());
     }
-    if (w.nS > 1) {
+    if (p.wk.rest > 0) {
         ProfScope prof(sizeof(T) == 8 ? "f64_reduce_kernel" : "f32_reduce_kernel", stream);
-        auto go = [&](auto gv) {
-            constexpr int G = decltype(gv)::value, TR = G == 1 ? 8 : 4, TC = 4 * (256 / G / TR);
-            const int64_t nt = ((w.M + TR - 1) / TR) * ((w.N + TC - 1) / TC);
-            RBX_REQUIRE(nt < (1ll << 31));
-            hipLaunchKernelGGL((wide_reduce_kernel<T, G>), dim3((unsigned)nt), dim3(256), 0, stream, (const T *)w.part,
-                               w.nS, w.M, w.N, w.ldp, pb.alpha, pb.beta, w.C, w.crs, w.ccs, w.xC, w.xcrs);
+        auto go = [&](auto nw) {
+            constexpr int NW = decltype(nw)::value, per = NW < 4 ? 4 : 1;  // sub-blocks of 256 per workgroup
+            const int64_t nsub = (WD_MT * p.tile / 256 + per - 1) / per;
+            RBX_REQUIRE(p.wk.rest < (1ll << 31) / nsub);
+            hipLaunchKernelGGL((wide_reduce_kernel<T, NW>), dim3((unsigned)(p.wk.rest * nsub)),
+                               dim3(NW < 4 ? 256 : 64 * NW), 0, stream, w, p.tile, (int)nsub, pb.alpha, pb.beta);
         };
-        // enough threads for about 16 waves per CU, at most one per 4 splits
-        const int64_t quads = w.M * w.ldp / 4, want = 256 * 1024;
-        if (quads >= want || w.nS < 8) go(std::integral_constant<int, 1>{});
-        else if (quads * 4 >= want || w.nS < 32) go(std::integral_constant<int, 4>{});
+        // enough threads for about 16 waves per CU, at most one per 4 pieces
+        const int64_t quads = (int64_t)p.wk.rest * WD_MT * p.tile / 4, want = 256 * 1024;
+        const int pieces = p.wk.each;
+        if (quads >= want || pieces < 8) go(std::integral_constant<int, 1>{});
+        else if (quads * 4 >= want || pieces < 32) go(std::integral_constant<int, 4>{});
         else go(std::integral_constant<int, 16>{});
         RBX_HIP(hipGetLastError());
     }
     if (p.tw > 0) {
-        const int64_t n = w.M * p.tw;
-        if (w.nS <= 16)
-            hipLaunchKernelGGL((wide_tail_reduce_kernel<T, 1>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream,
-                               (const T *)w.tpart, w.nS, w.M, Mt, w.mo, w.tc, pb.alpha, pb.beta);
-        else
-            hipLaunchKernelGGL((wide_tail_reduce_kernel<T, 64>), dim3((unsigned)((n + 3) / 4)), dim3(256), 0, stream,
-                               (const T *)w.tpart, w.nS, w.M, Mt, w.mo, w.tc, pb.alpha, pb.beta);
+        hipLaunchKernelGGL(wide_tail_reduce_kernel<T>, dim3((unsigned)nMB), dim3(1024), 0, stream, w, pb.alpha, pb.beta);
         RBX_HIP(hipGetLastError());
     }
 }

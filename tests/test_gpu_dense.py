@@ -621,3 +621,78 @@ def test_materialised_operator_same_bits(rb, orc, opS, n, m, co):
     b, _ = run_lskge3(rb, orc, np.float64, "C", opS, "N", 90, n, m, 1.0, 0.0, ro=2, co=co)
     assert np.array_equal(a, b)
     assert rel_fro(a, ref) <= 1e-13
+
+
+# ---------------------------------------------------------------- shared tiles, operator generated ahead
+def _against_fill(rb, dtype, layout, opS, d, n, m, alpha, beta, ro, co, fam, axis):
+    """lskge3 with a generated operator and the same product in float64 from fill_dense's entries
+    (bit-exact against the oracle above); the profile of the call."""
+    tdt = torch.float64 if dtype == np.float64 else torch.float32
+    win = (d, m) if opS == "N" else (m, d)
+    D = rb.DenseDist(win[0] + ro + 2, win[1] + co + 1, rb.ScalarDist(fam), rb.Axis(axis))
+    S = rb.DenseSkOp(D, rb.RNGState(11), dtype=tdt)
+    buff = torch.empty(D.n_rows * D.n_cols, dtype=tdt, device=DEV)
+    rb.fill_dense_unpacked("R", D, D.n_rows, D.n_cols, 0, 0, buff, rb.RNGState(11))
+    W = buff.view(D.n_rows, D.n_cols)[ro:ro + win[0], co:co + win[1]].double()
+    W = W if opS == "N" else W.t()
+    gen = torch.Generator(device=DEV).manual_seed(n + m)
+    A = torch.randn(m * n, dtype=tdt, device=DEV, generator=gen)
+    B = torch.randn(d * n, dtype=tdt, device=DEV, generator=gen)
+    mat = lambda x, r, c: x.view(r, c) if layout == "R" else x.view(c, r).t()
+    ref = alpha * (W @ mat(A, m, n).double()) + beta * mat(B, d, n).double()
+    rb.profile_collect()
+    rb.profile_enable(True)
+    try:
+        rb.lskge3(layout, opS, "N", d, n, m, alpha, S, ro, co, A, n if layout == "R" else m, beta, B,
+                  n if layout == "R" else d)
+        torch.cuda.synchronize()
+    finally:
+        rb.profile_enable(False)
+    got = mat(B, d, n).double()
+    return float((got - ref).norm() / ref.norm()), rb.profile_collect()
+
+
+@pytest.mark.parametrize("dtype,tol", [(np.float64, 1e-13), (np.float32, 1e-5)])
+@pytest.mark.parametrize("layout", ["C", "R"])
+@pytest.mark.parametrize("opS,fam,axis,ro,co", [("N", "G", "L", 0, 0), ("T", "U", "L", 3, 2), ("N", "U", "S", 2, 5)])
+def test_lskge3_operator_ahead(rb, dtype, tol, layout, opS, fam, axis, ro, co):
+    """Many columns of tiles: the operator's chunks are generated ahead of the product (both
+    directions of its counters, windows that start inside one, edges of every kind)."""
+    err, prof = _against_fill(rb, dtype, layout, opS, 501, 20011, 2021, 0.75, -0.5, ro, co, fam, axis)
+    assert "wide_pre_kernel" in prof
+    assert err <= tol
+
+
+@pytest.mark.parametrize("dtype,tol", [(np.float64, 1e-13), (np.float32, 1e-5)])
+@pytest.mark.parametrize("layout", ["C", "R"])
+@pytest.mark.parametrize("alpha,beta", [(1.0, 0.0), (0.5, 2.0)])
+@pytest.mark.parametrize("d,n,m,ro", [(64 * 256 + 65, 61, 700, 0), (64 * 258 - 3, 300, 333, 1), (64 * 300, 257, 1030, 3),
+                                      (130, 7, 40009, 2)])
+def test_lskge3_shared_tiles(rb, dtype, tol, layout, alpha, beta, d, n, m, ro):
+    """Row tiles just above a round of the CUs (whole tiles, then a few that are shared out), an odd
+    share of the chunks, output rows in front of the first and past the last, a tail column."""
+    err, _ = _against_fill(rb, dtype, layout, "N", d, n, m, alpha, beta, ro, 0, "G", "S")
+    assert err <= tol
+
+
+def test_lskge3_captured_without_scratch(rb):
+    """A stream whose workspace is empty, captured: the product takes no memory for itself, and every
+    replay gives the bits of the first."""
+    d, n, m = 200, 90, 3000
+    S = rb.DenseSkOp(rb.DenseDist(d, m), rb.RNGState(3))
+    A = torch.randn(m * n, dtype=torch.float64, device=DEV)
+    B, E = (torch.zeros(d * n, dtype=torch.float64, device=DEV) for _ in range(2))
+    rb.lskge3("C", "N", "N", d, n, m, 1.0, S, 0, 0, A, m, 0.0, E, d)
+    torch.cuda.synchronize()
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=side):
+        rb.lskge3("C", "N", "N", d, n, m, 1.0, S, 0, 0, A, m, 0.0, B, d)
+    first = None
+    for _ in range(3):
+        B.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        first = B.clone() if first is None else first
+        assert torch.equal(B, first)
+        rb.lskge3("C", "N", "N", d, n, m, 1.0, S, 0, 0, A, m, 0.0, E, d)
+    assert float((first - E).norm() / E.norm()) <= 1e-13
