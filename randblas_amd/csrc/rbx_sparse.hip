@@ -325,6 +325,38 @@ static void scale_only(T *C, int64_t d, int64_t n, int64_t crs, int64_t ccs, T b
     RBX_HIP(hipGetLastError());
 }
 
+// Lane l's x, l the same in all lanes: a scalar (no trip through the LDS).
+template <typename X>
+__device__ __forceinline__ X lane_value(X x, int l) {
+    static_assert(sizeof(X) % 4 == 0, "32-bit words");
+    int w[sizeof(X) / 4];
+    __builtin_memcpy(w, &x, sizeof(X));
+#pragma unroll
+    for (unsigned q = 0; q < sizeof(X) / 4; ++q) w[q] = __builtin_amdgcn_readlane(w[q], l);
+    __builtin_memcpy(&x, w, sizeof(X));
+    return x;
+}
+
+// The sum over 16 neighbouring lanes, in each of them, by rotations within DPP
+// rows; the additions are those of the butterfly 8, 4, 2, 1.
+template <int ROR, typename X>
+__device__ __forceinline__ X row_rotate(X x) {
+    int w[sizeof(X) / 4];
+    __builtin_memcpy(w, &x, sizeof(X));
+#pragma unroll
+    for (unsigned q = 0; q < sizeof(X) / 4; ++q) w[q] = __builtin_amdgcn_update_dpp(0, w[q], 0x120 + ROR, 0xf, 0xf, false);
+    __builtin_memcpy(&x, w, sizeof(X));
+    return x;
+}
+template <typename X>
+__device__ __forceinline__ X row16_sum(X p) {
+    p += row_rotate<8>(p);
+    p += row_rotate<4>(p);
+    p += row_rotate<2>(p);
+    p += row_rotate<1>(p);
+    return p;
+}
+
 // Sparse rows times a dense row-major G (C = op(A_sparse) * G), vectorised:
 // a workgroup owns 32 consecutive rows of C and a chunk of 64 * VEC columns;
 // each lane holds VEC consecutive columns, so one 16-byte gather per stored
@@ -427,8 +459,8 @@ __global__ __launch_bounds__(64 * NW) void csr_rows_vec_kernel(const int64_t *ro
                     T v[4];
 #pragma unroll
                     for (int u = 0; u < 4; ++u) {
-                        const int64_t c = __shfl(myc, q + u);  // lanes past cnt hold column 0
-                        v[u] = __shfl(myv, q + u);
+                        const int64_t c = lane_value(myc, q + u);  // lanes past cnt hold column 0
+                        v[u] = lane_value(myv, q + u);
                         if (cl < ncols_out) g[u] = *(const V *)(G + c * ldg + cl);
                     }
 #pragma unroll
@@ -473,6 +505,82 @@ __global__ __launch_bounds__(64 * NW) void csr_rows_vec_kernel(const int64_t *ro
             const int64_t j = col0 + cc;
             if (mine && j < ncols_out) C[i + j * ldc] = tile[rr][cc];
         }
+    }
+}
+
+// The same for few columns (up to LG * VEC) and row-major C: LG lanes own a row,
+// a wave 64 / LG rows, so that narrow outputs do not leave most lanes idle
+// (200000 x 50000, 3.83M entries, FP32: d = 64 217 -> 142 us, d = 20 206 -> 87
+// us; d = 33, whose operator rows are padded to whole pieces, 330 -> 137 us).
+template <typename T, typename IDX, int LG>
+__global__ __launch_bounds__(256) void csr_rows_narrow_kernel(const int64_t *rowptr, const IDX *colidx, const T *vals,
+                                                              int64_t mrows, int64_t ncols_out, T alpha, T beta,
+                                                              const T *G, int64_t ldg, T *C, int64_t ldc, int form,
+                                                              int cvec, int64_t lrow) {
+    using V = typename VecOf<T>::type;
+    constexpr int VEC = VecOf<T>::n;
+    const int lane = threadIdx.x & 63, grp0 = lane & ~(LG - 1), gl = lane & (LG - 1);
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) / LG;
+    int64_t p0 = 0, p1 = 0;
+    bool mine = i < mrows;
+    if (mine) {
+        p0 = rowptr[i];
+        p1 = rowptr[i + 1];
+        if (p1 - p0 > lrow) {  // a long row: summed in segments elsewhere
+            p1 = p0;
+            mine = false;
+        }
+    }
+    const int64_t cl = (int64_t)gl * VEC;
+    const bool in = cl < ncols_out;
+    T c0[VEC], acc[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+        c0[e] = mine && beta != (T)0 && cl + e < ncols_out ? beta * C[i * ldc + cl + e] : (T)0;
+        acc[e] = form == CRV_JIK ? (T)0 : c0[e];
+    }
+    if (alpha != (T)0) {
+        for (int64_t pb = p0; __any(pb < p1); pb += LG) {
+            const int cnt = p1 - pb < LG ? (p1 > pb ? (int)(p1 - pb) : 0) : LG;
+            const int64_t myc = gl < cnt ? (int64_t)colidx[pb + gl] : 0;
+            const T myv = gl < cnt ? vals[pb + gl] : (T)0;
+            for (int q = 0; q < LG && __any(q < cnt); q += 4) {
+                V g[4];
+                T v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int64_t c = __shfl(myc, grp0 + q + u);
+                    v[u] = __shfl(myv, grp0 + q + u);
+                    if (in && q + u < cnt) g[u] = *(const V *)(G + c * ldg + cl);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (q + u >= cnt) continue;
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) {
+                        const T b = vget<T>(g[u], e);
+                        if (form == CRV_KIB) acc[e] = acc[e] + (alpha * v[u]) * b;
+                        else if (form == CRV_JKI) acc[e] = acc[e] + v[u] * (alpha * b);
+                        else acc[e] = acc[e] + v[u] * b;
+                    }
+                }
+            }
+        }
+    }
+    if (!mine) return;
+    if (form == CRV_JIK) {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) acc[e] = alpha != (T)0 ? c0[e] + alpha * acc[e] : c0[e];
+    }
+    if (cvec && cl + VEC <= ncols_out) {
+        V o;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) reinterpret_cast<T *>(&o)[e] = acc[e];
+        *(V *)(C + i * ldc + cl) = o;
+    } else {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+            if (cl + e < ncols_out) C[i * ldc + cl + e] = acc[e];
     }
 }
 
@@ -823,6 +931,22 @@ static void launch_rows_vec(bool colmaj, const int64_t *rowptr, const IDX *colid
     constexpr int VEC = VecOf<T>::n;
     const int64_t lrow = launch_long_rows<T, IDX>(rowptr, colidx, vals, mrows, nnz, ncols_out, alpha, beta, G, ldg, C,
                                                   colmaj ? 1 : ldc, colmaj ? ldc : 1, st);
+    // few columns: several rows to a wave, where the rows still give every CU
+    // several waves (below, one row to a wave keeps more of them busy)
+    if (!colmaj && ncols_out <= 32 * VEC && mrows >= 64 * (int64_t)num_cus()) {
+        auto go = [&](auto lg) {
+            constexpr int LG = decltype(lg)::value;
+            const int64_t blocks = (mrows + 256 / LG - 1) / (256 / LG);
+            RBX_REQUIRE(blocks < (1ll << 31));
+            hipLaunchKernelGGL((csr_rows_narrow_kernel<T, IDX, LG>), dim3((unsigned)blocks), dim3(256), 0, st, rowptr,
+                               colidx, vals, mrows, ncols_out, alpha, beta, G, ldg, C, ldc, form, cvec, lrow);
+        };
+        if (ncols_out <= 8 * VEC) go(std::integral_constant<int, 8>{});
+        else if (ncols_out <= 16 * VEC) go(std::integral_constant<int, 16>{});
+        else go(std::integral_constant<int, 32>{});
+        RBX_HIP(hipGetLastError());
+        return;
+    }
     const int64_t nchunk = (ncols_out + 64 * VEC - 1) / (64 * VEC);
     const int64_t nrb = (mrows + CRV_ROWS - 1) / CRV_ROWS;
     RBX_REQUIRE(nchunk <= 65535 && nrb < (1ll << 31));
@@ -1299,36 +1423,6 @@ static void rskges_impl(char layout, char opA, char opS, int64_t m, int64_t d, i
 }
 
 // ---------------------------------------------------------------- CSR data x dense operator
-// left_spmm for CSR, opA = NoTrans (csr_spmm_impl.hh:51-155).  One wave per
-// output row; lanes walk output columns.
-//   jik: C[i,j] = RN(beta*C) + RN(alpha * sum_l RN(val_l * B[col_l, j]))
-//   ikb: C[i,j] = RN(beta*C), then C += RN(RN(alpha*val_l) * B[col_l, j])
-template <typename T>
-__global__ __launch_bounds__(256) void csr_rows_kernel(const int64_t *rowptr, const int64_t *colidx, const T *vals,
-                                                       int64_t mrows, int64_t ncols_out, T alpha, T beta, const T *B,
-                                                       int64_t brs, int64_t bcs, T *C, int64_t crs, int64_t ccs,
-                                                       int ikb, int64_t lrow) {
-    const int lane = threadIdx.x & 63;
-    const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (i >= mrows) return;
-    const int64_t p0 = rowptr[i], p1 = rowptr[i + 1];
-    if (p1 - p0 > lrow) return;  // a long row: summed in segments elsewhere
-    for (int64_t j = lane; j < ncols_out; j += 64) {
-        T *c = C + i * crs + j * ccs;
-        T acc = (beta == (T)0) ? (T)0 : beta * (*c);
-        if (alpha != (T)0) {
-            if (ikb) {
-                for (int64_t p = p0; p < p1; ++p) acc = acc + (alpha * vals[p]) * B[colidx[p] * brs + j * bcs];
-            } else {
-                T diff = (T)0;
-                for (int64_t p = p0; p < p1; ++p) diff = diff + vals[p] * B[colidx[p] * brs + j * bcs];
-                acc = acc + alpha * diff;
-            }
-        }
-        *c = acc;
-    }
-}
-
 // rows[p] = i for p in [rowptr[i], rowptr[i+1]); positions outside [0, nnz)
 // are never written
 __global__ __launch_bounds__(256) void csr_to_coo_rows_kernel(const int64_t *rowptr, int64_t nrows, int64_t nnz,
@@ -1340,29 +1434,31 @@ __global__ __launch_bounds__(256) void csr_to_coo_rows_kernel(const int64_t *row
 }
 
 // op(submat(S)) of a materialised operator (S.buff in S.layout) gathered into
-// a row-major n_p x n_q matrix.
+// a row-major n_p x n_q matrix of leading dimension ld.
 template <typename T>
 __global__ __launch_bounds__(256) void gather_op_kernel(const T *src, int64_t rs, int64_t cs, int64_t n_p,
-                                                        int64_t n_q, T *dst) {
+                                                        int64_t n_q, T *dst, int64_t ld) {
     const int64_t total = n_p * n_q;
     for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
          idx += (int64_t)gridDim.x * blockDim.x) {
         const int64_t p = idx / n_q, q = idx - p * n_q;
-        dst[idx] = src[p * rs + q * cs];
+        dst[p * ld + q] = src[p * rs + q * cs];
     }
 }
 
-// G = op(submat(S)) as a row-major n_p x n_q matrix in library scratch: the
+// G = op(submat(S)) as a row-major n_p x n_q matrix (leading dimension ld, n_q
+// when 0) in library scratch: the
 // operator is generated from its counters, or gathered from S.buff.
 template <typename T>
 static T *materialize_op(const rbx_dense_skop *S, char opS, int64_t ro_s, int64_t co_s, int64_t n_p, int64_t n_q,
-                         hipStream_t st) {
-    const size_t bytes = (size_t)safe_mul(n_p > 0 ? n_p : 1, n_q > 0 ? n_q : 1) * sizeof(T);
+                         hipStream_t st, int64_t ld = 0) {
+    if (ld == 0) ld = n_q;
+    const size_t bytes = (size_t)safe_mul(n_p > 0 ? n_p : 1, ld > 0 ? ld : 1) * sizeof(T);
     T *G = (T *)scratch(SCRATCH_DENSE_OP, bytes, st);
     if (n_p == 0 || n_q == 0) return G;
     if (S->buff == nullptr) {
         GenMap gm = gen_map(*S, opS, ro_s, co_s, false);
-        fill_generated<T>(gm, n_p, n_q, G, n_q, 1, st);
+        fill_generated<T>(gm, n_p, n_q, G, ld, 1, st);
         return G;
     }
     // S.buff holds the full operator in S.layout; G[p, q] = S[ro_s + p, co_s + q]
@@ -1373,7 +1469,8 @@ static T *materialize_op(const rbx_dense_skop *S, char opS, int64_t ro_s, int64_
     const int64_t rs = opS == 'N' ? frs : fcs, cs = opS == 'N' ? fcs : frs;
     int64_t blocks = (n_p * n_q + 255) / 256;
     if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL(gather_op_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, st, base, rs, cs, n_p, n_q, G);
+    hipLaunchKernelGGL(gather_op_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, st, base, rs, cs, n_p, n_q, G,
+                       ld);
     RBX_HIP(hipGetLastError());
     return G;
 }
@@ -1453,29 +1550,22 @@ static void rsksp3_impl(char layout, char opA, char opS, int64_t m, int64_t d, i
     // row-major op(B) with a row-major C selects the rank-one-update kernels
     // (spmm_dispatch.hh:147-176)
     const int kib = (layout == 'R' && opS_ref == 'N') ? 1 : 0;
-    // G = op(submat(S)), n x d, row-major in scratch
-    T *G = materialize_op<T>(S, opS, ro_s, co_s, n, d, st);
     // Which kernel family the reference reaches (spmm_dispatch.hh:72-90,
     // 139-176): CSR with op(A) = N, or CSC with op(A) = T (its transpose is the
     // CSR matrix sharing its arrays), runs row by row in stored order; every
     // other case runs column by column, i.e. ascending column of op(A).
     const bool row_kernel = (A.fmt == 'R' && opA == 'N') || (A.fmt == 'C' && opA == 'T');
+    // G = op(submat(S)), n x d, row-major in scratch; the row kernels gather
+    // 16-byte pieces of its rows
+    constexpr int VEC = VecOf<T>::n;
+    const int64_t ldg = row_kernel ? (d + VEC - 1) / VEC * VEC : d;
+    T *G = materialize_op<T>(S, opS, ro_s, co_s, n, d, st, ldg);
     if (row_kernel) {
         ProfScope prof("csr_rows_kernel", st);
-        constexpr int VEC = VecOf<T>::n;
-        // vector path: 16-byte aligned rows of G (d columns wide from a
-        // 256-byte base); a row-major B takes vector stores when aligned too
+        // a row-major B takes vector stores when aligned too
         const int cvec = layout == 'R' && ldb % VEC == 0 && ((uintptr_t)B % 16) == 0;
-        if (d % VEC == 0) {
-            launch_rows_vec<T, int64_t>(layout == 'C', A.ptr, A.idx, (const T *)A.vals, m, A.nnz, d, alpha, beta,
-                                        (const T *)G, d, B, ldb, kib ? CRV_KIB : CRV_JIK, cvec, st);
-        } else {
-            const int64_t lrow = launch_long_rows<T, int64_t>(A.ptr, A.idx, (const T *)A.vals, m, A.nnz, d, alpha,
-                                                              beta, (const T *)G, d, B, crs, ccs, st);
-            dim3 grid((unsigned)((m + 3) / 4));
-            hipLaunchKernelGGL(csr_rows_kernel<T>, grid, dim3(256), 0, st, A.ptr, A.idx, (const T *)A.vals, m, d,
-                               alpha, beta, (const T *)G, (int64_t)d, (int64_t)1, B, crs, ccs, kib, lrow);
-        }
+        launch_rows_vec<T, int64_t>(layout == 'C', A.ptr, A.idx, (const T *)A.vals, m, A.nnz, d, alpha, beta,
+                                    (const T *)G, ldg, B, ldb, kib ? CRV_KIB : CRV_JIK, cvec, st);
         RBX_HIP(hipGetLastError());
         return;
     }
@@ -1582,16 +1672,20 @@ __global__ __launch_bounds__(256) void sddmm_csr_kernel(const int64_t *rowptr, c
     }
 }
 
-// Vectorised form (d a multiple of the vector width): a group of 16 lanes
-// owns one stored entry, so a wave works on four entries of a row at once;
-// each lane gathers 16-byte pieces of op(S)'s row and the 16 partial dot
-// products are summed with four butterfly steps.
-template <typename T>
+// Vectorised form: a group of 16 lanes owns one stored entry, so a wave works
+// on four entries of a row at once; each lane gathers 16-byte pieces of op(S)'s
+// row, at any alignment, and the 16 partial dot products are summed with four
+// rotations.  Bbar's row is in registers for all its entries.  Bound by the
+// gathers: 200000 x 50000, 3.83M entries, d = 256: FP32 404 us, 9.7 TB/s of
+// operator rows (490 us with Bbar's row read from LDS for every entry and the
+// sums through ds_bpermute), FP64 760 (930).
+// WHOLE: d is a multiple of VEC.
+template <typename T, int NQ, bool WHOLE>
 __global__ __launch_bounds__(256) void sddmm_vec_kernel(const int64_t *rowptr, const int64_t *colidx, int64_t m,
                                                         int64_t d, T alpha, const T *Bb, int64_t brs, int64_t bcs,
                                                         const T *G, T *dvals) {
-    using V = typename VecOf<T>::type;
-    constexpr int VEC = VecOf<T>::n, DC = SddmmChunk<T>::DC, GS = 16 * VEC, NQ = DC / GS;
+    constexpr int VEC = VecOf<T>::n, GS = 16 * VEC, DC = NQ * GS;
+    typedef T V __attribute__((ext_vector_type(VEC), aligned(sizeof(T))));
     __shared__ T tile[SD_RB][DC + 1];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int grp = lane >> 4, gl = lane & 15;
@@ -1612,6 +1706,19 @@ __global__ __launch_bounds__(256) void sddmm_vec_kernel(const int64_t *rowptr, c
             const int64_t i = i0 + r;
             if (i >= m) break;
             const int64_t kb = rowptr[i], ke = rowptr[i + 1];
+            // the lane's part of Bbar's row: columns cc .. cc + VEC - 1 of
+            // each piece; one that would pass the end is moved back by `back`
+            // columns (into the chunk before this one if it has to)
+            T bv[NQ][VEC];
+            int cs[NQ], back[NQ];
+#pragma unroll
+            for (int u = 0; u < NQ; ++u) {
+                const int cc = gl * VEC + u * GS;
+                cs[u] = WHOLE || cc + VEC <= dc ? cc : (int)dc - VEC;
+                back[u] = cc - cs[u];
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) bv[u][e] = cc < dc && (WHOLE || e >= back[u]) ? tile[r][cs[u] + e] : (T)0;
+            }
             for (int64_t pb = kb; pb < ke; pb += 64) {
                 // the batch's columns loaded once (lane e: entry pb + e);
                 // two steps of four entries (one per 16-lane group) in flight,
@@ -1623,12 +1730,12 @@ __global__ __launch_bounds__(256) void sddmm_vec_kernel(const int64_t *rowptr, c
                     V gv[2][NQ];
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
-                        const int64_t c = __shfl(myc, q + 4 * h + grp);  // entries past cnt: column 0
+                        const int e = q + 4 * h + grp;
+                        const int64_t c = __shfl(myc, e);
                         const T *grow = G + c * d + j0;
 #pragma unroll
                         for (int u = 0; u < NQ; ++u) {
-                            const int cc = gl * VEC + u * GS;
-                            if (cc < dc) gv[h][u] = *(const V *)(grow + cc);
+                            if (gl * VEC + u * GS < dc && e < cnt) gv[h][u] = *(const V *)(grow + cs[u]);
                         }
                     }
 #pragma unroll
@@ -1636,13 +1743,12 @@ __global__ __launch_bounds__(256) void sddmm_vec_kernel(const int64_t *rowptr, c
                         T p = (T)0;
 #pragma unroll
                         for (int u = 0; u < NQ; ++u) {
-                            const int cc = gl * VEC + u * GS;
-                            if (cc < dc)
+                            if (gl * VEC + u * GS >= dc) continue;
 #pragma unroll
-                                for (int e = 0; e < VEC; ++e) p = fma(tile[r][cc + e], vget<T>(gv[h][u], e), p);
+                            for (int e = 0; e < VEC; ++e)
+                                p = WHOLE || e >= back[u] ? fma(bv[u][e], gv[h][u][e], p) : p;
                         }
-#pragma unroll
-                        for (int o = 8; o >= 1; o >>= 1) p += __shfl_xor(p, o);
+                        p = row16_sum(p);
                         const int e = q + 4 * h + grp;
                         if (e < cnt && gl == 0) {
                             const int64_t k = pb + e;
@@ -1682,9 +1788,18 @@ static void rsksp3_adjoint_impl(char layout, char opS, int64_t m, int64_t d, int
     const int64_t blocks = (m + SD_RB - 1) / SD_RB;
     RBX_REQUIRE(blocks < (1ll << 31));
     ProfScope prof("sddmm_csr_kernel", st);
-    if (d % VecOf<T>::n == 0)
-        hipLaunchKernelGGL(sddmm_vec_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, st, A->rowptr, A->colidxs, m, d,
-                           alpha, Bbar, brs, bcs, (const T *)G, dvals);
+    constexpr int VEC = VecOf<T>::n, GS = 16 * VEC, NQM = SddmmChunk<T>::DC / GS;
+    auto go = [&](auto nq, auto whole) {
+        hipLaunchKernelGGL((sddmm_vec_kernel<T, decltype(nq)::value, decltype(whole)::value>), dim3((unsigned)blocks),
+                           dim3(256), 0, st, A->rowptr, A->colidxs, m, d, alpha, Bbar, brs, bcs, (const T *)G, dvals);
+    };
+    auto with = [&](auto nq) {
+        if (d % VEC == 0) go(nq, std::true_type{});
+        else go(nq, std::false_type{});
+    };
+    if (d >= VEC && d <= GS) with(std::integral_constant<int, 1>{});
+    else if (d >= VEC && d <= 2 * GS) with(std::integral_constant<int, 2>{});
+    else if (d >= VEC) with(std::integral_constant<int, NQM>{});
     else
         hipLaunchKernelGGL(sddmm_csr_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, st, A->rowptr, A->colidxs, m, d,
                            alpha, Bbar, brs, bcs, (const T *)G, dvals);

@@ -786,3 +786,44 @@ def test_lskges_row_major_uneven_rows(rb, orc, dtype, tol, prepared):
     others = np.arange(d) != 4
     assert np.array_equal(got[others], ref[others])
     assert np.linalg.norm(got[4] - ref[4]) <= tol * np.linalg.norm(ref[4])
+
+
+@pytest.mark.parametrize("dtype,tol", [(np.float64, 1e-13), (np.float32, 1e-5)])
+@pytest.mark.parametrize("layout", ["C", "R"])
+@pytest.mark.parametrize("d", [1, 2, 3, 4, 5, 15, 16, 17, 31, 33, 64, 65, 127, 128, 129, 131, 257, 259])
+def test_rsksp3_and_adjoint_widths(rb, orc, dtype, tol, layout, d):
+    """Enough rows for several to a wave: widths around every number of lanes per row and every
+    chunk of the adjoint's, last pieces moved back (into the chunk before, where the last is
+    narrower than a vector).  The product bit-identical to the oracle, empty rows among the rows;
+    the adjoint of a smaller matrix."""
+    rng = np.random.default_rng(d)
+    m, n = 17000, 300
+    rowptr, colidx, vals = _csr(rng, m, n, 3)
+    vals = vals.astype(dtype)
+    pre, tdt = ("d", torch.float64) if dtype == np.float64 else ("s", torch.float32)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+    S = rb.DenseSkOp(rb.DenseDist(n, d), rb.RNGState(19))
+    ldb = m + 1 if layout == "C" else d + d % 2
+    B0 = rng.standard_normal(ldb * (d if layout == "C" else m)).astype(dtype)
+    Bd = t(B0)
+    rb.rsksp3(layout, "N", "N", m, d, n, -1.5, rb.CSRMatrix(m, n, t(vals), t(rowptr), t(colidx)), 0, 0, S, 0, 0, 0.25,
+              Bd, ldb)
+    full, _ = orc.fill_dense(n, d, [0, 0, 0, 0], [19, 0], dtype=dtype)
+    nat = orc.natural_layout(n, d, "L")
+    Sbuf = np.ascontiguousarray(full.reshape(-1, order="F" if nat == "C" else "C"))
+    ref = B0.copy()
+    orc.left_spmm_csr(pre, layout, "N" if nat == layout else "T", m, d, n, -1.5, vals, rowptr, colidx, Sbuf,
+                      n if nat == "C" else d, 0.25, ref, ldb)
+    assert np.array_equal(host(Bd), ref)
+
+    m = 70
+    rowptr, colidx, vals = rowptr[:m + 1], colidx[:rowptr[m]], vals[:rowptr[m]]
+    ldbb = m if layout == "C" else d
+    Bbar = rng.standard_normal(m * d).astype(dtype)
+    dvals = torch.zeros(len(vals), dtype=tdt, device=DEV)
+    rb.rsksp3_adjoint(layout, "N", m, d, n, 0.5, rb.CSRMatrix(m, n, t(vals), t(rowptr), t(colidx)), S, 0, 0, t(Bbar),
+                      ldbb, dvals)
+    brs, bcs = (1, ldbb) if layout == "C" else (ldbb, 1)
+    ref = orc.sddmm_csr("d", m, d, 0.5, rowptr, colidx, Bbar.astype(np.float64), brs, bcs,
+                        full.astype(np.float64).reshape(-1), d, 1)
+    assert np.linalg.norm(host(dvals) - ref) <= tol * np.linalg.norm(ref)
