@@ -634,13 +634,18 @@ static void bf16_split_sketch(char layout, char opS, char opA, int64_t d, int64_
     pb.g = gen_map(*S, opS, ro_s, co_s, false);
     // The pair kernel's tile is 256 cb columns wide.  A 32-deep chunk of a tile
     // costs its MFMAs (also for the zero columns past N) and the operator's
-    // generation, about as much as those of 160 columns with three terms.
+    // generation, about as much as those of 160 columns with three terms; the
+    // split of a column costs about 4.5 row tiles' MFMAs on it (1.8 ps an entry
+    // against 0.4: few output rows with many zero columns pay for it, 147 x
+    // 111947 times 616 columns: 488 us in one tile of 1024, 378 in three of 256).
     const bool pair = !pb.g.b_along_rows && (pb.g.b_off & 3) == 0;
+    const int64_t row_tiles = (M + BF_MT - 1) / BF_MT;
     int cb = BF_NT / 256;
     if (pair) {
         int64_t best = 0;
         for (int c = BF_CB; c >= 1; c /= 2) {
-            const int64_t nb = (N + 256 * c - 1) / (256 * c), cost = nb * (256 * c * n_terms + 480);
+            const int64_t nb = (N + 256 * c - 1) / (256 * c);
+            const int64_t cost = row_tiles * nb * (256 * c * n_terms + 480) + 14 * 256 * c * nb;
             if (c > 1 && nb * 8 * c > 65535) continue;  // the split's grid
             if (best == 0 || cost < best) {
                 best = cost;
@@ -648,7 +653,7 @@ static void bf16_split_sketch(char layout, char opS, char opA, int64_t d, int64_
             }
         }
     }
-    pb.nMB = (int)((M + BF_MT - 1) / BF_MT);
+    pb.nMB = (int)row_tiles;
     pb.nNB = (int)((N + 256 * cb - 1) / (256 * cb));
     pb.Np = pair ? (int64_t)pb.nNB * 256 * cb : (N + 255) / 256 * 256;
     pb.ldp = (N + 3) / 4 * 4;
