@@ -985,13 +985,13 @@ __global__ __launch_bounds__(256) void csr_stripe_kernel(const int64_t *__restri
                                                          const int32_t *__restrict__ colidx,
                                                          const T *__restrict__ vals, int64_t mrows, int64_t n, T alpha,
                                                          T beta, const T *__restrict__ B, int64_t ldb, T *C,
-                                                         int64_t crs, int64_t ccs, int64_t lrow, int nrb, int nstripes) {
+                                                         int64_t crs, int64_t ccs, int64_t lrow, int nrb, int nstripes,
+                                                         int by_xcd) {
     typedef T V __attribute__((ext_vector_type(VEC), aligned(sizeof(T))));
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    // XCD-aware order: the rows of one stripe on one XCD, whose L2 then holds
-    // the part of Bm that they are all going through
+    // by_xcd: the rows of one stripe on one XCD
     const int W = nrb * nstripes, xcd = blockIdx.x % 8, xi = blockIdx.x / 8;
-    const int t = xcd * (W / 8) + (xcd < W % 8 ? xcd : W % 8) + xi;
+    const int t = by_xcd ? xcd * (W / 8) + (xcd < W % 8 ? xcd : W % 8) + xi : (int)blockIdx.x;
     const int64_t i = 4 * (int64_t)(t % nrb) + wave;
     if (i >= mrows) return;
     const int64_t p0 = rowptr[i], p1 = rowptr[i + 1];
@@ -1052,6 +1052,13 @@ static int stripe_vec(int64_t n) {
     return g4 > g2 && g4 > g1 ? 4 : (g2 > g1 ? 2 : 1);
 }
 
+// Up to this many rows the workgroups of a stripe go to one XCD, whose L2 holds
+// what its rows share of Bm (FP32 300 x 131072, 1000 columns: 283 us against
+// 350); more rows drift apart too far for that, and in plain order all XCDs are
+// at the same stripe, which the last-level cache holds (FP32 8000 x 100000, 400
+// columns: 199 us against 231).
+constexpr int64_t STRIPE_XCD_MAX_ROWS = 1024;
+
 // C = alpha * A * Bm + beta * C by csr_stripe_kernel; rows longer than lrow are left out.
 template <typename T>
 static void launch_stripes(const int64_t *rowptr, const int32_t *colidx, const T *vals, int64_t mrows, int64_t n,
@@ -1061,10 +1068,11 @@ static void launch_stripes(const int64_t *rowptr, const int32_t *colidx, const T
     const int64_t nrb = (mrows + 3) / 4, ns = (n + 64 * vec - 1) / (64 * vec);
     RBX_REQUIRE(nrb < (1ll << 31) / ns);
     const dim3 grid((unsigned)(nrb * ns));
+    const int by_xcd = mrows <= STRIPE_XCD_MAX_ROWS;
     auto go = [&](auto vc, auto form) {
         hipLaunchKernelGGL((csr_stripe_kernel<T, decltype(vc)::value, decltype(form)::value, 8>), grid, dim3(256), 0,
                            st, rowptr, colidx, vals, mrows, n, alpha, beta, B, ldb, C, crs, ccs, lrow, (int)nrb,
-                           (int)ns);
+                           (int)ns, by_xcd);
     };
     auto with_form = [&](auto vc) {
         if (kib) go(vc, std::true_type{});
