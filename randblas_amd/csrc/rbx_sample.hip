@@ -336,11 +336,13 @@ __global__ __launch_bounds__(1024) void iid_cdf_table_kernel(Ctr128 ctr, uint32_
 //                       left.  No result depends on the guesses.
 //   cdf_write_kernel    each block's partial sums from its exact start, scaled
 // 10^6 FP64 weights: 9 blocks leave a binade.  Bound by latency: the chain
-// kernel's dependent scans.  Arrays of a few blocks skip the first three.
+// kernel's dependent scans (157 us of them; 135 with the first CDF_HEAD terms
+// added one by one; 3122 weights and as many draws 106 -> 79 us).  Arrays of a few blocks skip the first three.
 // Meta: status 0 ok (inv = 1 / sum); 1 + i: w[i] < error_if_below (w[0..i)
 // hold the partial sums, as when the reference throws there); -1: the total
 // is below sqrt(n) * eps (w holds the partial sums, unscaled).
 constexpr int CDF_BLK = 2048, CDF_PER = CDF_BLK / 256;
+constexpr int CDF_HEAD = 192;  // terms (2 us) whose sums may leave eight binades (3 us each in scans)
 constexpr int64_t CDF_DIRECT = 4;  // blocks that the chain kernel takes by itself
 struct CdfMeta {
     long long status, first;  // first: weights before the first refused one
@@ -529,6 +531,22 @@ __global__ __launch_bounds__(256) void cdf_chain_kernel(int64_t n, T *w, T error
             first = i0 + len;
         }
         int pos = 0;  // terms of the block already in the sum
+        if (b == 0) {
+            // the first sums leave a binade every few terms: added one by one
+            pos = len < CDF_HEAD ? len : CDF_HEAD;
+            if (tid == 0) {
+                T s = (T)0;
+#pragma unroll 8
+                for (int i = 0; i < pos; ++i) {
+                    s = s + wbuf[i];
+                    obuf[i] = s;
+                }
+                base_sh = (long long)chain_bits(s);
+            }
+            __syncthreads();
+            bits = (int64_t)base_sh;
+            __syncthreads();  // (base_sh is written again below)
+        }
         while (true) {
             const int e = chain_exp<T>(bits);
             const uint64_t limit = chain_limit<T>(e);
