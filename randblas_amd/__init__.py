@@ -653,17 +653,18 @@ def fill_sparse(S: SparseSkOp) -> None:
         S.vals = torch.empty(full, dtype=S.dtype, device="cuda")
         S.rows = torch.empty(full, dtype=torch.int64, device="cuda")
         S.cols = torch.empty(full, dtype=torch.int64, device="cuda")
-    nnz = C.c_int64()
-    nxt = c_rng_state()
     pre = "d" if S.dtype == torch.float64 else "s"
-    _need("S.vals", S.vals, S.dtype, full)
-    _need("S.rows", S.rows, torch.int64, full)
-    _need("S.cols", S.cols, torch.int64, full)
+    for name, t, dtype in (("S.vals", S.vals, S.dtype), ("S.rows", S.rows, torch.int64), ("S.cols", S.cols, torch.int64)):
+        _need(name, t, dtype, full)
+        _ptr(t)  # (a GPU tensor)
     S.release()
-    _call(f"rbx_{pre}fill_sparse_unpacked_nosub", C.byref(S.dist.c()), C.byref(nnz), _ptr(S.vals), _ptr(S.rows),
-          _ptr(S.cols), C.byref(S.seed_state.c()), C.byref(nxt), _stream())
-    S.nnz = nnz.value
-    S.prepare()
+    s = S.c()
+    try:
+        _call(f"rbx_{pre}fill_sparse_skop", C.byref(s), _stream())  # and S's prepared copy
+    finally:
+        S.nnz = s.nnz
+        S._prep = s.prep
+        S._prep_key = S._key()
 
 
 def fill_sparse_unpacked_nosub(D: SparseDist, vals, rows, cols, seed: RNGState):
