@@ -275,6 +275,8 @@ static WidePlan wide_plan(const GemmProblem &pb, int ko, int mo, bool NU, bool s
             }
         }
     }
+    // partials too large for any number of shares: whole tiles, longer sums
+    if (best.tile == 0 && split_ok) return wide_plan<T>(pb, ko, mo, NU, false, pre_ok);
     return best;
 }
 
