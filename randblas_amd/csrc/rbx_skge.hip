@@ -17,7 +17,7 @@ namespace rbx {
 
 // ---------------------------------------------------------------- one column
 // C (M x 1) = alpha * X * y + beta * C with X the generated operator: a
-// vector sketch.  The tile kernels would run their MFMAs over 255 empty
+// vector sketch.  The wide kernel would run its MFMAs over 31 empty
 // columns; here each workgroup takes GV_ROWS rows and a K range of kw (a
 // multiple of 4, chosen so the grid holds several workgroups per CU),
 // every thread generates whole Philox cells of those rows (exact values, as
